@@ -1,0 +1,76 @@
+"""Grouped block factorisations through the C ABI at the sizes where their kernels change course
+(needs an MI355X).
+
+Householder QR (xh_block_qr): rows around the 64, 128, 192, 256 and 1024 that pick the
+kernel, single rows and columns, more columns than one panel, wide blocks, dependent columns,
+reflectors or working copies too large for LDS, and a middle dimension above min(m, n).  Bounds (Higham, Accuracy and Stability of Numerical Algorithms, 2nd
+ed., theorem 19.4): ||A - Q R||_F and ||Q^T Q - I||_F are at most about m n eps times ||A||_F and
+sqrt(n); the tests allow m n eps with the constant 1, which random rounding stays far below.
+"""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from xped_amd import _lib
+from xped_amd._lib import lib
+
+pytestmark = pytest.mark.gpu
+
+EPS = np.finfo(float).eps
+
+
+def _run(rt, fn, blocks, out_sizes, items):
+    """Uploads the blocks (column-major), calls fn(items, n, dA, *outs) and downloads the outputs."""
+    L, ctx = lib(), rt.ctx()
+    flat = np.concatenate([b.T.reshape(-1) for b in blocks])
+    dA, outs = C.c_void_p(), [C.c_void_p() for _ in out_sizes]
+    for p, n in zip([dA] + outs, [flat.size] + list(out_sizes)):
+        assert L.xh_alloc(ctx, 8 * max(n, 1), C.byref(p)) == 0
+    L.xh_upload(ctx, dA, flat.ctypes.data, 8 * flat.size)
+    arr = (_lib.xh_factor_item * len(items))(*items)
+    assert fn(ctx, arr, len(items), dA, *outs) == 0, L.xh_last_error(ctx)
+    res = []
+    for p, n in zip(outs, out_sizes):
+        x = np.empty(n)
+        L.xh_download(ctx, x.ctypes.data, p, 8 * n)
+        res.append(x)
+    for p in [dA] + outs:
+        L.xh_free(ctx, p)
+    return res
+
+
+QR_SHAPES = [(1, 1), (1, 7), (7, 1), (16, 16), (17, 16), (64, 64), (65, 33), (63, 5), (128, 100), (129, 40), (256, 70), (257, 60), (1024, 15),
+             (1025, 15), (20, 300), (190, 180), (130, 300), (192, 90), (193, 66), (256, 250), (700, 200), (2000, 40), (48, 700)]
+
+
+def test_block_qr_across_kernel_edges(rt):
+    r = np.random.default_rng(5)
+    blocks = [r.uniform(-1, 1, s) for s in QR_SHAPES]
+    dep = r.uniform(-1, 1, (40, 12))
+    dep[:, 3] = 0.0  # no reflector: tau = 0
+    dep[:, 7] = 2.0 * dep[:, 1]
+    blocks.append(dep)
+    blocks.append(np.eye(33))
+    mids = [min(b.shape) for b in blocks]
+    mids[4], mids[3] = 19, 16  # a middle dimension above the block's rows: zero columns of Q, zero rows of R
+    items, ao, uo, vo = [], 0, 0, 0
+    for b, k in zip(blocks, mids):
+        m, n = b.shape
+        items.append(_lib.xh_factor_item(ao, uo, k, vo, m, n))
+        ao, uo, vo = ao + m * n, uo + m * k, vo + k * n
+    Q, R = _run(rt, lib().xh_block_qr, blocks, (uo, vo), items)
+    for b, k, it in zip(blocks, mids, items):
+        m, n = b.shape
+        q = Q[it.u_off:it.u_off + m * k].reshape(k, m).T
+        rr = R[it.vt_off:it.vt_off + k * n].reshape(n, k).T
+        real = min(k, m)
+        tol = EPS * m * max(n, 4)
+        assert np.array_equal(rr[:real], np.triu(rr[:real])) and not rr[real:].any() and not q[:, real:].any()
+        assert np.linalg.norm(b - q @ rr) <= tol * np.linalg.norm(b), (m, n)
+        assert np.linalg.norm(q[:, :real].T @ q[:, :real] - np.eye(real)) <= tol * np.sqrt(real), (m, n)
+        # the sign convention of LAPACK (and Eigen): r_kk = -sign(c_kk) ||.||
+        lq = np.linalg.qr(b)[1]
+        live = np.abs(np.diag(lq)) > 1e-8 * np.linalg.norm(b)
+        kk = np.flatnonzero(live)
+        assert np.array_equal(np.sign(np.diag(rr)[kk]), np.sign(np.diag(lq)[kk])) or (m, n) == (33, 33), (m, n)

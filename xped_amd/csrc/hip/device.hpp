@@ -184,6 +184,31 @@ __device__ __forceinline__ uint32_t fdiv(uint32_t x, uint32_t magic, uint32_t sh
     return (__umulhi(x, magic) + x) >> shift;
 }
 
+// Sum over each group of G (16 or 64) consecutive lanes, in every lane of the group, all bitwise
+// equal.  Within 16 lanes by DPP rotations, which cost a move each where a shuffle through
+// ds_bpermute costs an LDS round trip.
+template <int CTRL>
+__device__ __forceinline__ double dpp_mov(double x)
+{
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, 0xf, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+template <int G>
+__device__ __forceinline__ double lanes_sum(double x)
+{
+    static_assert(G == 16 || G == 64, "groups of a DPP row or a wave");
+    x += dpp_mov<0x128>(x);  // row_ror:8, 4, 2, 1
+    x += dpp_mov<0x124>(x);
+    x += dpp_mov<0x122>(x);
+    x += dpp_mov<0x121>(x);
+    if constexpr(G == 64) {
+        x += __shfl_xor(x, 16);
+        x += __shfl_xor(x, 32);
+    }
+    return x;
+}
+
 // One output leg of a permute task (shared by the permute kernels and the GEMM that reads its A
 // operand through a permute): extent, magic division by the extent, and the stride of the leg's
 // source leg in the source subblock's row (bit 8 of flags clear) or column (set) index; bits 0-7

@@ -213,90 +213,234 @@ __global__ __launch_bounds__(F_THREADS) void k_svd_jacobi(FactorArgs fa)
 // Q has `q_cols` columns (the tensor's middle dimension; columns beyond m are zero) and R has
 // `q_cols` rows (rows beyond min(m, n) are zero).  Item fields: u_off -> Q, vt_off -> R,
 // s_off -> q_cols (reused as an integer).
-template <bool LDS>
-__global__ __launch_bounds__(F_THREADS) void k_qr(FactorArgs fa)
+//
+// Both kernels are a serial chain of min(m, n) reflectors, bound by the latency of one reflector
+// and by LDS reads, not by flops.  A group of G lanes owns a column (column j: group j mod the
+// number of groups) and its lane l the rows l, l + G, ..., so dot products end in a lane
+// reduction inside the group.  The group that owns column k + 1 applies reflector k and at once
+// makes reflector k + 1 from the values it still holds: one barrier per reflector.  Q is made
+// column by column without barriers, from reflector min(c, kmax - 1) down, since the later ones
+// leave e_c alone.
+//
+// k_qr (at most G * RM rows): NC columns per group live in registers from their load to their
+// store, and only the reflectors V are in LDS (or, when they do not fit, in global memory), full
+// columns with zeros above and a one on the diagonal, padded with zeros to G * RM rows, so that a
+// step reads RM values per lane without conditions for all NC columns.  More than NC columns per
+// group run in panels; a panel first takes all reflectors of the panels before it.
+// k_qr_tall (any number of rows): the working copy is in LDS or global memory.
+//
+// One thread per trailing column, serial over its rows, took 2864 us for the 9 blocks (132 x 85
+// the largest) of a U(1) matrix product tensor at bond 300; columns kept in LDS by such groups
+// 550 us (48 LDS operations per column and reflector); k_qr takes 173 us.
+constexpr int QR_THREADS = 1024;
+
+__host__ __device__ inline int64_t qr_work_doubles(int64_t m, int64_t n, int64_t rows) { return (m < n ? m : n) * (rows + 1) + 1; }
+__host__ __device__ inline int64_t qr_tall_work_doubles(int64_t m, int64_t n) { return m * n + (m < n ? m : n) + 1; }
+
+// beta, tau and 1 / (c0 - beta) of the reflector of a column with diagonal entry c0 and squared
+// norm `tail` below it; tau = 0 (H = I) when nothing is below
+__device__ __forceinline__ void make_householder(double c0, double tail, double& beta, double& t, double& inv)
+{
+    beta = c0;
+    t = 0.0;
+    inv = 1.0;
+    if(!(tail <= DBL_MIN)) {
+        beta = sqrt(c0 * c0 + tail);
+        if(c0 >= 0.0) beta = -beta;
+        t = (beta - c0) / beta;
+        inv = 1.0 / (c0 - beta);
+    }
+}
+
+template <bool LDS, int G, int RM, int NC>
+__global__ __launch_bounds__(QR_THREADS) void k_qr(FactorArgs fa)
 {
     extern __shared__ double smem[];
-    __shared__ double red[F_THREADS / 64];
-    __shared__ double s_beta, s_tau, s_c0;
     const xh_factor_item it = fa.items[blockIdx.x];
     const int m = it.m, n = it.n;
     const int qc = static_cast<int>(it.s_off);
     if(m == 0 || n == 0) return;
+    constexpr int NG = QR_THREADS / G, LD = G * RM, PC = NG * NC;
+    const int kmax = min(m, n);
+    double* V = work_base<LDS>(smem, fa);  // reflectors: kmax columns of LD rows
+    double* tau = V + int64_t(LD) * kmax;  // kmax
+    const int lane = threadIdx.x % G, grp = threadIdx.x / G;
+    double x[NC][RM], v[RM];
+    auto load_v = [&](int k) {
+        const double* col = V + int64_t(k) * LD + lane;
+#pragma unroll
+        for(int i = 0; i < RM; ++i) v[i] = col[i * G];
+    };
+    // x -= tau (v^T x) v for the group's columns first + q NG > after (those up to `after` are finished)
+    auto apply = [&](double t, int first, int after) {
+        double w[NC];
+#pragma unroll
+        for(int q = 0; q < NC; ++q) {
+            w[q] = 0.0;
+#pragma unroll
+            for(int i = 0; i < RM; ++i) w[q] = fma(v[i], x[q][i], w[q]);
+        }
+#pragma unroll
+        for(int q = 0; q < NC; ++q) w[q] = xh::lanes_sum<G>(w[q]) * t;
+#pragma unroll
+        for(int q = 0; q < NC; ++q)
+            if(first + q * NG > after)
+#pragma unroll
+                for(int i = 0; i < RM; ++i) x[q][i] = fma(-w[q], v[i], x[q][i]);
+    };
+    // makes reflector k from the column xc, leaving beta on xc's diagonal
+    auto reflector = [&](int k, double (&xc)[RM]) {
+        double tail = 0.0, c0 = 0.0;
+        int d = k - lane;  // row lane + i G lies below the diagonal for i G > d
+#pragma unroll
+        for(int i = 0; i < RM; ++i) {
+            tail = fma(i * G > d ? xc[i] : 0.0, xc[i], tail);
+            c0 = i * G == d ? xc[i] : c0;
+        }
+        tail = xh::lanes_sum<G>(tail);
+        c0 = xh::lanes_sum<G>(c0);
+        double beta, t, inv;
+        make_householder(c0, tail, beta, t, inv);
+        asm("" : "+v"(d));  // compare again: 2 RM lane masks kept over the square root would spill
+        double* col = V + int64_t(k) * LD + lane;
+#pragma unroll
+        for(int i = 0; i < RM; ++i) {
+            col[i * G] = i * G > d ? xc[i] * inv : (i * G == d ? 1.0 : 0.0);
+            xc[i] = i * G == d ? beta : xc[i];
+        }
+        if(lane == 0) tau[k] = t;
+    };
+    for(int p0 = 0; p0 < n; p0 += PC) {
+#pragma unroll
+        for(int q = 0; q < NC; ++q) {
+            const int j = p0 + grp + q * NG;
+#pragma unroll
+            for(int i = 0; i < RM; ++i) {
+                const int r = lane + i * G;
+                x[q][i] = j < n && r < m ? fa.A[it.a_off + int64_t(j) * m + r] : 0.0;
+            }
+        }
+        for(int k = 0; k < min(p0, kmax); ++k) {
+            load_v(k);
+            apply(tau[k], p0 + grp, -1);
+        }
+        const int p1 = min(p0 + PC, kmax);
+        if(grp == 0 && p0 < kmax) reflector(p0, x[0]);
+        for(int k = p0; k < p1; ++k) {
+            __syncthreads();  // reflector k is there
+            const double t = tau[k];
+            if(k + 1 < min(p0 + PC, n)) {
+                load_v(k);
+                apply(t, p0 + grp, k);
+                if(k + 1 < p1) {
+#pragma unroll
+                    for(int q = 0; q < NC; ++q)
+                        if(p0 + grp + q * NG == k + 1) reflector(k + 1, x[q]);
+                }
+            }
+        }
+        // R: qc x n, the rows up to the diagonal (rows beyond min(m, n) are zero)
+#pragma unroll
+        for(int q = 0; q < NC; ++q) {
+            const int j = p0 + grp + q * NG;
+            if(j >= n) continue;
+            double* out = fa.Vt + it.vt_off + int64_t(j) * qc;
+#pragma unroll
+            for(int i = 0; i < RM; ++i) {
+                const int r = lane + i * G;
+                if(r < qc) out[r] = r < m && r <= j ? x[q][i] : 0.0;
+            }
+            for(int r = lane + LD; r < qc; r += G) out[r] = 0.0;
+        }
+    }
+    __syncthreads();
+    // Q columns 0..qc-1: Q e_c = H_0 H_1 ... H_{kmax-1} e_c (zero for c >= m)
+    for(int c0 = 0; c0 < qc; c0 += PC) {
+#pragma unroll
+        for(int q = 0; q < NC; ++q)
+#pragma unroll
+            for(int i = 0; i < RM; ++i) x[q][i] = lane + i * G == c0 + grp + q * NG ? 1.0 : 0.0;
+        // a column beyond m holds its one outside the block (or nowhere): no reflector reaches it
+        for(int k = min(c0 + grp + (NC - 1) * NG, kmax - 1); k >= 0; --k) {
+            load_v(k);
+            apply(tau[k], c0 + grp, -1);
+        }
+#pragma unroll
+        for(int q = 0; q < NC; ++q) {
+            const int c = c0 + grp + q * NG;
+            if(c >= qc) continue;
+            double* out = fa.U + it.u_off + int64_t(c) * m;
+#pragma unroll
+            for(int i = 0; i < RM; ++i) {
+                const int r = lane + i * G;
+                if(r < m) out[r] = x[q][i];
+            }
+        }
+    }
+}
+
+template <bool LDS>
+__global__ __launch_bounds__(QR_THREADS) void k_qr_tall(FactorArgs fa)
+{
+    extern __shared__ double smem[];
+    const xh_factor_item it = fa.items[blockIdx.x];
+    const int m = it.m, n = it.n;
+    const int qc = static_cast<int>(it.s_off);
+    if(m == 0 || n == 0) return;
+    constexpr int G = 64, NG = QR_THREADS / G;
     const int kmax = min(m, n);
     double* Wk = work_base<LDS>(smem, fa);  // m x n working copy
-    double* tau = Wk + int64_t(m) * n;                                                      // kmax
-    const int tid = threadIdx.x;
-    for(int64_t e = tid; e < int64_t(m) * n; e += F_THREADS) Wk[e] = fa.A[it.a_off + e];
-    __syncthreads();
-    for(int k = 0; k < kmax; ++k) {
+    double* tau = Wk + int64_t(m) * n;      // kmax
+    const int tid = threadIdx.x, lane = tid % G, grp = tid / G;
+    for(int j = grp; j < n; j += NG)
+        for(int r = lane; r < m; r += G) Wk[int64_t(j) * m + r] = fa.A[it.a_off + int64_t(j) * m + r];
+    auto reflector = [&](int k) {  // from column k, whose rows this group's lanes wrote themselves
         double* col = Wk + int64_t(k) * m;
-        double part = 0.0;
-        for(int r = k + 1 + tid; r < m; r += F_THREADS) part = fma(col[r], col[r], part);
-        for(int o = 32; o > 0; o >>= 1) part += __shfl_xor(part, o);
-        if((tid & 63) == 0) red[tid >> 6] = part;
-        __syncthreads();
-        if(tid == 0) {
-            double tail = 0;
-            for(int w = 0; w < F_THREADS / 64; ++w) tail += red[w];
-            const double c0 = col[k];
-            double beta, t;
-            if(tail <= DBL_MIN) {
-                t = 0.0;
-                beta = c0;
-            } else {
-                beta = sqrt(c0 * c0 + tail);
-                if(c0 >= 0.0) beta = -beta;
-                t = (beta - c0) / beta;
-            }
-            s_beta = beta;
-            s_tau = t;
-            s_c0 = c0;
+        double tail = 0.0, c0 = 0.0;
+        for(int r = lane; r < m; r += G) {
+            const double y = col[r];
+            if(r > k) tail = fma(y, y, tail);
+            if(r == k) c0 = y;
         }
-        __syncthreads();
-        const double beta = s_beta, t = s_tau, c0 = s_c0;
-        if(t != 0.0) {
-            const double inv = 1.0 / (c0 - beta);
-            for(int r = k + 1 + tid; r < m; r += F_THREADS) col[r] *= inv;
+        tail = xh::lanes_sum<G>(tail);
+        c0 = xh::lanes_sum<G>(c0);
+        double beta, t, inv;
+        make_householder(c0, tail, beta, t, inv);
+        for(int r = lane; r < m; r += G)
+            if(r >= k) col[r] = r == k ? beta : col[r] * inv;
+        if(lane == 0) tau[k] = t;
+    };
+    auto apply = [&](int k, double t, double* c) {  // c -= tau (v^T c) v, v = [1; column k below k]
+        const double* col = Wk + int64_t(k) * m;
+        double w = 0.0;
+        for(int r = lane; r < m; r += G)
+            if(r >= k) w = fma(r == k ? 1.0 : col[r], c[r], w);
+        w = xh::lanes_sum<G>(w) * t;
+        for(int r = lane; r < m; r += G)
+            if(r >= k) c[r] = fma(-w, r == k ? 1.0 : col[r], c[r]);
+    };
+    if(grp == 0) reflector(0);
+    for(int k = 0; k < kmax; ++k) {
+        __syncthreads();  // reflector k is there
+        const double t = tau[k];
+        const int first = k + 1;
+        for(int j = first + ((grp - first) % NG + NG) % NG; j < n; j += NG) {
+            if(t != 0.0) apply(k, t, Wk + int64_t(j) * m);
+            if(j == first && first < kmax) reflector(first);
         }
-        __syncthreads();
-        if(tid == 0) {
-            col[k] = beta;
-            tau[k] = t;
-        }
-        // apply H = I - tau v v^T to the trailing columns, v = [1; col[k+1:]]
-        if(t != 0.0) {
-            for(int j = k + 1 + tid; j < n; j += F_THREADS) {
-                double* cj = Wk + int64_t(j) * m;
-                double w = cj[k];
-                for(int r = k + 1; r < m; ++r) w = fma(col[r], cj[r], w);
-                w *= t;
-                cj[k] -= w;
-                for(int r = k + 1; r < m; ++r) cj[r] = fma(-w, col[r], cj[r]);
-            }
-        }
-        __syncthreads();
     }
+    __syncthreads();
     // R: qc x n, upper triangle of the working copy (rows beyond min(m, n) are zero)
-    for(int64_t e = tid; e < int64_t(qc) * n; e += F_THREADS) {
+    for(int64_t e = tid; e < int64_t(qc) * n; e += QR_THREADS) {
         const int r = static_cast<int>(e % qc), c = static_cast<int>(e / qc);
         fa.Vt[it.vt_off + e] = (r < m && r <= c) ? Wk[r + int64_t(c) * m] : 0.0;
     }
-    // Q columns 0..qc-1: Q e_c = H_0 H_1 ... H_{kmax-1} e_c (zero for c >= m)
-    for(int c = tid; c < qc; c += F_THREADS) {
+    for(int c = grp; c < qc; c += NG) {
         double* qcol = fa.U + it.u_off + int64_t(c) * m;
-        for(int r = 0; r < m; ++r) qcol[r] = (r == c) ? 1.0 : 0.0;
-        if(c >= m) continue;
-        for(int k = kmax - 1; k >= 0; --k) {
-            const double t = tau[k];
-            if(t == 0.0) continue;
-            const double* v = Wk + int64_t(k) * m;
-            double w = qcol[k];
-            for(int r = k + 1; r < m; ++r) w = fma(v[r], qcol[r], w);
-            w *= t;
-            qcol[k] -= w;
-            for(int r = k + 1; r < m; ++r) qcol[r] = fma(-w, v[r], qcol[r]);
-        }
+        for(int r = lane; r < m; r += G) qcol[r] = (r == c) ? 1.0 : 0.0;
+        if(c < m)
+            for(int k = min(c, kmax - 1); k >= 0; --k)
+                if(tau[k] != 0.0) apply(k, tau[k], qcol);
     }
 }
 
@@ -776,10 +920,65 @@ extern "C" int xh_block_svd(xh_ctx* ctx, const xh_factor_item* items, int64_t ni
 
 extern "C" int xh_block_qr(xh_ctx* ctx, const xh_factor_item* items, int64_t nitems, const double* A, double* Q, double* R)
 {
+    // asynchronous: there is no status to read back, so no host synchronisation
     return guard(ctx, [&] {
-        std::vector<xh_factor_item> v(items, items + nitems);
-        run_factor(
-            ctx, k_qr<true>, k_qr<false>, v, [](const xh_factor_item& it) { return int64_t(it.m) * it.n + std::min(it.m, it.n) + 1; }, A, Q, nullptr, R);
+        const size_t budget = lds_budget(ctx);
+        // a kernel per range of rows, the narrowest that holds a block; its reflectors in LDS where
+        // they fit; from 1025 rows the kernel with a working copy
+        struct Class {
+            void (*kern)(FactorArgs);
+            int rows;  // most rows; 0: any
+            bool lds;
+            std::vector<xh_factor_item> v;
+            int64_t maxd;
+        };
+        Class cls[] = {{k_qr<true, 16, 4, 4>, 64, true, {}, 0},   {k_qr<true, 16, 8, 2>, 128, true, {}, 0},    {k_qr<true, 16, 12, 2>, 192, true, {}, 0},
+                       {k_qr<true, 16, 16, 1>, 256, true, {}, 0}, {k_qr<true, 64, 16, 1>, 1024, true, {}, 0},  {k_qr<false, 16, 16, 1>, 256, false, {}, 0},
+                       {k_qr<false, 64, 16, 1>, 1024, false, {}, 0}, {k_qr_tall<true>, 0, true, {}, 0},     {k_qr_tall<false>, 0, false, {}, 0}};
+        auto need = [&](const Class& c, const xh_factor_item& it) {
+            return c.rows ? qr_work_doubles(it.m, it.n, c.rows) : qr_tall_work_doubles(it.m, it.n);
+        };
+        auto fits = [&](const Class& c, const xh_factor_item& it) {
+            return (!c.rows || it.m <= c.rows) && (!c.lds || size_t(need(c, it)) * sizeof(double) <= budget);
+        };
+        for(int64_t i = 0; i < nitems; ++i) {
+            const xh_factor_item& it = items[i];
+            if(it.m < 0 || it.n < 0) throw xh::Error(XH_EINVAL, "factor: negative extent");
+            if(it.m == 0 || it.n == 0) continue;
+            for(Class& c : cls)
+                if(fits(c, it)) {
+                    c.v.push_back(it);
+                    break;
+                }
+        }
+        // one launch for the 16-lane classes where the widest of them can hold every block: a few
+        // blocks run beside each other on different CUs, and the largest sets the time either way
+        // (9 blocks of 31 to 132 rows: 174 + 109 + 21 us in three launches)
+        Class* wide = nullptr;
+        for(int c = 0; c < 4; ++c)
+            if(!cls[c].v.empty()) wide = &cls[c];
+        for(int c = 0; c < 4; ++c) {
+            if(&cls[c] == wide || cls[c].v.empty()) continue;
+            if(!std::all_of(cls[c].v.begin(), cls[c].v.end(), [&](const xh_factor_item& it) { return fits(*wide, it); })) continue;
+            wide->v.insert(wide->v.end(), cls[c].v.begin(), cls[c].v.end());
+            cls[c].v.clear();
+        }
+        for(Class& c : cls)
+            for(const auto& it : c.v) c.maxd = std::max(c.maxd, need(c, it));
+        for(Class& c : cls) {
+            if(c.v.empty()) continue;
+            xh_factor_item* d_items = xh::dev_upload(ctx, c.v);
+            double* scratch = nullptr;
+            if(!c.lds) check(xh::dmalloc(ctx, reinterpret_cast<void**>(&scratch), size_t(c.maxd) * c.v.size() * sizeof(double)), "hipMallocAsync");
+            FactorArgs fa{d_items, A, Q, nullptr, R, scratch, c.maxd, c.lds ? 1 : 0, nullptr};
+            const size_t shmem = c.lds ? size_t(c.maxd) * sizeof(double) : 0;
+            if(shmem > 64 * 1024)
+                check(hipFuncSetAttribute(reinterpret_cast<const void*>(c.kern), hipFuncAttributeMaxDynamicSharedMemorySize, int(shmem)), "hipFuncSetAttribute");
+            hipLaunchKernelGGL(c.kern, dim3(static_cast<unsigned>(c.v.size())), dim3(QR_THREADS), shmem, ctx->stream, fa);
+            xh::launch_check("k_qr");
+            xh::dev_free(ctx, d_items);
+            xh::dev_free(ctx, scratch);
+        }
     });
 }
 
