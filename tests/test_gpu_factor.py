@@ -74,3 +74,50 @@ def test_block_qr_across_kernel_edges(rt):
         live = np.abs(np.diag(lq)) > 1e-8 * np.linalg.norm(b)
         kk = np.flatnonzero(live)
         assert np.array_equal(np.sign(np.diag(rr)[kk]), np.sign(np.diag(lq)[kk])) or (m, n) == (33, 33), (m, n)
+
+
+def _svd_blocks():
+    r = np.random.default_rng(8)
+    out = [r.uniform(-1, 1, s) for s in
+           [(1, 1), (1, 9), (9, 1), (2, 2), (31, 32), (33, 32), (65, 31), (64, 64), (63, 64), (130, 33), (129, 64), (66, 65), (97, 97), (98, 98), (99, 99), (100, 96),
+            (300, 20), (1500, 9), (40, 400)]]
+    out.append(np.zeros((7, 5)))
+    out.append(np.ones((20, 20)))  # rank one, equal columns
+    out.append(np.diag(np.arange(12.0)))
+    out.append(1e-140 * r.uniform(-1, 1, (24, 24)))  # squares far below, but not under, the normal range
+    out.append(1e140 * r.uniform(-1, 1, (24, 24)))
+    out.append(r.uniform(-1, 1, (30, 30)) * np.logspace(0, -14, 30))
+    z = r.uniform(-1, 1, (20, 6))
+    z[:, 2] = 0.0
+    out.append(z)
+    return out
+
+
+@pytest.mark.parametrize("alone", [False, True], ids=["grouped", "alone"])
+def test_block_svd_across_kernel_edges(rt, alone):
+    """Single-workgroup Jacobi SVD at the rows and columns that pick its variant and its neighbour,
+    block Jacobi.  Singular values within sqrt(n) 1e-12 sigma_max of LAPACK's, reconstruction and
+    orthonormality likewise (the bounds of test_gpu_svd.py)."""
+    blocks = _svd_blocks()
+    for group in ([[b] for b in blocks] if alone else [blocks]):
+        items, ao, uo, so, vo = [], 0, 0, 0, 0
+        for b in group:
+            m, n = b.shape
+            k = min(m, n)
+            items.append(_lib.xh_factor_item(ao, uo, so, vo, m, n))
+            ao, uo, so, vo = ao + m * n, uo + m * k, so + k, vo + k * n
+        U, S, V = _run(rt, lib().xh_block_svd, group, (uo, so, vo), items)
+        for b, it in zip(group, items):
+            m, n = b.shape
+            k = min(m, n)
+            u = U[it.u_off:it.u_off + m * k].reshape(k, m).T
+            s = S[it.s_off:it.s_off + k]
+            v = V[it.vt_off:it.vt_off + k * n].reshape(n, k).T
+            ref = np.linalg.svd(b, compute_uv=False)
+            tol = 1e-12 * np.sqrt(k)
+            assert np.abs(s - ref).max() <= tol * ref[0], (m, n)
+            assert np.linalg.norm((u * s) @ v - b) <= tol * max(ref[0], 0.0), (m, n)
+            live = s > 1e-12 * ref[0]
+            e = np.eye(int(live.sum()))
+            assert np.abs(u[:, live].T @ u[:, live] - e).max(initial=0.0) <= tol, (m, n)
+            assert np.abs(v[live] @ v[live].T - e).max(initial=0.0) <= tol, (m, n)

@@ -20,6 +20,7 @@
 #include <cfloat>
 #include <cmath>
 #include <numeric>
+#include <utility>
 
 #include "device.hpp"
 
@@ -28,7 +29,7 @@ using xh::check;
 namespace {
 
 constexpr int BJ_W = 32;          // column block width; pairs are 64 columns wide
-constexpr int BJ_THREADS = 256;
+constexpr int BJ_THREADS = 1024;
 constexpr int BJ_MAX_SWEEPS = 60;
 constexpr int BJ_INNER_SWEEPS = 2;  // inexact pair solves: the outer sweeps finish the job
 
@@ -41,131 +42,197 @@ struct BjPair {
     double z;        // squared norm below which a column counts as numerically zero
 };
 
-__device__ __forceinline__ int bj_player(int pos, int step, int np)
-{
-    if(pos == 0) return 0;
-    return ((pos - 1 + step) % (np - 1)) + 1;
-}
+// Eigen-decomposition G = J diag(g) J^T of one pair's Gram matrix, eigenvalues descending: cyclic
+// two-sided Jacobi in LDS, at most BJ_INNER_SWEEPS sweeps of np - 1 steps (np = n2 rounded up to
+// even; a padding row and column of zeros never rotates).
+//
+// A step turns np / 2 disjoint planes at once and is bound by its latency and by LDS traffic.  The
+// rows of A are kept by position in the tournament, so that the plane of pair P is always that
+// of positions P and np - 1 - P; a step writes its result to the other of two buffers, every row
+// already at its position of the next step (q -> q - 1, 1 -> np - 1, 0 -> 0).  So the addresses a
+// thread reads and writes never change, and are computed once.  By symmetry only the 2 x 2 blocks
+// of pairs I < J are kept (row in I, column in J), one per thread, and the diagonal blocks apart.
+// V never touches LDS: half a wave holds two rows of it, lane k the entries at positions k and
+// np - 1 - k, so a rotation stays inside a lane and the move to the next step is a shift by one
+// lane (DPP).  Between two barriers one half wave turns the diagonal blocks into (c, s) while all
+// waves apply the rotations of the step before to V and fetch their blocks of A; between the next
+// two they turn the blocks.
+// (256 threads, each rotating columns, then rows, of a square A in place, with 16 lanes of a wave
+// on one bank in the row pass: 313 us per call at bond 701, up to two sweeps at n2 = 64; V in LDS
+// and the blocks of A as here 102 us; this takes 76 us.)
+constexpr int BJ_NMAX = 2 * BJ_W;
+constexpr int BJ_LD = BJ_NMAX;
+constexpr int BJ_BUF = BJ_NMAX * BJ_LD + 3 * BJ_W;  // one buffer: blocks, then app, aqq, apq per pair
+constexpr double BJ_FAR = 1e-16;  // squared cosine above which another sweep follows
+typedef double d2 __attribute__((ext_vector_type(2)));
 
-// Eigen-decomposition G = J diag(g) J^T of one pair's Gram matrix, eigenvalues descending.
 __global__ __launch_bounds__(BJ_THREADS) void k_bj_pair(const BjPair* __restrict__ pairs, const double* __restrict__ G, double* __restrict__ J,
                                                          int* __restrict__ flags)
 {
-    extern __shared__ double sm[];
-    __shared__ int need, rotated;
+    extern __shared__ __attribute__((aligned(16))) double sm[];
+    __shared__ int need, far;
+    __shared__ double s_diag[BJ_NMAX];
     const BjPair pr = pairs[blockIdx.x];
     const int n = pr.n2;
-    double* A = sm;
-    double* V = A + n * n;
-    double* cs = V + n * n;                          // n doubles: c, s per pair
-    int* pi = reinterpret_cast<int*>(cs + n + 2);     // n ints: i, j per pair
+    const int np = n + (n & 1), P = np / 2;
+    double* buf0 = sm;                                  // two buffers
+    d2* cs = reinterpret_cast<d2*>(buf0 + 2 * BJ_BUF);  // per pair, of an even and an odd step
+    int* rank = reinterpret_cast<int*>(cs + 2 * BJ_W);
     const int tid = threadIdx.x;
-    for(int e = tid; e < n * n; e += BJ_THREADS) {
-        const int i = e % n, j = e / n;
-        A[e] = (i >= j) ? G[pr.g + e] : G[pr.g + j + i * n];
-        V[e] = (i == j) ? 1.0 : 0.0;
-    }
-    if(tid == 0) need = 0;
+    const double* Gp = G + pr.g;
+    // offset of element (x, y) of A, by position, in a buffer: a block of pairs I < J, or the diagonal
+    auto pair_of = [&](int x) { return min(x, np - 1 - x); };
+    auto place = [&](int x, int y) {
+        const int a = pair_of(x), b = pair_of(y);
+        if(a != b) return a < b ? x * BJ_LD + y : y * BJ_LD + x;
+        return BJ_NMAX * BJ_LD + 3 * a + (x != y ? 2 : (x < P ? 0 : 1));
+    };
+    auto next = [&](int x) { return x == 0 ? 0 : x == 1 ? np - 1 : x - 1; };  // position after a step
+    if(tid == 0) need = far = 0;
+    if(tid < BJ_NMAX) s_diag[tid] = tid < n ? Gp[tid + tid * n] : 0.0;
     __syncthreads();
+    // scaled by a power of two to a largest diagonal entry of [1/2, 1): J does not change
+    double mx = fabs(s_diag[tid & 63]);
+    for(int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o));
+    int ex = 0;
+    if(mx > 0.0 && mx <= DBL_MAX) frexp(mx, &ex);
     // a computed inner product carries rounding noise of about sqrt(rows) eps relative to the
     // column norms, and the GEMM update of a pair adds about sqrt(n2) eps: pairs are orthogonal
     // once below a small multiple of both
-    const double tol = 8.0 * fmax(1.0, sqrt(static_cast<double>(pr.rows))) * sqrt(static_cast<double>(n)) * DBL_EPSILON;
-    for(int e = tid; e < n * n; e += BJ_THREADS) {
-        const int i = e % n, j = e / n;
-        if(i < j) {
-            const double aii = A[i + i * n], ajj = A[j + j * n], aij = A[i + j * n];
-            if(aii > pr.z && ajj > pr.z && fabs(aij) > tol * sqrt(aii) * sqrt(ajj)) need = 1;
+    const double tol2 = 64.0 * fmax(1, pr.rows) * double(n) * DBL_EPSILON * DBL_EPSILON;
+    const double z = ldexp(pr.z, -ex);
+    const int ti = tid & 63, tj = tid >> 6;  // row, and first column, of this thread's entries
+    for(int j = tj; j < np; j += BJ_THREADS / 64)
+        if(ti >= j && ti < np) {  // the lower triangle of G
+            const double g = ti < n ? ldexp(Gp[ti + j * n], -ex) : 0.0;
+            buf0[place(ti, j)] = g;
+            const double gi = ldexp(s_diag[ti], -ex), gj = ldexp(s_diag[j], -ex);
+            if(ti > j && gi > z && gj > z && g * g > tol2 * (gi * gj)) need = 1;
         }
-    }
     __syncthreads();
-    if(need) {
+    const int todo = need;
+    double* cur = buf0;
+    double* nxt = buf0 + BJ_BUF;
+    // rows vrow, vrow + 2, ... of V at positions vk and np - 1 - vk
+    constexpr int VR = BJ_NMAX * 32 / BJ_THREADS;
+    const int vk = tid & 31, vrow = (tid >> 6) * 2 * VR + ((tid >> 5) & 1);
+    double vt[VR], vb[VR];
+#pragma unroll
+    for(int q = 0; q < VR; ++q) {
+        vt[q] = vrow + 2 * q == vk ? 1.0 : 0.0;
+        vb[q] = vrow + 2 * q == np - 1 - vk ? 1.0 : 0.0;
+    }
+    if(todo) {
         if(tid == 0) atomicOr(flags + pr.sector, 1);
-        const int np = n + (n & 1), npairs = np / 2;
+        // this thread's block of pairs I < J: blocks of one I on consecutive lanes
+        const int nblk = P * (P - 1) / 2;
+        int I = 0, Jb = 0, rd[4] = {}, wr[4] = {};
+        if(tid < nblk) {
+            int t = tid;
+            while(t >= P - 1 - I) t -= P - 1 - I++;
+            Jb = I + 1 + t;
+            const int xi[2] = {I, np - 1 - I}, yj[2] = {Jb, np - 1 - Jb};
+            for(int k = 0; k < 4; ++k) {
+                rd[k] = place(xi[k >> 1], yj[k & 1]);
+                wr[k] = place(next(xi[k >> 1]), next(yj[k & 1]));
+            }
+        }
+        // the diagonal block of pair dg, on the last threads of the workgroup
+        const int dg = tid - (BJ_THREADS - P);
+        int dwr[3] = {};
+        if(dg >= 0) {
+            const int x = dg, y = np - 1 - dg;
+            dwr[0] = place(next(x), next(x));
+            dwr[1] = place(next(y), next(y));
+            dwr[2] = place(next(x), next(y));
+        }
+        // the rotations r of a step applied to V, and its entries moved to the next step's positions
+        auto turn_v = [&](const d2 r) {
+#pragma unroll
+            for(int q = 0; q < VR; ++q) {
+                const double t = r[0] * vt[q] - r[1] * vb[q], b = r[1] * vt[q] + r[0] * vb[q];
+                const double up = xh::dpp_mov<0x130>(t), down = xh::dpp_mov<0x138>(b);  // of lane vk + 1, of lane vk - 1
+                vt[q] = vk == 0 ? t : vk == P - 1 ? b : up;
+                vb[q] = vk == 0 ? (P > 1 ? up : b) : down;
+            }
+        };
+        d2* cs_now = cs;
+        d2* cs_last = cs + BJ_W;
         for(int sweep = 0; sweep < BJ_INNER_SWEEPS; ++sweep) {
-            if(tid == 0) rotated = 0;
-            __syncthreads();
             for(int step = 0; step < np - 1; ++step) {
-                for(int p = tid; p < npairs; p += BJ_THREADS) {
-                    int i = bj_player(p, step, np), j = bj_player(np - 1 - p, step, np);
-                    if(i > j) {
-                        const int t = i;
-                        i = j;
-                        j = t;
+                double app = 0, aqq = 0, apq = 0, c = 1.0, s = 0.0;
+                if(dg >= 0) {
+                    __builtin_amdgcn_s_setprio(3);  // everyone waits for these lanes
+                    const double* D = cur + BJ_NMAX * BJ_LD + 3 * dg;
+                    app = D[0];
+                    aqq = D[1];
+                    apq = D[2];
+                    const double q2 = apq * apq, pq = fabs(app * aqq);
+                    if(q2 > DBL_EPSILON * DBL_EPSILON * pq && q2 > 1e-280) {
+                        xh::jacobi_rotation(0.5 * (aqq - app), apq, c, s);
+                        if(q2 > BJ_FAR * pq) far = 1;
                     }
-                    double c = 1.0, s = 0.0;
-                    if(j < n) {
-                        const double apq = A[i + j * n], app = A[i + i * n], aqq = A[j + j * n];
-                        if(fabs(apq) > DBL_EPSILON * sqrt(fabs(app) * fabs(aqq)) && fabs(apq) > 1e-300) {
-                            const double theta = (aqq - app) / (2.0 * apq);
-                            const double t = copysign(1.0, theta) / (fabs(theta) + sqrt(theta * theta + 1.0));
-                            c = 1.0 / sqrt(t * t + 1.0);
-                            s = t * c;
-                            rotated = 1;
-                        }
-                    } else {
-                        i = -1;
-                    }
-                    cs[2 * p] = c;
-                    cs[2 * p + 1] = s;
-                    pi[2 * p] = i;
-                    pi[2 * p + 1] = j;
+                    cs_now[dg] = d2{c, s};
+                    __builtin_amdgcn_s_setprio(0);
                 }
+                double x[4];
+                if(tid < nblk)
+#pragma unroll
+                    for(int k = 0; k < 4; ++k) x[k] = cur[rd[k]];
+                if(step > 0) turn_v(cs_last[vk]);
                 __syncthreads();
-                // thread (p, q): pair p = tid / G with G = BJ_THREADS / npairs lanes per pair, rows
-                // (then columns) q, q + G, ...: no index division inside the loops
-                const int G = BJ_THREADS / npairs;
-                const int pp = tid / G, q0 = tid - pp * G;
-                int ri = -1, rj = 0;
-                double rc = 1.0, rs = 0.0;
-                if(pp < npairs) {
-                    ri = pi[2 * pp];
-                    rj = pi[2 * pp + 1];
-                    rc = cs[2 * pp];
-                    rs = cs[2 * pp + 1];
+                if(tid < nblk) {
+                    const d2 ci = cs_now[I], cj = cs_now[Jb];
+                    // rows by the rotation of I, then columns by that of J
+                    const double y0 = ci[0] * x[0] - ci[1] * x[2], y2 = ci[1] * x[0] + ci[0] * x[2];
+                    const double y1 = ci[0] * x[1] - ci[1] * x[3], y3 = ci[1] * x[1] + ci[0] * x[3];
+                    nxt[wr[0]] = cj[0] * y0 - cj[1] * y1;
+                    nxt[wr[1]] = cj[1] * y0 + cj[0] * y1;
+                    nxt[wr[2]] = cj[0] * y2 - cj[1] * y3;
+                    nxt[wr[3]] = cj[1] * y2 + cj[0] * y3;
                 }
-                const bool act = ri >= 0 && rs != 0.0;
-                if(act) {  // columns: A <- A R, V <- V R
-                    for(int r = q0; r < n; r += G) {
-                        double x = A[r + ri * n], y = A[r + rj * n];
-                        A[r + ri * n] = rc * x - rs * y;
-                        A[r + rj * n] = rs * x + rc * y;
-                        x = V[r + ri * n];
-                        y = V[r + rj * n];
-                        V[r + ri * n] = rc * x - rs * y;
-                        V[r + rj * n] = rs * x + rc * y;
-                    }
+                if(dg >= 0) {
+                    const double cc = c * c, ss = s * s, sc = s * c;
+                    nxt[dwr[0]] = cc * app - 2.0 * sc * apq + ss * aqq;
+                    nxt[dwr[1]] = ss * app + 2.0 * sc * apq + cc * aqq;
+                    nxt[dwr[2]] = sc * (app - aqq) + (cc - ss) * apq;
                 }
-                __syncthreads();
-                if(act) {  // rows: A <- R^T A
-                    for(int col = q0; col < n; col += G) {
-                        const double x = A[ri + col * n], y = A[rj + col * n];
-                        A[ri + col * n] = rc * x - rs * y;
-                        A[rj + col * n] = rs * x + rc * y;
-                    }
-                }
+                std::swap(cur, nxt);
+                std::swap(cs_now, cs_last);
                 __syncthreads();
             }
-            const int any = rotated;
+            turn_v(cs_last[vk]);
+            const int again = far;
             __syncthreads();
-            if(!any) break;
+            if(!again) break;
+            if(tid == 0) far = 0;
+            __syncthreads();
         }
     }
-    // descending eigenvalues (NaN last), ties by index; J columns in that order
-    for(int j = tid; j < n; j += BJ_THREADS) {
-        const double vj = A[j + j * n] == A[j + j * n] ? A[j + j * n] : -2.0 * DBL_MAX;
-        int rank = 0;
-        for(int k = 0; k < n; ++k) {
-            const double vk = A[k + k * n] == A[k + k * n] ? A[k + k * n] : -2.0 * DBL_MAX;
-            rank += (vk > vj) || (vk == vj && k < j);
+    // descending eigenvalues (NaN last), ties by index; J columns in that order.  A sweep ends with
+    // every row back at its own position.
+    if(tid < n) {
+        const double v = cur[place(tid, tid)];
+        s_diag[tid] = v == v ? v : -2.0 * DBL_MAX;
+    }
+    // V by columns through the buffer that is free
+#pragma unroll
+    for(int q = 0; q < VR; ++q)
+        if(vk < P && vrow + 2 * q < np) {
+            nxt[vk * BJ_LD + vrow + 2 * q] = vt[q];
+            nxt[(np - 1 - vk) * BJ_LD + vrow + 2 * q] = vb[q];
         }
-        pi[rank] = j;
+    __syncthreads();
+    for(int j = tid >> 4; j < n; j += BJ_THREADS / 16) {  // 16 lanes count the values above value j
+        const double vj = s_diag[j];
+        int r = 0;
+        for(int k = tid & 15; k < n; k += 16) r += (s_diag[k] > vj) || (s_diag[k] == vj && k < j);
+        for(int o = 8; o > 0; o >>= 1) r += __shfl_xor(r, o);
+        if((tid & 15) == 0) rank[r] = j;
     }
     __syncthreads();
-    for(int e = tid; e < n * n; e += BJ_THREADS) {
-        const int r = e % n, c = e / n;
-        J[pr.g + e] = need ? V[r + pi[c] * n] : (r == c ? 1.0 : 0.0);
-    }
+    for(int c = tj; c < n; c += BJ_THREADS / 64)
+        if(ti < n) J[pr.g + ti + c * n] = todo ? nxt[ti + rank[c] * BJ_LD] : (ti == c ? 1.0 : 0.0);
 }
 
 __global__ void k_set_ones(const int64_t* __restrict__ pos, int64_t n, double* __restrict__ x)
@@ -379,7 +446,7 @@ void block_jacobi_svd(xh_ctx* ctx, const std::vector<xh_factor_item>& items, con
         hipLaunchKernelGGL(k_set_ones, dim3(static_cast<unsigned>(std::min<int64_t>((ones.size() + 255) / 256, 65535))), dim3(256), 0, ctx->stream, d_ones,
                            static_cast<int64_t>(ones.size()), buf[0]);
         xh::launch_check("k_set_ones");
-        const size_t pair_lds = size_t(2 * 2 * BJ_W * 2 * BJ_W + 2 * 2 * BJ_W + 4) * sizeof(double);
+        const size_t pair_lds = size_t(2 * BJ_BUF + 4 * BJ_W + BJ_NMAX / 2) * sizeof(double);
         check(hipFuncSetAttribute(reinterpret_cast<const void*>(k_bj_pair), hipFuncAttributeMaxDynamicSharedMemorySize, int(pair_lds)), "hipFuncSetAttribute");
         int cur = 0;
         int64_t gcap = 0;

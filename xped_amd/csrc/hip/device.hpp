@@ -190,8 +190,8 @@ __device__ __forceinline__ uint32_t fdiv(uint32_t x, uint32_t magic, uint32_t sh
 template <int CTRL>
 __device__ __forceinline__ double dpp_mov(double x)
 {
-    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, 0xf, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, 0xf, 0xf, false);
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, 0xf, 0xf, true);
     return __hiloint2double(hi, lo);
 }
 template <int G>
@@ -207,6 +207,25 @@ __device__ __forceinline__ double lanes_sum(double x)
         x += __shfl_xor(x, 32);
     }
     return x;
+}
+
+// Rotation (c, s) by the smaller angle that makes two columns orthogonal, d half the difference of
+// their squared norms (second minus first) and ga != 0 their inner product.  The tangent t comes
+// from the hardware's estimates (22 bits): it only steers convergence.  What must be exact is
+// c^2 + s^2 = 1, and without a bias, which thousands of rotations would add up: c and s are taken
+// from w ~ tan(angle / 2), s = 2 w / (1 + w^2) to one rounding and c = 1 - w s.  (c = 1 / sqrt(1 + t^2)
+// with IEEE operations is 1.1e-16 too long on average for t from 1e-8 to 1e-4: the factors of a
+// 390 x 390 block then left norm 1 by 1.2e-13.)
+__device__ __forceinline__ void jacobi_rotation(double d, double ga, double& c, double& s)
+{
+    const double h = fma(d, d, ga * ga);
+    double t = fabs(ga) * __builtin_amdgcn_rcp(fma(h, __builtin_amdgcn_rsq(h), fabs(d)));
+    t = (signbit(d) != signbit(ga)) ? -t : t;
+    const double r = __builtin_amdgcn_rsq(fma(t, t, 1.0));
+    const double w = t * r * __builtin_amdgcn_rcp(1.0 + r);
+    const double z = fma(w, w, 1.0), y = __builtin_amdgcn_rcp(z), e = fma(-z, y, 1.0);
+    s = 2.0 * w * fma(y, fma(e, e, e), y);
+    c = fma(-w, s, 1.0);
 }
 
 // One output leg of a permute task (shared by the permute kernels and the GEMM that reads its A

@@ -11,7 +11,7 @@
 #include <algorithm>
 #include <cfloat>
 #include <cstring>
-
+#include <iterator>
 
 #include "device.hpp"
 
@@ -23,17 +23,12 @@ namespace {
 constexpr int F_THREADS = 256;
 constexpr int MAX_SWEEPS = 60;
 
-__device__ __forceinline__ double group_sum(double v, int g)
-{
-    for(int o = g >> 1; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    return v;
-}
-
 __device__ __forceinline__ int rr_player(int pos, int step, int n2)
 {
-    // circle method: position 0 is fixed, the others rotate by one each step
+    // circle method: position 0 is fixed, the others rotate by one each step (step < n2 - 1)
     if(pos == 0) return 0;
-    return ((pos - 1 + step) % (n2 - 1)) + 1;
+    const int q = pos + step;
+    return q >= n2 ? q - (n2 - 1) : q;
 }
 
 // total orders over doubles for rank-based sorting: NaN below (above) every number
@@ -64,113 +59,226 @@ __device__ __forceinline__ double* work_base(double* smem, const FactorArgs& fa)
         return fa.scratch + int64_t(blockIdx.x) * fa.scratch_stride;
 }
 
-// Working set of the Jacobi SVD for a block of mm x nn (mm >= nn):
-//   W (mm*nn), V (nn*nn), sigma (nn), order (nn ints)
-__host__ __device__ inline int64_t svd_work_doubles(int64_t mm, int64_t nn) { return mm * nn + nn * nn + nn + (nn + 1) / 2 + 2; }
+// One-sided Jacobi SVD of a block worked on as mm x nn (mm >= nn, transposed where needed), one
+// workgroup per block.  Working set in LDS: W (nn columns of ldw), V (nn columns of ldv), sigma
+// (nn), order (nn ints).
+//
+// The kernel is a serial chain of (nn - 1) steps per sweep, each the latency of one rotation: the
+// columns of a pair read from LDS, an inner product, the angle, the update, a barrier.  So 16
+// lanes own a pair (two rows each per 16-byte LDS access) and reduce by DPP; the columns of W stay
+// in registers between the inner product and the update (RM > 0: rows <= 32 RM; RM = 0: any
+// number, read twice); V is read only when the pair rotates.  Squared column norms are kept beside
+// W, moved with each rotation, summed afresh where a rotation takes most of a
+// column away and for every column before each sweep, so the last sweep, which finds every pair
+// orthogonal, judges by fresh norms.  The block is scaled by a power of two to a largest entry of
+// [1/2, 1), so that squares and their products stay in range.
+// (64 to 8 lanes per pair, three reductions through ds_bpermute, IEEE divisions and square roots
+// took 542 us for the 9 blocks, 32 x 32 the largest, of a two-site tensor at bond 64; three DPP
+// reductions and refined quotients 220 us; this takes 184 us.)
+constexpr int SVD_THREADS = 1024;
 
-template <bool LDS>
-__global__ __launch_bounds__(F_THREADS) void k_svd_jacobi(FactorArgs fa)
+__host__ __device__ inline int svd_ld(int rows) { return (rows + 1) & ~1; }
+__host__ __device__ inline int64_t svd_work_doubles(int64_t mm, int64_t nn)
 {
-    extern __shared__ double smem[];
-    __shared__ int rotated;
+    return nn * (svd_ld(int(mm)) + svd_ld(int(nn))) + nn + (nn + 1) / 2 + 2;
+}
+
+typedef double d2 __attribute__((ext_vector_type(2)));
+
+constexpr double SVD_TINY = 1e-135;  // squared norm of a column taken as zero (largest entry scaled to 1)
+
+constexpr double SVD_NEAR = 1e-14;    // squared cosine below which a sweep counts as nearly converged
+
+template <int RM, int VM>
+__global__ __launch_bounds__(SVD_THREADS) void k_svd_jacobi(FactorArgs fa)
+{
+    extern __shared__ __attribute__((aligned(16))) double smem[];
+    __shared__ int rotated, far;  // a pair was rotated this sweep; one by more than SVD_NEAR
+    __shared__ double s_max[SVD_THREADS / 64];
     const xh_factor_item it = fa.items[blockIdx.x];
     const int m = it.m, n = it.n;
     if(m == 0 || n == 0) return;
     const bool tr = m < n;
     const int mm = tr ? n : m, nn = tr ? m : n;
-    double* W = work_base<LDS>(smem, fa);
-    double* V = W + int64_t(mm) * nn;
-    double* sig = V + int64_t(nn) * nn;
+    const int ldw = svd_ld(mm), ldv = svd_ld(nn);
+    double* W = smem;
+    double* V = W + int64_t(ldw) * nn;
+    double* sig = V + int64_t(ldv) * nn;
     int* ord = reinterpret_cast<int*>(sig + nn);
-    const int tid = threadIdx.x;
-    for(int64_t e = tid; e < int64_t(mm) * nn; e += F_THREADS) {
-        const int i = static_cast<int>(e % mm), j = static_cast<int>(e / mm);
-        W[e] = tr ? fa.A[it.a_off + j + int64_t(i) * m] : fa.A[it.a_off + i + int64_t(j) * m];
+    constexpr int G = 16, RR = RM > 0 ? RM : 1;
+    const int tid = threadIdx.x, gl = tid % G, grp = tid / G, ngroups = blockDim.x / G;
+    double mx = 0.0;
+    for(int j = grp; j < nn; j += ngroups) {
+        for(int i = gl; i < ldw; i += G) {
+            const double v = i >= mm ? 0.0 : tr ? fa.A[it.a_off + j + int64_t(i) * m] : fa.A[it.a_off + i + int64_t(j) * m];
+            W[j * ldw + i] = v;
+            mx = fmax(mx, fabs(v));
+        }
+        for(int i = gl; i < ldv; i += G) V[j * ldv + i] = i == j ? 1.0 : 0.0;
     }
-    for(int64_t e = tid; e < int64_t(nn) * nn; e += F_THREADS) V[e] = ((e % nn) == (e / nn)) ? 1.0 : 0.0;
+    for(int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o));
+    if((tid & 63) == 0) s_max[tid >> 6] = mx;
     __syncthreads();
+    int ex = 0;
+    for(int w = 0; w < int(blockDim.x >> 6); ++w) mx = fmax(mx, s_max[w]);
+    if(mx > 0.0 && mx <= DBL_MAX) frexp(mx, &ex);
 
     const int n2 = nn + (nn & 1);
     const int npairs = n2 / 2;
-    int g = 64;
-    while(g > 8 && g * npairs > F_THREADS) g >>= 1;
-    const int ngroups = F_THREADS / g;
-    const int grp = tid / g, gl = tid % g;
-    const double tol = fmax(1.0, sqrt(static_cast<double>(mm))) * DBL_EPSILON;
+    const double tol = fmax(1.0, sqrt(static_cast<double>(mm))) * DBL_EPSILON, tol2 = tol * tol;
+    const int nw = (ldw >> 1) - gl, nv = (ldv >> 1) - gl;  // this lane's row pairs: 0, G, 2 G, ... below these
+    auto norm2 = [&](int j) {
+        double s = 0.0;
+        const d2* w = reinterpret_cast<const d2*>(W + j * ldw) + gl;
+        for(int k = 0; k < nw; k += G) {
+            const d2 a = w[k];
+            s = fma(a[0], a[0], s);
+            s = fma(a[1], a[1], s);
+        }
+        return xh::lanes_sum<G>(s);
+    };
+    for(int j = grp; j < nn; j += ngroups)
+        for(int i = gl; i < ldw; i += G) W[j * ldw + i] = ldexp(W[j * ldw + i], -ex);
+    // the pair of positions (grp, n2 - 1 - grp) of the circle: position 0 keeps its column, the
+    // others move on by one each step and are back after the n2 - 1 steps of a sweep
+    int a = grp, b = n2 - 1 - grp;
     int sweep = 0;
     if(nn > 1) {
         for(sweep = 0; sweep < MAX_SWEEPS; ++sweep) {
-            if(tid == 0) rotated = 0;
+            __syncthreads();
+            for(int j = grp; j < nn; j += ngroups) {
+                const double s = norm2(j);
+                if(gl == 0) sig[j] = s;
+            }
+            if(tid == 0) rotated = far = 0;
             __syncthreads();
             for(int step = 0; step < n2 - 1; ++step) {
-                for(int pbase = 0; pbase < npairs; pbase += ngroups) {
-                    const int p = pbase + grp;
-                    int i = -1, j = -1;
-                    if(p < npairs) {
-                        i = rr_player(p, step, n2);
-                        j = rr_player(n2 - 1 - p, step, n2);
-                        if(i > j) {
-                            int t = i;
-                            i = j;
-                            j = t;
+                if(grp < npairs && max(a, b) < nn) {  // a dummy column fills an odd count
+                    d2* wi = reinterpret_cast<d2*>(W + __mul24(a, ldw)) + gl;
+                    d2* wj = reinterpret_cast<d2*>(W + __mul24(b, ldw)) + gl;
+                    const double al = sig[a], be = sig[b];
+                    d2 x[RR], y[RR];
+                    double ga = 0;
+                    if constexpr(RM > 0) {
+#pragma unroll
+                        for(int k = 0; k < RM; ++k) {
+                            x[k] = d2{0.0, 0.0};
+                            y[k] = d2{0.0, 0.0};
+                            if(k * G < nw) {
+                                x[k] = wi[k * G];
+                                y[k] = wj[k * G];
+                            }
                         }
-                        if(j >= nn) i = -1;
+#pragma unroll
+                        for(int k = 0; k < RM; ++k) {
+                            ga = fma(x[k][0], y[k][0], ga);
+                            ga = fma(x[k][1], y[k][1], ga);
+                        }
+                    } else {
+                        for(int k = 0; k < nw; k += G) {
+                            const d2 p = wi[k], q = wj[k];
+                            ga = fma(p[0], q[0], ga);
+                            ga = fma(p[1], q[1], ga);
+                        }
                     }
-                    double al = 0, be = 0, ga = 0;
-                    if(i >= 0) {
-                        const double* wi = W + int64_t(i) * mm;
-                        const double* wj = W + int64_t(j) * mm;
-                        for(int r = gl; r < mm; r += g) {
-                            const double x = wi[r], y = wj[r];
-                            al = fma(x, x, al);
-                            be = fma(y, y, be);
-                            ga = fma(x, y, ga);
+                    ga = xh::lanes_sum<G>(ga);
+                    if(fmin(al, be) > SVD_TINY && ga * ga > tol2 * (al * be)) {
+                        d2* vi = reinterpret_cast<d2*>(V + __mul24(a, ldv)) + gl;
+                        d2* vj = reinterpret_cast<d2*>(V + __mul24(b, ldv)) + gl;
+                        d2 u[VM], v[VM];
+#pragma unroll
+                        for(int k = 0; k < VM; ++k)
+                            if(k * G < nv) {
+                                u[k] = vi[k * G];
+                                v[k] = vj[k * G];
+                            }
+                        double c, s;
+                        xh::jacobi_rotation(0.5 * (be - al), ga, c, s);
+                        if constexpr(RM > 0) {
+#pragma unroll
+                            for(int k = 0; k < RM; ++k) {
+                                const d2 p = x[k];
+                                x[k] = c * p - s * y[k];
+                                y[k] = s * p + c * y[k];
+                                if(k * G < nw) {
+                                    wi[k * G] = x[k];
+                                    wj[k * G] = y[k];
+                                }
+                            }
+                        } else {
+                            for(int k = 0; k < nw; k += G) {
+                                const d2 p = wi[k], q = wj[k];
+                                wi[k] = c * p - s * q;
+                                wj[k] = s * p + c * q;
+                            }
                         }
-                    }
-                    al = group_sum(al, g);
-                    be = group_sum(be, g);
-                    ga = group_sum(ga, g);
-                    if(i >= 0 && al > 0.0 && be > 0.0 && fabs(ga) > tol * sqrt(al) * sqrt(be)) {
-                        const double zeta = (be - al) / (2.0 * ga);
-                        const double t = copysign(1.0, zeta) / (fabs(zeta) + sqrt(1.0 + zeta * zeta));
-                        const double c = 1.0 / sqrt(1.0 + t * t);
-                        const double s = c * t;
-                        double* wi = W + int64_t(i) * mm;
-                        double* wj = W + int64_t(j) * mm;
-                        for(int r = gl; r < mm; r += g) {
-                            const double x = wi[r], y = wj[r];
-                            wi[r] = c * x - s * y;
-                            wj[r] = s * x + c * y;
+#pragma unroll
+                        for(int k = 0; k < VM; ++k)
+                            if(k * G < nv) {
+                                vi[k * G] = c * u[k] - s * v[k];
+                                vj[k * G] = s * u[k] + c * v[k];
+                            }
+                        const double g2 = 2.0 * s * c * ga;
+                        double na = fma(c * c, al, fma(s * s, be, -g2)), nb = fma(s * s, al, fma(c * c, be, g2));
+                        if(fmin(na, nb) < 1e-3 * fmin(al, be)) {  // cancellation (rare): sum afresh
+                            na = norm2(a);
+                            nb = norm2(b);
                         }
-                        double* vi = V + int64_t(i) * nn;
-                        double* vj = V + int64_t(j) * nn;
-                        for(int r = gl; r < nn; r += g) {
-                            const double x = vi[r], y = vj[r];
-                            vi[r] = c * x - s * y;
-                            vj[r] = s * x + c * y;
+                        if(gl == 0) {
+                            sig[a] = na;
+                            sig[b] = nb;
+                            rotated = 1;
+                            if(ga * ga > SVD_NEAR * (al * be)) far = 1;
                         }
-                        if(gl == 0) rotated = 1;
                     }
                 }
+                if(grp != 0) a = a == n2 - 1 ? 1 : a + 1;
+                b = b == n2 - 1 ? 1 : b + 1;
                 __syncthreads();
             }
-            const int any = rotated;
-            __syncthreads();
-            if(!any) break;
+            if(!rotated) break;
+            // Every angle of this sweep was small, so the next one will most likely find all pairs
+            // orthogonal: test them all at once, without the steps' barriers (same test).
+            if(!far) {
+                for(int j = grp; j < nn; j += ngroups) {
+                    const double s = norm2(j);
+                    if(gl == 0) sig[j] = s;
+                }
+                __syncthreads();
+                if(tid == 0) rotated = 0;
+                __syncthreads();
+                for(int i = grp; i < nn; i += ngroups)
+                    for(int d = 1; d <= nn / 2; ++d) {
+                        const int j = i + d < nn ? i + d : i + d - nn;
+                        const d2* wi = reinterpret_cast<const d2*>(W + i * ldw) + gl;
+                        const d2* wj = reinterpret_cast<const d2*>(W + j * ldw) + gl;
+                        double ga = 0.0;
+                        for(int k = 0; k < nw; k += G) {
+                            const d2 p = wi[k], q = wj[k];
+                            ga = fma(p[0], q[0], ga);
+                            ga = fma(p[1], q[1], ga);
+                        }
+                        ga = xh::lanes_sum<G>(ga);
+                        if(gl == 0 && fmin(sig[i], sig[j]) > SVD_TINY && ga * ga > tol2 * (sig[i] * sig[j])) rotated = 1;
+                    }
+                __syncthreads();
+                if(!rotated) break;
+            }
         }
     }
     if(sweep >= MAX_SWEEPS && tid == 0) atomicExch(fa.status, XH_ENOTCONV);
     // column norms
-    for(int j = tid; j < nn; j += F_THREADS) {
-        const double* wj = W + int64_t(j) * mm;
+    for(int j = grp; j < nn; j += ngroups) {
+        const double* wj = W + j * ldw;
         double s = 0;
-        for(int r = 0; r < mm; ++r) s = fma(wj[r], wj[r], s);
-        sig[j] = sqrt(s);
+        for(int r = gl; r < mm; r += G) s = fma(wj[r], wj[r], s);
+        s = xh::lanes_sum<G>(s);
+        if(gl == 0) sig[j] = sqrt(s);  // of the scaled block
     }
     __syncthreads();
     // descending order, ties broken by column index; NaN (from non-finite input) sorts last so
     // that the ranks stay a permutation of 0..nn-1 for any input
-    for(int j = tid; j < nn; j += F_THREADS) {
+    for(int j = tid; j < nn; j += blockDim.x) {
         const double sj = nan_low(sig[j]);
         int rank = 0;
         for(int k = 0; k < nn; ++k) {
@@ -180,31 +288,25 @@ __global__ __launch_bounds__(F_THREADS) void k_svd_jacobi(FactorArgs fa)
         ord[rank] = j;
     }
     __syncthreads();
-    for(int r = tid; r < nn; r += F_THREADS) fa.S[it.s_off + r] = sig[ord[r]];
-    // U (m x nn) and Vt (nn x n)
-    for(int64_t e = tid; e < int64_t(m) * nn; e += F_THREADS) {
-        const int i = static_cast<int>(e % m), r = static_cast<int>(e / m);
+    for(int r = tid; r < nn; r += blockDim.x) fa.S[it.s_off + r] = ldexp(sig[ord[r]], ex);
+    // U (m x nn) and Vt (nn x n): W / sigma on the long side, V on the other
+    for(int r = grp; r < nn; r += ngroups) {
         const int c = ord[r];
-        double v;
-        if(!tr) {
-            const double s = sig[c];
-            v = s > 0.0 ? W[i + int64_t(c) * mm] / s : 0.0;
-        } else {
-            v = V[i + int64_t(c) * nn];
+        const double s = sig[c];
+        for(int i = gl; i < mm; i += G) {
+            const double v = s > 0.0 ? W[i + c * ldw] / s : 0.0;
+            if(!tr)
+                fa.U[it.u_off + i + int64_t(r) * m] = v;
+            else
+                fa.Vt[it.vt_off + r + int64_t(i) * nn] = v;
         }
-        fa.U[it.u_off + e] = v;
-    }
-    for(int64_t e = tid; e < int64_t(nn) * n; e += F_THREADS) {
-        const int r = static_cast<int>(e % nn), col = static_cast<int>(e / nn);
-        const int c = ord[r];
-        double v;
-        if(!tr) {
-            v = V[col + int64_t(c) * nn];
-        } else {
-            const double s = sig[c];
-            v = s > 0.0 ? W[col + int64_t(c) * mm] / s : 0.0;
+        for(int i = gl; i < nn; i += G) {
+            const double v = V[i + c * ldv];
+            if(!tr)
+                fa.Vt[it.vt_off + r + int64_t(i) * nn] = v;
+            else
+                fa.U[it.u_off + i + int64_t(r) * m] = v;
         }
-        fa.Vt[it.vt_off + e] = v;
     }
 }
 
@@ -889,8 +991,55 @@ void run_factor(xh_ctx* ctx, void (*kern_lds)(FactorArgs), void (*kern_global)(F
 
 }  // namespace
 
-// blocks with more columns than this (after transposition) use the block Jacobi path
-constexpr int BJ_MIN_COLS = 64;
+// Blocks with more columns than this (after transposition) use the block Jacobi path: any block of
+// a call where some block has to (a block of 65 to 98 columns then adds nothing to steps that run
+// anyway, but 1.4 ms by itself), and only those that do not fit LDS in a call of smaller blocks
+// (15 sectors of up to 74 columns: 0.46 ms by themselves, 1.07 ms with block Jacobi and its products).
+constexpr int BJ_MIN_COLS = 64, BJ_MIN_COLS_ALONE = 98;
+
+namespace {
+// The single-workgroup Jacobi kernel on blocks whose working set fits LDS: one launch, in the
+// variant of the tallest and widest block.  The singular values are read back by every caller, so
+// the convergence status waits with them.
+void small_svd(xh_ctx* ctx, const std::vector<xh_factor_item>& v, const double* A, double* U, double* S, double* Vt)
+{
+    if(v.empty()) return;
+    int mm = 0, nn = 0;
+    int64_t maxd = 0;
+    for(const auto& it : v) {
+        const int a = std::max(it.m, it.n), b = std::min(it.m, it.n);
+        mm = std::max(mm, a);
+        nn = std::max(nn, b);
+        maxd = std::max(maxd, svd_work_doubles(a, b));
+    }
+    void (*kern)(FactorArgs) = nullptr;
+    if(nn <= 32)
+        kern = mm <= 32 ? k_svd_jacobi<1, 1> : mm <= 64 ? k_svd_jacobi<2, 1> : mm <= 128 ? k_svd_jacobi<4, 1> : k_svd_jacobi<0, 1>;
+    else if(nn <= 64)
+        kern = mm <= 64 ? k_svd_jacobi<2, 2> : mm <= 128 ? k_svd_jacobi<4, 2> : k_svd_jacobi<0, 2>;
+    else
+        kern = mm <= 128 ? k_svd_jacobi<4, 4> : k_svd_jacobi<0, 4>;
+    static_assert(BJ_MIN_COLS_ALONE <= 128, "k_svd_jacobi's V rows");
+    const int npairs = (nn + 1) / 2;
+    const int threads = std::min(SVD_THREADS, (npairs * 16 + 63) / 64 * 64);
+    int* d_status = nullptr;
+    check(xh::dmalloc(ctx, reinterpret_cast<void**>(&d_status), sizeof(int)), "hipMallocAsync");
+    check(hipMemsetAsync(d_status, 0, sizeof(int), ctx->stream), "hipMemsetAsync");
+    xh_factor_item* d_items = xh::dev_upload(ctx, v);
+    FactorArgs fa{d_items, A, U, S, Vt, nullptr, 0, 1, d_status};
+    const size_t shmem = size_t(maxd) * sizeof(double);
+    if(shmem > 64 * 1024)
+        check(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, int(shmem)), "hipFuncSetAttribute");
+    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(v.size())), dim3(threads), shmem, ctx->stream, fa);
+    xh::launch_check("k_svd_jacobi");
+    int status = 0;
+    check(hipMemcpyAsync(&status, d_status, sizeof(int), hipMemcpyDeviceToHost, ctx->stream), "hipMemcpyAsync");
+    check(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
+    xh::dev_free(ctx, d_items);
+    xh::dev_free(ctx, d_status);
+    if(status != 0) throw xh::Error(XH_ENOTCONV, "Jacobi iteration did not converge within the sweep limit");
+}
+}  // namespace
 
 extern "C" int xh_block_svd(xh_ctx* ctx, const xh_factor_item* items, int64_t nitems, const double* A, double* U, double* S, double* Vt)
 {
@@ -902,19 +1051,18 @@ extern "C" int xh_block_svd(xh_ctx* ctx, const xh_factor_item* items, int64_t ni
             const xh_factor_item& it = items[i];
             if(it.m <= 0 || it.n <= 0) continue;
             const int mn = std::min(it.m, it.n), mx = std::max(it.m, it.n);
-            if(mn > BJ_MIN_COLS || size_t(svd_work_doubles(mx, mn)) * sizeof(double) > budget)
+            if(mn > BJ_MIN_COLS_ALONE || size_t(svd_work_doubles(mx, mn)) * sizeof(double) > budget)
                 big.push_back(it);
             else
                 v.push_back(it);
         }
+        if(!big.empty()) {
+            auto wide = [](const xh_factor_item& it) { return std::min(it.m, it.n) > BJ_MIN_COLS; };
+            std::copy_if(v.begin(), v.end(), std::back_inserter(big), wide);
+            v.erase(std::remove_if(v.begin(), v.end(), wide), v.end());
+        }
         block_jacobi_svd(ctx, big, A, U, S, Vt);
-        run_factor(
-            ctx, k_svd_jacobi<true>, k_svd_jacobi<false>, v,
-            [](const xh_factor_item& it) {
-                const int64_t mm = std::max(it.m, it.n), nn = std::min(it.m, it.n);
-                return svd_work_doubles(mm, nn);
-            },
-            A, U, S, Vt);
+        small_svd(ctx, v, A, U, S, Vt);
     });
 }
 
