@@ -121,3 +121,37 @@ def test_block_svd_across_kernel_edges(rt, alone):
             e = np.eye(int(live.sum()))
             assert np.abs(u[:, live].T @ u[:, live] - e).max(initial=0.0) <= tol, (m, n)
             assert np.abs(v[live] @ v[live].T - e).max(initial=0.0) <= tol, (m, n)
+
+
+def test_block_chol_inv_across_kernel_edges(rt):
+    """X = R^-1 of Gram blocks G = R^T R around the 16-wide tiles and the largest block in LDS (192),
+    well and badly conditioned.  X is upper triangular, and X^T G X = I up to n eps times the
+    condition number of G (forward error of a Cholesky factor, Higham, theorem 10.3 and 14.1); the
+    same bound with the constant 4 holds numpy's factor inverted by substitution."""
+    r = np.random.default_rng(9)
+    blocks, conds = [], []
+    for n in (1, 2, 15, 16, 17, 31, 33, 48, 74, 100, 176, 177, 191, 192, 193, 208, 257, 300):
+        for logc in (0.5, 4.0):
+            q = np.linalg.qr(r.standard_normal((n, n)))[0]
+            G = (q * np.logspace(0, -2 * logc, n)) @ q.T
+            blocks.append(0.5 * (G + G.T))
+            conds.append(10.0 ** (2 * logc))
+    items, ao = [], 0
+    for b in blocks:
+        items.append(_lib.xh_factor_item(ao, ao, 0, 0, b.shape[0], b.shape[0]))
+        ao += b.size
+    shift = (C.c_double * len(blocks))(*([0.0] * len(blocks)))
+    X, = _run(rt, lambda ctx, arr, k, dA, dX: lib().xh_block_chol_inv(ctx, arr, k, dA, dX, shift), blocks, (ao,), items)
+    for b, it, c in zip(blocks, items, conds):
+        n = b.shape[0]
+        x = X[it.u_off:it.u_off + n * n].reshape(n, n).T
+        assert np.array_equal(x, np.triu(x)), n
+        assert np.linalg.norm(x.T @ b @ x - np.eye(n)) <= 4.0 * n * EPS * c, (n, c)
+    # a shift of 0.5 trace / n on the diagonal
+    b = blocks[17]
+    n = b.shape[0]
+    rel = (C.c_double * 1)(0.5 / n)
+    x, = _run(rt, lambda ctx, arr, k, dA, dX: lib().xh_block_chol_inv(ctx, arr, k, dA, dX, rel), [b], (n * n,), [_lib.xh_factor_item(0, 0, 0, 0, n, n)])
+    x = x.reshape(n, n).T
+    g = b + 0.5 * np.trace(b) / n * np.eye(n)
+    assert np.linalg.norm(x.T @ g @ x - np.eye(n)) <= 4.0 * n * EPS * np.linalg.cond(g)

@@ -553,266 +553,236 @@ __global__ __launch_bounds__(QR_THREADS) void k_qr_tall(FactorArgs fa)
 // column's original diagonal marks a numerically dependent column: its row and column of X are
 // zero, so Y X has a zero column there.
 //
-// One workgroup per block, one barrier per pivot.  The upper triangle of G (then R) is kept
-// packed column by column, (i, j) at j (j + 1) / 2 + i, in LDS when it fits (n <= 199) and in a
-// global working copy otherwise; X^T is written straight into the output's strict lower triangle
-// (X_ij at U[j + i n]) and reflected at the end; sv[k] = 1 / r_kk (0 for a dependent pivot) is the
-// diagonal of X.  Pivot step k runs three disjoint phases:
-//   (a) row k-1 of R is scaled by sv[k-1] (the division by r_{k-1,k-1}, deferred one step);
-//   (b) right-looking update with the unscaled row k: W_ij -= W_ki W_kj / d_k for k < i <= j,
-//       columns paired (j, t-1-j) so that every thread gets the same number of entries;
-//   (c) column k-1 of X from the finished rows/columns < k-1, 16 lanes per entry:
-//       X_{i,k-1} = -sv[k-1] * sum_{l=i}^{k-2} X_il R_{l,k-1}  (X R = I by columns).
-// (a) writes row k-1 (columns >= k), (b) reads row k and writes rows > k, (c) reads rows < k-1 of
-// R and columns < k-1 of X and writes column k-1 of X, so one barrier per step suffices.
-// Blocks in the global working copy use a panel variant (PANEL = true) of the same steps,
-// described at its loop; in LDS the per-pivot barrier, not the trailing update's traffic, bounds
-// the time, and the plain loop is as fast.
+// One workgroup per block, in 16 x 16 tiles on the matrix cores.  The time is the serial chain of
+// ceil(n / 16) diagonal tiles and of the barriers between them, not the n^3 / 3 flops (which one CU
+// does in a few microseconds at n = 74), so a panel has two barriers:
+//   solve     R_pj = R_pp^-T A_pj for the tiles right of the diagonal, one per wave;
+//   update    A_ij -= R_pi^T R_pj; wave 0 takes the next diagonal tile first and factorises it
+//             while the other waves update the rest.
+// Then X R = I by block columns J: S = sum_l X_il R_lJ, X_iJ = -S R_JJ^-1, one tile row per wave.
+// Multiplying by the explicit inverse of a diagonal tile is followed by one step of refinement
+// with the tile itself, which gives back the stability of substitution.
+//
+// The tiles (i, j), i <= j, are packed by columns in LDS (n <= 192) or in a global working copy.
+// Element (r, c) of a tile is at 16 r + (c ^ r), so that a wave reads and writes rows, columns and
+// transposes without bank conflicts, and so that one set of four offsets per lane serves the A
+// operand R^T, the B operand and the accumulators of v_mfma_f64_16x16x4f64: an accumulator is the
+// B operand of the next product as it is.  A factorised diagonal tile holds R above and X^T = R^-T
+// on and below its diagonal, with R's diagonal in rdiag; X is kept transposed, in LDS in the place
+// of R's block column once that is used up.
+// (One barrier per pivot and 16 lanes per dot product of X: 134 us at n = 74, 673 us at n = 190;
+// these tiles 30 and 98 us, 2286 -> 227 us at n = 250.)
 constexpr int CI_THREADS = 1024;
-constexpr int CI_LANES = 16;  // lanes per dot product in (c)
-constexpr int CI_PANEL = 8;   // pivots per trailing update of the panel variant
-constexpr int CI_MAX_N = 40000;  // packed indices of a block fit in 32 bits
+constexpr int CI_MAX_N = 40000;
 
-__host__ __device__ inline int64_t chol_work_doubles(int64_t n) { return n * (n + 1) / 2 + 4 * n; }
-__device__ __forceinline__ int64_t pk(int i, int j) { return int64_t(j) * (j + 1) / 2 + i; }
-__device__ __forceinline__ int pk32(int i, int j) { return ((j * (j + 1)) >> 1) + i; }  // n <= CI_MAX_N
+__host__ __device__ inline int64_t chol_tiles(int64_t n) { return ((n + 15) / 16) * ((n + 15) / 16 + 1) / 2; }
+__host__ __device__ inline int64_t chol_work_doubles(int64_t n, bool lds) { return chol_tiles(n) * 256 * (lds ? 1 : 2) + 2 * ((n + 15) / 16) * 16; }
 
-template <bool PANEL>
+typedef double d4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ double lane_value(double x, int lane)
+{
+    const int lo = __builtin_amdgcn_readlane(__double2loint(x), lane), hi = __builtin_amdgcn_readlane(__double2hiint(x), lane);
+    return __hiloint2double(hi, lo);
+}
+
+template <bool LDS>
 __global__ __launch_bounds__(CI_THREADS) void k_chol_inv(FactorArgs fa)
 {
-    extern __shared__ double smem[];
+    extern __shared__ __attribute__((aligned(16))) double smem[];
     __shared__ double s_part[CI_THREADS / 64];
     const xh_factor_item it = fa.items[blockIdx.x];
     const int n = it.n;
     if(n == 0) return;
-    double* W = work_base<!PANEL>(smem, fa);
-    const int64_t np = int64_t(n) * (n + 1) / 2;
-    double* rd = W + np;  // shifted original diagonal (dependence threshold)
-    double* sv = rd + n;  // 1 / r_kk, or 0
-    double* Y = sv + n;   // LDS variant: two columns of X in flight
-    double* X = fa.U + it.u_off;
-    const int tid = threadIdx.x;
-    const double* G = fa.A + it.a_off;
-    const int64_t nn = int64_t(n) * n;
-    double tr = 0.0;
-    for(int64_t e = tid; e < nn; e += CI_THREADS) {
-        const int i = static_cast<int>(e % n), j = static_cast<int>(e / n);
-        if(i <= j) {
-            const double g = G[e];
-            W[pk(i, j)] = g;
-            if(i == j) tr += g;
-        }
+    const int nt = (n + 15) / 16;
+    const int64_t ntri = chol_tiles(n);
+    double* W = work_base<LDS>(smem, fa);
+    double* XT = LDS ? W : W + ntri * 256;          // X's tiles off the diagonal
+    double* rd = W + ntri * (LDS ? 256 : 512);       // shifted original diagonal (dependence threshold)
+    double* rdiag = rd + nt * 16;                    // diagonal of R
+    constexpr int NW = CI_THREADS / 64;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int col = lane & 15, row0 = lane >> 4;     // element (row0 + 4 q, col) of a tile for q = 0 .. 3
+    int o[4], ot[4];                                 // its offset, and that of its mirror image
+#pragma unroll
+    for(int q = 0; q < 4; ++q) {
+        const int r = row0 + 4 * q;
+        o[q] = r * 16 + (col ^ r);
+        ot[q] = col * 16 + (r ^ col);
     }
-    for(int o = 32; o > 0; o >>= 1) tr += __shfl_xor(tr, o);
-    if((tid & 63) == 0) s_part[tid >> 6] = tr;
+    auto tri = [](int i, int j) { return (int64_t(j) * (j + 1) / 2 + i) * 256; };
+    auto tile = [&](int i, int j) { return W + tri(i, j); };
+    // the identity continues G beyond n
+    const double* G = fa.A + it.a_off;
+    double tr = 0.0;
+    for(int j = 0; j < nt; ++j)
+        for(int i = (wave + NW - j % NW) % NW; i <= j; i += NW) {
+            double* t = tile(i, j);
+#pragma unroll
+            for(int q = 0; q < 4; ++q) {  // lanes along a column of G
+                const int gi = 16 * i + col, gj = 16 * j + row0 + 4 * q;
+                const double v = gj < n && gi <= gj ? G[gi + int64_t(gj) * n] : (gi == gj ? 1.0 : 0.0);
+                t[ot[q]] = v;
+                if(gi == gj && gj < n) tr += v;
+            }
+        }
+    for(int k = 32; k > 0; k >>= 1) tr += __shfl_xor(tr, k);
+    if(lane == 0) s_part[wave] = tr;
     __syncthreads();
     {
         double t = 0.0;
-        for(int w = 0; w < CI_THREADS / 64; ++w) t += s_part[w];
+        for(int w = 0; w < NW; ++w) t += s_part[w];
         const double shift = fa.S[it.s_off] * t;
-        for(int k = tid; k < n; k += CI_THREADS) {
-            const double d = W[pk(k, k)] + shift;
-            W[pk(k, k)] = d;
-            rd[k] = d;
-        }
-    }
-    if constexpr(!PANEL) {
-        for(int k = 0; k <= n; ++k) {
-            __syncthreads();
-            double inv_d = 0.0;
-            if(k < n) {
-                const double d = W[pk32(k, k)];
-                const bool ok = d > 64.0 * DBL_EPSILON * rd[k] && d <= DBL_MAX;
-                inv_d = ok ? 1.0 / d : 0.0;
-                if(tid == 0) sv[k] = ok ? 1.0 / sqrt(d) : 0.0;  // read from step k + 1 on
-            }
-            if(k >= 1) {
-                // (a) deferred scaling of row k - 1
-                const double s = sv[k - 1];
-                for(int j = k + tid; j < n; j += CI_THREADS) W[pk32(k - 1, j)] *= s;
-            }
-            if(k + 1 < n && inv_d != 0.0) {
-                // (b) columns a = k+1+pp (rows k+1 .. a) and b = n-1-pp (rows k+1 .. b) as one list
-                const int t = n - k - 1;
-                const int npairs = (t + 1) / 2;
-                const int c2 = npairs <= CI_THREADS ? CI_THREADS / npairs : 1;
-                const int p0 = npairs <= CI_THREADS ? tid % npairs : tid;
-                const int s0 = npairs <= CI_THREADS ? tid / npairs : 0;
-                if(s0 < c2) {
-                    for(int pp = p0; pp < npairs; pp += (npairs <= CI_THREADS ? npairs : CI_THREADS)) {
-                        const int a = pp, b = t - 1 - pp;
-                        const int la = a + 1;
-                        const int len = (a == b) ? la : la + b + 1;
-                        const double wka = W[pk32(k, k + 1 + a)] * inv_d, wkb = W[pk32(k, k + 1 + b)] * inv_d;
-                        // entries s0, s0 + c2, ... of the list: column a's rows, then column b's;
-                        // a column's rows are contiguous in the packed triangle
-                        const int ca = pk32(k + 1, k + 1 + a), cb = pk32(k + 1, k + 1 + b);
-                        int e = s0;
-                        for(; e < la; e += c2) W[ca + e] -= W[pk32(k, k + 1 + e)] * wka;
-                        for(; e < len; e += c2) W[cb + e - la] -= W[pk32(k, k + 1 + e - la)] * wkb;
-                    }
-                }
-            }
-            if(k >= 1) {
-                // (c) column j = k - 1 of X into Yc, rows i < j, from the columns of X before it
-                // (in place in W, the last one still in Yp) and column j of R; then column j - 1
-                // of X (computed last step) goes from Yp into W, over R's column j - 1
-                const int j = k - 1;
-                const double* Yp = Y + ((k - 1) & 1) * n;
-                double* Yc = Y + (k & 1) * n;
-                constexpr int per = CI_THREADS / CI_LANES;
-                const double sj = sv[j];
-                for(int base = 0; base < j; base += per) {
-                    const int i = base + tid / CI_LANES, part = tid & (CI_LANES - 1);
-                    double acc0 = 0.0, acc1 = 0.0;
-                    if(i < j) {
-                        // X_il for l < j - 1 in place (its diagonal is sv), X_i,j-1 in Yp.  For
-                        // l = j - 1 (column j - 1 of W is being written back this step) the load
-                        // reads R's column j instead and its value is not used, so that the select
-                        // is a value select, not a branch
-                        const double yp = Yp[i];
-                        int l = i + part;
-                        for(; l + CI_LANES < j; l += 2 * CI_LANES) {
-                            const bool last = l + CI_LANES == j - 1;
-                            const double x0 = W[pk32(i, l)];
-                            const double w1 = W[last ? pk32(l + CI_LANES, j) : pk32(i, l + CI_LANES)];
-                            const double x1 = last ? yp : w1;
-                            acc0 = fma(x0, W[pk32(l, j)], acc0);
-                            acc1 = fma(x1, W[pk32(l + CI_LANES, j)], acc1);
-                        }
-                        if(l < j) {
-                            const bool last = l == j - 1;
-                            const double w0 = W[last ? pk32(l, j) : pk32(i, l)];
-                            const double x0 = last ? yp : w0;
-                            acc0 = fma(x0, W[pk32(l, j)], acc0);
-                        }
-                    }
-                    double acc = acc0 + acc1;
-                    for(int o = CI_LANES >> 1; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
-                    if(i < j && part == 0) Yc[i] = -acc * sj;
-                }
-                if(tid == 0) Yc[j] = sj;
-                if(k >= 2)
-                    for(int i = tid; i <= j - 1; i += CI_THREADS) W[pk32(i, j - 1)] = Yp[i];
-            }
-        }
-        // the last column of X into W, then X (upper triangle of W, zeros below) to the output
-        __syncthreads();
-        {
-            const double* Yl = Y + (n & 1) * n;
-            for(int i = tid; i < n; i += CI_THREADS) W[pk32(i, n - 1)] = Yl[i];
-        }
-        __syncthreads();
-        for(int64_t e = tid; e < nn; e += CI_THREADS) {
-            const int i = static_cast<int>(e % n), j = static_cast<int>(e / n);
-            X[e] = i <= j ? W[pk32(i, j)] : 0.0;
-        }
-        return;
-    } else {
-        // panel variant (blocks in the global working copy): rows of W stay unscaled (row k of R is
-        // W's row k times sv[k]) and are never written after their pivot step.  Inside a panel of
-        // CI_PANEL pivots, (a) updates the panel's remaining rows by pivot k; at the panel's last
-        // pivot, (b) applies the rank-CI_PANEL update of all its pivots to the rows below, so the
-        // trailing triangle is read and written once per panel.  (c) is as above with R_lj =
-        // sv[l] W_lj.  1 / d_r of an earlier pivot of the panel is taken as sv[r]^2.
-        for(int k = 0; k <= n; ++k) {
-            __syncthreads();
-            if(k < n) {
-                const double d = W[pk32(k, k)];
-                const bool ok = d > 64.0 * DBL_EPSILON * rd[k] && d <= DBL_MAX;
-                const double s = ok ? 1.0 / sqrt(d) : 0.0;
-                const double inv_d = s * s;
-                if(tid == 0) sv[k] = s;  // read from step k + 1 on
-                const int k0 = k - k % CI_PANEL;
-                const int kl = min(k0 + CI_PANEL, n) - 1;
-                const int t = n - k - 1;
-                if(k < kl) {
-                    if(inv_d != 0.0) {
-                        const int ne = (kl - k) * t;
-                        for(int e = tid; e < ne; e += CI_THREADS) {
-                            const int i = k + 1 + e / t, j = k + 1 + e % t;
-                            if(j >= i) W[pk32(i, j)] -= W[pk32(k, i)] * (W[pk32(k, j)] * inv_d);
-                        }
-                    }
-                } else if(t > 0) {
-                    // k == kl < n - 1 implies a full panel: k - k0 + 1 == CI_PANEL
-                    const int npairs = (t + 1) / 2;
-                    const int c2 = npairs <= CI_THREADS ? CI_THREADS / npairs : 1;
-                    const int p0 = npairs <= CI_THREADS ? tid % npairs : tid;
-                    const int s0 = npairs <= CI_THREADS ? tid / npairs : 0;
-                    if(s0 < c2) {
-                        double idr[CI_PANEL];
-#pragma unroll
-                        for(int r = 0; r < CI_PANEL - 1; ++r) idr[r] = sv[k0 + r] * sv[k0 + r];
-                        idr[CI_PANEL - 1] = inv_d;
-                        for(int pp = p0; pp < npairs; pp += (npairs <= CI_THREADS ? npairs : CI_THREADS)) {
-                            const int a = pp, b = t - 1 - pp;
-                            const int la = a + 1;
-                            const int len = (a == b) ? la : la + b + 1;
-                            const int ca = pk32(0, k + 1 + a), cb = pk32(0, k + 1 + b);
-                            double fa[CI_PANEL], fb[CI_PANEL];
-#pragma unroll
-                            for(int r = 0; r < CI_PANEL; ++r) {
-                                fa[r] = W[ca + k0 + r] * idr[r];
-                                fb[r] = W[cb + k0 + r] * idr[r];
-                            }
-                            for(int e = s0; e < len; e += c2) {
-                                const bool first = e < la;
-                                const int i = k + 1 + (first ? e : e - la);
-                                const int bi = pk32(k0, i);
-                                const int pos = (first ? ca : cb) + i;
-                                double acc = W[pos];
-#pragma unroll
-                                for(int r = 0; r < CI_PANEL; ++r) acc = fma(-W[bi + r], first ? fa[r] : fb[r], acc);
-                                W[pos] = acc;
-                            }
-                        }
-                    }
-                }
-            }
-            if(k >= 2) {
-                const int j = k - 1;
-                const int cj = pk32(0, j);
-                constexpr int per = CI_THREADS / CI_LANES;
-                const double sj = sv[j];
-                for(int base = 0; base < j; base += per) {
-                    const int i = base + tid / CI_LANES, part = tid & (CI_LANES - 1);
-                    double acc0 = 0.0, acc1 = 0.0, acc2 = 0.0, acc3 = 0.0;
-                    if(i < j) {
-                        const double* xr = X + int64_t(i) * n;
-                        int l = i + part;
-                        for(; l + 3 * CI_LANES < j; l += 4 * CI_LANES) {
-                            const double xg = xr[l], xs = sv[i];  // both read: selecting a value, not an address space
-                            const double x0 = (l == i) ? xs : xg;
-                            const double x1 = xr[l + CI_LANES], x2 = xr[l + 2 * CI_LANES], x3 = xr[l + 3 * CI_LANES];
-                            acc0 = fma(x0 * sv[l], W[cj + l], acc0);
-                            acc1 = fma(x1 * sv[l + CI_LANES], W[cj + l + CI_LANES], acc1);
-                            acc2 = fma(x2 * sv[l + 2 * CI_LANES], W[cj + l + 2 * CI_LANES], acc2);
-                            acc3 = fma(x3 * sv[l + 3 * CI_LANES], W[cj + l + 3 * CI_LANES], acc3);
-                        }
-                        for(; l < j; l += CI_LANES) {
-                            const double xg = xr[l], xs = sv[i];  // both read: selecting a value, not an address space
-                            const double x0 = (l == i) ? xs : xg;
-                            acc0 = fma(x0 * sv[l], W[cj + l], acc0);
-                        }
-                    }
-                    double acc = (acc0 + acc1) + (acc2 + acc3);
-                    for(int o = CI_LANES >> 1; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
-                    if(i < j && part == 0) X[j + int64_t(i) * n] = -acc * sj;
-                }
-            }
+        for(int k = threadIdx.x; k < 16 * nt; k += CI_THREADS) {
+            double* d = tile(k / 16, k / 16) + (k & 15) * 16;  // (r, r) is at 16 r + 0
+            if(k < n) *d += shift;
+            rd[k] = *d;
         }
     }
     __syncthreads();
-    // reflect X^T into the upper triangle, zero the lower one, set the diagonal
-    for(int64_t e = tid; e < nn; e += CI_THREADS) {
-        const int i = static_cast<int>(e % n), j = static_cast<int>(e / n);
-        if(i < j) {
-            const int64_t lo = j + int64_t(i) * n;
-            X[e] = X[lo];
-            X[lo] = 0.0;
-        } else if(i == j) {
-            X[e] = sv[j];
+
+    // Cholesky factor and inverse of a diagonal tile by one wave: lane j holds column j of the
+    // tile, lane 16 + j column j of the identity, and both take the same row operations
+    auto factor = [&](int p) {
+        double* t = tile(p, p);
+        double x[16];
+#pragma unroll
+        for(int i = 0; i < 16; ++i) x[i] = lane < 16 ? t[i * 16 + (col ^ i)] : lane < 32 && i == col ? 1.0 : 0.0;
+        const double thr = 64.0 * DBL_EPSILON * rd[16 * p + col];
+        double diag = 0.0;
+#pragma unroll
+        for(int k = 0; k < 16; ++k) {
+            const double d = lane_value(x[k], k);
+            const bool ok = d > lane_value(thr, k) && d <= DBL_MAX;
+            // 1 / sqrt(d): the hardware estimate and its second-order correction
+            const double y = __builtin_amdgcn_rsq(ok ? d : 1.0);
+            const double e = fma(-d * y, y, 1.0);
+            const double s = ok ? fma(y * e, fma(e, 0.375, 0.5), y) : 0.0;
+            x[k] *= s;
+            if(lane == k) diag = x[k];
+#pragma unroll
+            for(int i = k + 1; i < 16; ++i) x[i] = fma(-lane_value(x[k], i), x[k], x[i]);
+        }
+        if(lane < 32) {
+#pragma unroll
+            for(int i = 0; i < 16; ++i)
+                if(lane < 16 ? i < col : i >= col) t[i * 16 + (col ^ i)] = x[i];
+            if(lane < 16) rdiag[16 * p + col] = diag;
+        }
+    };
+    // a diagonal tile as A operands: X_pp^T and R_pp^T
+    auto load_diag = [&](int p, double (&x)[4], double (&r)[4]) {
+        const double* t = tile(p, p);
+        const double dg = rdiag[16 * p + col];
+#pragma unroll
+        for(int q = 0; q < 4; ++q) {
+            const int k = row0 + 4 * q;
+            const double a = t[ot[q]], b = t[o[q]];
+            x[q] = k <= col ? a : 0.0;
+            r[q] = k < col ? b : (k == col ? dg : 0.0);
+        }
+    };
+    auto mfma = [](double a, double b, d4 c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); };
+    // sign * X_pp^T c with one refinement against R_pp^T
+    auto solve = [&](const double (&x)[4], const double (&r)[4], const d4 c, double sign) {
+        d4 y = {0, 0, 0, 0};
+#pragma unroll
+        for(int q = 0; q < 4; ++q) y = mfma(x[q], c[q], y);
+        d4 res = c;
+#pragma unroll
+        for(int q = 0; q < 4; ++q) res = mfma(-r[q], y[q], res);
+#pragma unroll
+        for(int q = 0; q < 4; ++q) y = mfma(x[q], res[q], y);
+        return sign * y;
+    };
+    auto update = [&](int p, int i, int j) {
+        const double *a = tile(p, i), *b = tile(p, j);
+        double* t = tile(i, j);
+        d4 c;
+        double u[4], v[4];
+#pragma unroll
+        for(int q = 0; q < 4; ++q) {
+            c[q] = t[o[q]];
+            u[q] = a[o[q]];
+            v[q] = b[o[q]];
+        }
+#pragma unroll
+        for(int q = 0; q < 4; ++q) c = mfma(-u[q], v[q], c);
+#pragma unroll
+        for(int q = 0; q < 4; ++q) t[o[q]] = c[q];
+    };
+    if(wave == 0) factor(0);
+    __syncthreads();
+    for(int p = 0; p + 1 < nt; ++p) {
+        if(p + 1 + wave < nt) {
+            double x[4], r[4];
+            load_diag(p, x, r);
+            for(int j = p + 1 + wave; j < nt; j += NW) {
+                double* t = tile(p, j);
+                d4 c;
+#pragma unroll
+                for(int q = 0; q < 4; ++q) c[q] = t[o[q]];
+                c = solve(x, r, c, 1.0);
+#pragma unroll
+                for(int q = 0; q < 4; ++q) t[o[q]] = c[q];
+            }
+        }
+        __syncthreads();
+        if(wave == 0) {
+            update(p, p + 1, p + 1);
+            factor(p + 1);
+        } else {
+            int left = wave;  // tiles of the trailing triangle by columns; number 0 is wave 0's
+            for(int j = p + 1; j < nt; ++j) {
+                for(; left <= j - p - 1; left += NW - 1) update(p, p + 1 + left, j);
+                left -= j - p;
+            }
+        }
+        __syncthreads();
+    }
+    for(int J = 1; J < nt; ++J) {
+        d4 c = {0, 0, 0, 0};
+        if(wave < J) {
+            double x[4], r[4];
+            load_diag(J, x, r);
+            for(int i = wave; i < J; i += NW) {
+                c = d4{0, 0, 0, 0};  // S^T = sum_l R_lJ^T X_il^T
+                for(int l = i; l < J; ++l) {
+                    const double *a = tile(l, J), *b = l == i ? tile(i, i) : XT + tri(i, l);
+                    double u[4], v[4];
+#pragma unroll
+                    for(int q = 0; q < 4; ++q) {
+                        u[q] = a[o[q]];
+                        v[q] = b[o[q]];
+                    }
+#pragma unroll
+                    for(int q = 0; q < 4; ++q) c = mfma(u[q], l > i || row0 + 4 * q >= col ? v[q] : 0.0, c);
+                }
+                c = solve(x, r, c, -1.0);
+                if constexpr(!LDS) {
+#pragma unroll
+                    for(int q = 0; q < 4; ++q) XT[tri(i, J) + o[q]] = c[q];
+                }
+            }
+        }
+        __syncthreads();
+        if constexpr(LDS) {  // at most NW tile rows: one per wave
+            if(wave < J) {
+#pragma unroll
+                for(int q = 0; q < 4; ++q) XT[tri(wave, J) + o[q]] = c[q];
+            }
+            __syncthreads();
+        }
+    }
+    // X to the output, zeros below its diagonal
+    double* X = fa.U + it.u_off;
+    for(int t = wave; t < nt * nt; t += NW) {
+        const int i = t % nt, j = t / nt;
+        const double* b = i == j ? tile(i, i) : i < j ? XT + tri(i, j) : nullptr;
+#pragma unroll
+        for(int q = 0; q < 4; ++q) {
+            const int gi = 16 * i + col, gj = 16 * j + row0 + 4 * q;
+            if(gi < n && gj < n) X[gi + int64_t(gj) * n] = gi <= gj ? b[o[q]] : 0.0;
         }
     }
 }
@@ -1157,13 +1127,12 @@ extern "C" int xh_block_chol_inv(xh_ctx* ctx, const xh_factor_item* items, int64
             if(it.n == 0) continue;
             it.s_off = static_cast<int64_t>(sh.size());
             sh.push_back(shift_rel ? shift_rel[i] : 0.0);
-            const int64_t need = chol_work_doubles(it.n);
-            if(size_t(need) * sizeof(double) <= budget) {
+            if(it.n <= 16 * (CI_THREADS / 64) && size_t(chol_work_doubles(it.n, true)) * sizeof(double) <= budget) {
                 small.push_back(it);
-                small_max = std::max(small_max, need);
+                small_max = std::max(small_max, chol_work_doubles(it.n, true));
             } else {
                 big.push_back(it);
-                big_max = std::max(big_max, need);
+                big_max = std::max(big_max, chol_work_doubles(it.n, false));
             }
         }
         if(sh.empty()) return;
@@ -1174,16 +1143,16 @@ extern "C" int xh_block_chol_inv(xh_ctx* ctx, const xh_factor_item* items, int64
         if(!small.empty()) {
             const size_t shmem = size_t(small_max) * sizeof(double);
             if(shmem > 64 * 1024)
-                check(hipFuncSetAttribute(reinterpret_cast<const void*>(k_chol_inv<false>), hipFuncAttributeMaxDynamicSharedMemorySize, int(shmem)), "hipFuncSetAttribute");
+                check(hipFuncSetAttribute(reinterpret_cast<const void*>(k_chol_inv<true>), hipFuncAttributeMaxDynamicSharedMemorySize, int(shmem)), "hipFuncSetAttribute");
             FactorArgs fa{up.ptr<xh_factor_item>(o_small), G, X, d_sh, nullptr, nullptr, 0, 1, nullptr};
-            hipLaunchKernelGGL(k_chol_inv<false>, dim3(static_cast<unsigned>(small.size())), dim3(CI_THREADS), shmem, ctx->stream, fa);
+            hipLaunchKernelGGL(k_chol_inv<true>, dim3(static_cast<unsigned>(small.size())), dim3(CI_THREADS), shmem, ctx->stream, fa);
             xh::launch_check("k_chol_inv");
         }
         if(!big.empty()) {
             double* scratch = nullptr;
             check(xh::dmalloc(ctx, reinterpret_cast<void**>(&scratch), size_t(big_max) * big.size() * sizeof(double)), "hipMallocAsync");
             FactorArgs fa{up.ptr<xh_factor_item>(o_big), G, X, d_sh, nullptr, scratch, big_max, 0, nullptr};
-            hipLaunchKernelGGL(k_chol_inv<true>, dim3(static_cast<unsigned>(big.size())), dim3(CI_THREADS), 0, ctx->stream, fa);
+            hipLaunchKernelGGL(k_chol_inv<false>, dim3(static_cast<unsigned>(big.size())), dim3(CI_THREADS), 0, ctx->stream, fa);
             xh::launch_check("k_chol_inv");
             xh::dev_free(ctx, scratch);
         }
