@@ -1,0 +1,85 @@
+"""FP64 grouped GEMM at the edges of its tile shapes (needs an MI355X): output sides around 32, 64,
+96, 128 and 192, K around the steps of 8 and 16 and with a split K, all four transposes, against
+numpy.  Bound: |error| <= k u |A| |B| elementwise (Higham, Accuracy and Stability of Numerical
+Algorithms, 2nd ed., section 3.5), doubled for the reference's own.  Non-finite entries reach only
+the rows and columns that hold them: tiles read past a matrix's last row and the end of K, into
+neighbouring values."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from xped_amd import _lib
+from xped_amd._lib import lib
+
+pytestmark = pytest.mark.gpu
+
+U = 2.0 ** -53
+SIDES = [1, 31, 32, 33, 64, 65, 95, 96, 97, 128, 129, 191, 193, 200, 257]
+
+
+def _products(rt, mats, ta, tb):
+    """C of every (A, B) in one grouped call; operands stored column-major, transposed where asked."""
+    L, ctx = lib(), rt.ctx()
+    items, ao, bo, co, fa, fb = [], 0, 0, 0, [], []
+    for A, B in mats:
+        m, k = A.shape
+        n = B.shape[1]
+        items.append(_lib.xh_gemm_item(ao, bo, co, m, n, k))
+        fa.append((A if ta else A.T).reshape(-1))
+        fb.append((B if tb else B.T).reshape(-1))
+        ao, bo, co = ao + m * k, bo + k * n, co + m * n
+    bufs = [C.c_void_p() for _ in range(3)]
+    for p, n in zip(bufs, (ao, bo, co)):
+        assert L.xh_alloc(ctx, 8 * n, C.byref(p)) == 0
+    for p, x in ((bufs[0], np.concatenate(fa)), (bufs[1], np.concatenate(fb))):
+        x = np.ascontiguousarray(x)
+        L.xh_upload(ctx, p, x.ctypes.data, 8 * x.size)
+    arr = (_lib.xh_gemm_item * len(items))(*items)
+    plan = C.c_void_p()
+    assert L.xh_gemm_plan_create(ctx, arr, len(items), ta, tb, C.byref(plan)) == 0
+    assert L.xh_gemm(ctx, plan, *bufs, 1.0, 0.0, _lib.XH_FP64) == 0, L.xh_last_error(ctx)
+    out = np.empty(co)
+    L.xh_download(ctx, out.ctypes.data, bufs[2], 8 * co)
+    L.xh_gemm_plan_destroy(ctx, plan)
+    for p in bufs:
+        L.xh_free(ctx, p)
+    return [out[it.c_off:it.c_off + it.m * it.n].reshape(it.n, it.m).T for it in items]
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (1, 0), (0, 1), (1, 1)])
+@pytest.mark.parametrize("ks", [(33, 48, 64, 200), (35, 47, 63, 129), (777,)], ids=["even", "odd", "split"])
+def test_tile_shapes(rt, ta, tb, ks):
+    r = np.random.default_rng(3)
+    sides = SIDES if len(ks) > 1 else SIDES[:7]
+    shapes = [(m, n, ks[(i + j) % len(ks)]) for i, m in enumerate(sides) for j, n in enumerate(sides)]
+    mats = [(r.uniform(-1, 1, (m, k)), r.uniform(-1, 1, (k, n))) for m, n, k in shapes]
+    for (A, B), c in zip(mats, _products(rt, mats, ta, tb)):
+        assert np.all(np.abs(c - A @ B) <= 2 * A.shape[1] * U * (np.abs(A) @ np.abs(B))), (A.shape, B.shape)
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (1, 0), (0, 1), (1, 1)])
+def test_nonfinite_entries_stay_in_their_rows_and_columns(rt, ta, tb):
+    r = np.random.default_rng(4)
+    mats, clean = [], []
+    for m, n, k in [(65, 70, 41), (97, 33, 43), (193, 257, 35), (70, 300, 47), (40, 40, 519)]:
+        A, B = r.uniform(-1, 1, (m, k)), r.uniform(-1, 1, (k, n))
+        A[5, :3], A[m - 1, 0], B[:2, 7], B[0, n - 1] = np.nan, np.inf, np.nan, -np.inf
+        mats.append((A, B))
+        rows, cols = np.ones(m, bool), np.ones(n, bool)
+        rows[[5, m - 1]] = cols[[7, n - 1]] = False
+        clean.append((rows, cols))
+    for (A, B), (rows, cols), c in zip(mats, clean, _products(rt, mats, ta, tb)):
+        ref = A[rows] @ B[:, cols]
+        assert np.all(np.abs(c[np.ix_(rows, cols)] - ref) <= 2 * A.shape[1] * U * (np.abs(A[rows]) @ np.abs(B[:, cols])))
+        assert not np.isfinite(c[~rows]).any() and not np.isfinite(c[:, ~cols]).any()
+
+
+def test_operands_beyond_32_bit_tile_offsets(rt):
+    # K of 2.1 million: 128 rows of a K-contiguous operand span more than 2 GiB, so the item takes
+    # the tiles with checked 64-bit loads (three rows keep the operands small)
+    r = np.random.default_rng(5)
+    k = 2_100_000
+    A, B = r.uniform(-1, 1, (3, k)), r.uniform(-1, 1, (k, 2))
+    c, = _products(rt, [(A, B)], 1, 0)
+    assert np.all(np.abs(c - A @ B) <= 2 * k * U * (np.abs(A) @ np.abs(B)))

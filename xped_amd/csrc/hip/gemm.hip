@@ -38,6 +38,7 @@ using xh::guard;
 
 namespace {
 
+typedef double d2 __attribute__((ext_vector_type(2)));
 typedef double d4 __attribute__((ext_vector_type(4)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef short s4 __attribute__((ext_vector_type(4)));
@@ -48,8 +49,9 @@ constexpr int G_THREADS = 256;
 constexpr int NPART = 8;  // XCDs of an MI355X
 
 struct Tile {
-    int32_t item, m0, n0, ks;  // ks: K chunk
+    int32_t item, m0, n0, ks;  // ks: K chunk, and from bit KS_BITS on the tile shape of k_gemm_f64 (0: 64 x 64)
 };
+constexpr int KS_BITS = 24, KS_MASK = (1 << KS_BITS) - 1;
 
 // K split of an item: chunks of kc (the last one shorter); split > 1 writes partials to ws.
 struct ItemExt {
@@ -80,6 +82,20 @@ __device__ __forceinline__ double load_b(const GemmArgs& g, const xh_gemm_item& 
     if(kk >= kend || j >= it.n) return 0.0;
     return g.tb ? g.B[it.b_off + int64_t(kk) * it.n + j] : g.B[it.b_off + int64_t(j) * it.k + kk];
 }
+
+// A tile, its item and its K split, told to the compiler as uniform over the wave: what follows from
+// them (bases, sizes, loop counts) is then scalar.
+__device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
+__device__ __forceinline__ int64_t uniform(int64_t x)
+{
+    return (int64_t(uniform(int(x >> 32))) << 32) | uint32_t(uniform(int(uint32_t(x))));
+}
+__device__ __forceinline__ Tile uniform(const Tile& t) { return Tile{uniform(t.item), uniform(t.m0), uniform(t.n0), uniform(t.ks)}; }
+__device__ __forceinline__ xh_gemm_item uniform(const xh_gemm_item& i)
+{
+    return xh_gemm_item{uniform(i.a_off), uniform(i.b_off), uniform(i.c_off), uniform(i.m), uniform(i.n), uniform(i.k)};
+}
+__device__ __forceinline__ ItemExt uniform(const ItemExt& e) { return ItemExt{uniform(e.split), uniform(e.kc), uniform(e.ws_off)}; }
 
 // The tile loop of workgroup blockIdx.x: its XCD's part, strided by the workgroups of that XCD.
 struct TileRange {
@@ -126,112 +142,292 @@ __global__ __launch_bounds__(256) void k_splitk_reduce(const RedItem* __restrict
 {
     const RedItem r = red[blockIdx.y];
     for(int64_t e = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; e < r.mn; e += int64_t(gridDim.x) * blockDim.x) {
+        // the chunks in order, 8 loads in flight (one load and one sum after the other took 16.5 us
+        // for 15 Gram blocks of 74 x 74 in 15 chunks)
         double acc = 0.0;
-        for(int s = 0; s < r.split; ++s) acc += ws[r.ws_off + s * r.mn + e];
+        const double* w = ws + r.ws_off + e;
+        int s = 0;
+        for(; s + 8 <= r.split; s += 8) {
+            double x[8];
+#pragma unroll
+            for(int u = 0; u < 8; ++u) x[u] = w[(s + u) * r.mn];
+#pragma unroll
+            for(int u = 0; u < 8; ++u) acc += x[u];
+        }
+        {
+            double x[8];
+#pragma unroll
+            for(int u = 0; u < 7; ++u) x[u] = s + u < r.split ? w[(s + u) * r.mn] : 0.0;
+#pragma unroll
+            for(int u = 0; u < 7; ++u)
+                if(s + u < r.split) acc += x[u];
+        }
         double* p = C + r.c_off + e;
         *p = (beta == 0.0) ? alpha * acc : alpha * acc + beta * *p;
     }
 }
 
-// ---------------------------------------------------------------- FP64, pipelined
-// BM x BN output tiles, 4 waves in 2 x 2, each owning (BM/2) x (BN/2) = MI x NI blocks of 16 x 16.
-// K steps of 16 run through two LDS stages: the operands of step t+1 are fetched into registers
-// while the matrix cores work on step t, then written to the other stage; one barrier per step.
-// Tiles that lie inside their item (all rows, columns and the whole K step in range) load without
-// bounds checks from per-thread offsets computed once per tile.
-template <int BM, int BN, int BK, int WGM, int WGN>
-__global__ __launch_bounds__(64 * WGM * WGN, 4) void k_gemm_f64p(GemmArgs g)
+// ---------------------------------------------------------------- FP64 tiles
+// One output tile of (16 MI WGM) x (16 NI WGN) by WGM x WGN waves of MI x NI blocks of 16 x 16.  An
+// FP64 MFMA of 16 x 16 x 4 keeps a SIMD's matrix core busy for 64 cycles, so nothing but the work
+// around the matrix cores can slow the loop down: it has no bounds checks, no address arithmetic
+// beyond a base pointer per K step, one barrier per K step of 16 and 16-byte loads throughout.
+//  * Operands come through buffer resources that end with the operand: rows beyond m (columns
+//    beyond n) read neighbouring values or zeros and reach only outputs that are not stored; the
+//    K beyond the end is zeroed in the last step alone (a neighbour may be NaN).
+//  * The next K step is fetched into registers before the products of the present one and put
+//    into the other of two LDS stages after them.
+//  * An operand that is contiguous along K lies in LDS as [row][16 + 2], one along the rows as
+//    [k][rows + 8]: writes are 16 bytes wide, and the reads of a wave spread evenly over the
+//    banks.  A step of 8 in K is two MFMAs; lane group g takes k = 2 g of it to the first and
+//    2 g + 1 to the second, the same in both layouts, so that a K-contiguous operand is read 16
+//    bytes at a time.  The order of an element's sum is the same for every tile shape.
+//  * The operands enter the MFMA swapped, so that an accumulator register holds 16 consecutive
+//    rows of a column of C: stores of 128 bytes.
+// Checked loads with 64-bit addresses per element, one LDS stage with two barriers and a lane's
+// column of C per store took 22.6 ms for the grouped product at leg dimension 512 (1.15 TFLOP, 8 %
+// of the tiles outside the blocks), this 20.5 ms on the same card, with the matrix cores busy 87 %
+// of the time; a sketch product of the projector SVD at chi 256 (1.6 GFLOP) went from 165 to 100 us.
+constexpr int BK = 16;
+
+constexpr int lds_ld(bool kcontig, int rows) { return kcontig ? BK + 2 : rows + 8; }
+constexpr int lds_doubles(bool kcontig, int rows) { return kcontig ? rows * (BK + 2) : BK * (rows + 8); }
+
+// K step of an operand: `rows` rows (from row r0) by 16, NT threads, 2 consecutive doubles a load
+template <bool KC, int ROWS, int NT>
+struct OperandStep {
+    static constexpr int PER = ROWS * (BK / 2) / NT;
+    static_assert(PER * NT == ROWS * (BK / 2), "loads divide evenly");
+    d2 v[PER];
+    int off[PER];    // bytes from the K step's base
+    const char* base;
+    int64_t left;    // bytes from base to the operand's end
+    int64_t step;    // bytes per K step
+    __device__ __forceinline__ void init(const double* op, int rows, int depth, int r0, int k0)
+    {
+        const int64_t ld = KC ? depth : rows;
+        const int64_t start = KC ? int64_t(r0) * ld + k0 : int64_t(k0) * ld + r0;
+        base = reinterpret_cast<const char*>(op + start);
+        left = (int64_t(rows) * depth - start) * 8;
+        step = (KC ? BK : int64_t(BK) * ld) * 8;
+#pragma unroll
+        for(int r = 0; r < PER; ++r) {
+            const int idx = int(threadIdx.x) + NT * r;
+            off[r] = static_cast<int>((KC ? int64_t(idx / 8) * ld + 2 * (idx % 8) : int64_t(idx / (ROWS / 2)) * ld + 2 * (idx % (ROWS / 2))) * 8);
+        }
+    }
+    __device__ __forceinline__ void fetch()
+    {
+        const int64_t n = left < 0 ? 0 : left > 0x7ffffff8 ? 0x7ffffff8 : left;
+        const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base), 0, static_cast<int>(n), 0x00020000);
+#pragma unroll
+        for(int r = 0; r < PER; ++r) v[r] = __builtin_bit_cast(d2, __builtin_amdgcn_raw_buffer_load_b128(rsrc, off[r], 0, 0));
+        base += step;
+        left -= step;
+    }
+    // the elements k >= k_left of the step to zero
+    __device__ __forceinline__ void clip(int k_left)
+    {
+#pragma unroll
+        for(int r = 0; r < PER; ++r) {
+            const int idx = int(threadIdx.x) + NT * r;
+            const int k = KC ? 2 * (idx % 8) : idx / (ROWS / 2);
+            if(k >= k_left) v[r][0] = 0.0;
+            if(k + (KC ? 1 : 0) >= k_left) v[r][1] = 0.0;
+        }
+    }
+    __device__ __forceinline__ void put(double* lds) const
+    {
+#pragma unroll
+        for(int r = 0; r < PER; ++r) {
+            const int idx = int(threadIdx.x) + NT * r;
+            const int at = KC ? (idx / 8) * lds_ld(true, ROWS) + 2 * (idx % 8) : (idx / (ROWS / 2)) * lds_ld(false, ROWS) + 2 * (idx % (ROWS / 2));
+            *reinterpret_cast<d2*>(lds + at) = v[r];
+        }
+    }
+};
+
+// the values of rows r (this lane's) at k = kc + 2 g and kc + 2 g + 1
+template <bool KC, int ROWS>
+__device__ __forceinline__ d2 operand_pair(const double* lds, int r, int k)
 {
-    constexpr int NT = 64 * WGM * WGN;                 // threads
-    constexpr int WTM = BM / WGM, WTN = BN / WGN;       // wave tile
-    constexpr int MI = WTM / 16, NI = WTN / 16;
-    constexpr int RA = BM * BK / NT, RB = BN * BK / NT;  // operand elements per thread and step
-    __shared__ double sA[2][BK][BM + 1];
-    __shared__ double sB[2][BK][BN + 1];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if constexpr(KC) return *reinterpret_cast<const d2*>(lds + r * lds_ld(true, ROWS) + k);
+    const double* p = lds + k * lds_ld(false, ROWS) + r;
+    return d2{p[0], p[lds_ld(false, ROWS)]};
+}
+
+template <int MI, int NI, int WGM, int WGN, bool TA, bool TB>
+__device__ __forceinline__ void tile_f64(const GemmArgs& g, const xh_gemm_item& it, const ItemExt& ex, int m0, int n0, int ks, double* smem)
+{
+    constexpr int NT = 64 * WGM * WGN, TM = 16 * MI * WGM, TN = 16 * NI * WGN;
+    constexpr bool KA = TA, KB = !TB;  // contiguous along K
+    constexpr int SA = lds_doubles(KA, TM), STAGE = SA + lds_doubles(KB, TN);
+    const int lane = threadIdx.x & 63, wave = uniform(int(threadIdx.x >> 6));
     const int wm = wave % WGM, wn = wave / WGM;
-    const TileRange tr = my_tiles(g);
-    for(int t = tr.begin; t < tr.end; t += tr.stride) {
-        const Tile tl = g.tiles[t];
-        const xh_gemm_item it = g.items[tl.item];
-        const ItemExt ex = g.ext[tl.item];
-        const int kbeg = tl.ks * ex.kc, kend = min(it.k, kbeg + ex.kc);
-        const bool full_mn = tl.m0 + BM <= it.m && tl.n0 + BN <= it.n;
-        // element r of this thread: A (i, kk) and B (kk, j), lanes along each operand's contiguous direction
-        int ai[RA], ak[RA], bk[RB], bj[RB];
-        int64_t aoff[RA], boff[RB];  // offset of the element at k = 0 of the item
-        for(int r = 0; r < RA; ++r) {
-            const int idx = tid + NT * r;
-            ai[r] = g.ta ? idx / BK : idx % BM;
-            ak[r] = g.ta ? idx % BK : idx / BM;
-            aoff[r] = g.ta ? int64_t(tl.m0 + ai[r]) * it.k + ak[r] : int64_t(ak[r]) * it.m + tl.m0 + ai[r];
+    const int kbeg = ks * ex.kc, kend = min(it.k, kbeg + ex.kc);
+    OperandStep<KA, TM, NT> A;
+    OperandStep<KB, TN, NT> B;
+    A.init(g.A + it.a_off, it.m, it.k, m0, kbeg);
+    B.init(g.B + it.b_off, it.n, it.k, n0, kbeg);
+    d4 acc[MI][NI];
+#pragma unroll
+    for(int a = 0; a < MI; ++a)
+#pragma unroll
+        for(int b = 0; b < NI; ++b) acc[a][b] = d4{0, 0, 0, 0};
+    auto fetch = [&](int k0) {
+        A.fetch();
+        B.fetch();
+        if(k0 + BK > kend) {
+            A.clip(kend - k0);
+            B.clip(kend - k0);
         }
-        for(int r = 0; r < RB; ++r) {
-            const int idx = tid + NT * r;
-            bj[r] = g.tb ? idx % BN : idx / BK;
-            bk[r] = g.tb ? idx / BN : idx % BK;
-            boff[r] = g.tb ? int64_t(bk[r]) * it.n + tl.n0 + bj[r] : int64_t(tl.n0 + bj[r]) * it.k + bk[r];
-        }
-        const int64_t astep = g.ta ? 1 : it.m, bstep = g.tb ? it.n : 1;  // offset per unit of k
-        const double* A = g.A + it.a_off;
-        const double* B = g.B + it.b_off;
-        double ra[RA], rb[RB];
-        auto fetch = [&](int k0) {
-            if(full_mn && k0 + BK <= kend) {
-                for(int r = 0; r < RA; ++r) ra[r] = A[aoff[r] + int64_t(k0) * astep];
-                for(int r = 0; r < RB; ++r) rb[r] = B[boff[r] + int64_t(k0) * bstep];
-            } else {
-                for(int r = 0; r < RA; ++r)
-                    ra[r] = (tl.m0 + ai[r] < it.m && k0 + ak[r] < kend) ? A[aoff[r] + int64_t(k0) * astep] : 0.0;
-                for(int r = 0; r < RB; ++r)
-                    rb[r] = (tl.n0 + bj[r] < it.n && k0 + bk[r] < kend) ? B[boff[r] + int64_t(k0) * bstep] : 0.0;
+    };
+    __syncthreads();  // the last reads of the tile before are done
+    if(kbeg < kend) {
+        fetch(kbeg);
+        A.put(smem);
+        B.put(smem + SA);
+    }
+    __syncthreads();
+    int cur = 0;
+    const int ra = wm * 16 * MI + (lane & 15), rb = wn * 16 * NI + (lane & 15), kg = 2 * (lane >> 4);
+    // a wave of an edge tile with nothing to store leaves the matrix cores to the others (leaving out
+    // single blocks of a wave as well made the compiler copy accumulators and spill)
+    const bool live = m0 + wm * 16 * MI < it.m && n0 + wn * 16 * NI < it.n;
+    for(int k0 = kbeg; k0 < kend; k0 += BK) {
+        const bool more = k0 + BK < kend;
+        if(more) fetch(k0 + BK);
+        const double *sA = smem + cur * STAGE, *sB = sA + SA;
+        // waves in their products go first: the others would only reach the barrier sooner
+        __builtin_amdgcn_s_setprio(1);
+        if(live) {
+#pragma unroll
+            for(int kc = 0; kc < BK; kc += 8) {
+                d2 av[MI], bv[NI];
+#pragma unroll
+                for(int a = 0; a < MI; ++a) av[a] = operand_pair<KA, TM>(sA, ra + 16 * a, kc + kg);
+#pragma unroll
+                for(int b = 0; b < NI; ++b) bv[b] = operand_pair<KB, TN>(sB, rb + 16 * b, kc + kg);
+#pragma unroll
+                for(int h = 0; h < 2; ++h)
+#pragma unroll
+                    for(int a = 0; a < MI; ++a)
+#pragma unroll
+                        for(int b = 0; b < NI; ++b) acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(bv[b][h], av[a][h], acc[a][b], 0, 0, 0);
             }
-        };
-        auto put = [&](int s) {
-            for(int r = 0; r < RA; ++r) sA[s][ak[r]][ai[r]] = ra[r];
-            for(int r = 0; r < RB; ++r) sB[s][bk[r]][bj[r]] = rb[r];
-        };
-        d4 acc[MI][NI];
-        for(int a = 0; a < MI; ++a)
-            for(int b = 0; b < NI; ++b) acc[a][b] = d4{0, 0, 0, 0};
-        __syncthreads();  // the previous tile's last reads of stage 0 are done
-        if(kbeg < kend) {
-            fetch(kbeg);
-            put(0);
+        }
+        __builtin_amdgcn_s_setprio(0);
+        cur ^= 1;
+        if(more) {
+            A.put(smem + cur * STAGE);
+            B.put(smem + cur * STAGE + SA);
         }
         __syncthreads();
-        int cur = 0;
-        for(int k0 = kbeg; k0 < kend; k0 += BK) {
-            const bool more = k0 + BK < kend;
-            if(more) fetch(k0 + BK);
-            for(int kq = 0; kq < BK; kq += 4) {
-                const int kr = kq + (lane >> 4);
-                double av[MI], bv[NI];
-                for(int mi = 0; mi < MI; ++mi) av[mi] = sA[cur][kr][wm * WTM + mi * 16 + (lane & 15)];
-                for(int ni = 0; ni < NI; ++ni) bv[ni] = sB[cur][kr][wn * WTN + ni * 16 + (lane & 15)];
-                for(int mi = 0; mi < MI; ++mi)
-                    for(int ni = 0; ni < NI; ++ni) acc[mi][ni] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[mi], bv[ni], acc[mi][ni], 0, 0, 0);
-            }
-            if(more) put(cur ^ 1);
-            __syncthreads();
-            cur ^= 1;
-        }
-        const bool part = ex.split > 1;
-        double* base = part ? g.ws + ex.ws_off + int64_t(tl.ks) * it.m * it.n : g.C + it.c_off;
-        const double alpha = part ? 1.0 : g.alpha, beta = part ? 0.0 : g.beta;
-        for(int mi = 0; mi < MI; ++mi)
-            for(int ni = 0; ni < NI; ++ni)
-                for(int r = 0; r < 4; ++r) {
-                    const int row = tl.m0 + wm * WTM + mi * 16 + (lane >> 4) + 4 * r;
-                    const int col = tl.n0 + wn * WTN + ni * 16 + (lane & 15);
-                    if(row < it.m && col < it.n) {
-                        double* p = base + int64_t(col) * it.m + row;
-                        const double v = acc[mi][ni][r];
-                        *p = (beta == 0.0) ? alpha * v : alpha * v + beta * *p;
-                    }
+    }
+    // a K chunk of a split item stores its raw partial product into the workspace
+    const bool part = ex.split > 1;
+    double* base = part ? g.ws + ex.ws_off + int64_t(ks) * it.m * it.n : g.C + it.c_off;
+    const double alpha = part ? 1.0 : g.alpha, beta = part ? 0.0 : g.beta;
+#pragma unroll
+    for(int b = 0; b < NI; ++b)
+#pragma unroll
+        for(int r = 0; r < 4; ++r) {
+            const int col = n0 + (wn * NI + b) * 16 + (lane >> 4) + 4 * r;
+            double* p = base + int64_t(col) * it.m + m0 + ra;
+#pragma unroll
+            for(int a = 0; a < MI; ++a) {
+                if(col < it.n && m0 + ra + 16 * a < it.m) {
+                    const double v = acc[a][b][r];
+                    p[16 * a] = (beta == 0.0) ? alpha * v : alpha * v + beta * p[16 * a];
                 }
+            }
+        }
+}
+
+// Items with an operand whose tile is out of reach of 32-bit byte offsets (far_item) take 64 x 64 tiles
+// with checked loads from 64-bit offsets.
+__device__ void tile_f64_far(const GemmArgs& g, const xh_gemm_item& it, const ItemExt& ex, const Tile& tl, int ks, double* smem)
+{
+    double(*sA)[BM + 1] = reinterpret_cast<double(*)[BM + 1]>(smem);
+    double(*sB)[BN + 1] = reinterpret_cast<double(*)[BN + 1]>(smem + BK * (BM + 1));
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wm = wave & 1, wn = wave >> 1;
+    const int kbeg = ks * ex.kc, kend = min(it.k, kbeg + ex.kc);
+    d4 acc[2][2] = {};
+    for(int k0 = kbeg; k0 < kend; k0 += BK) {
+        __syncthreads();
+        for(int e = tid; e < BK * BM; e += G_THREADS) {
+            const int i = g.ta ? e / BK : e % BM, ka = g.ta ? e % BK : e / BM;
+            sA[ka][i] = load_a(g, it, tl.m0 + i, k0 + ka, kend);
+            const int j = g.tb ? e % BN : e / BK, kb = g.tb ? e / BN : e % BK;
+            sB[kb][j] = load_b(g, it, k0 + kb, tl.n0 + j, kend);
+        }
+        __syncthreads();
+        for(int kq = 0; kq < BK; kq += 4) {
+            const int kr = kq + (lane >> 4);
+            for(int a = 0; a < 2; ++a)
+                for(int b = 0; b < 2; ++b)
+                    acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(sA[kr][wm * 32 + a * 16 + (lane & 15)], sB[kr][wn * 32 + b * 16 + (lane & 15)], acc[a][b], 0, 0, 0);
+        }
+    }
+    __syncthreads();
+    Tile t = tl;
+    t.ks = ks;
+    store_tile<true>(g, it, ex, t, wm, wn, lane, acc);
+}
+
+// 128 x 128 tiles, 8 waves of 64 x 32, two workgroups per CU: for items with both output sides of
+// at least BIG_MIN that do not waste much of such tiles.
+constexpr int BM2 = 128, BN2 = 128;
+constexpr int BIG_MIN = 192;
+constexpr int G8_THREADS = 512;
+
+template <bool TA, bool TB>
+__global__ __launch_bounds__(G8_THREADS, 4) void k_gemm_f64_128(GemmArgs g)
+{
+    extern __shared__ __attribute__((aligned(16))) double smem[];
+    const TileRange tr = my_tiles(g);
+    for(int t = tr.begin; t < tr.end; t += tr.stride) {
+        const Tile tl = uniform(g.tiles[t]);
+        tile_f64<4, 2, 2, 4, TA, TB>(g, uniform(g.items[tl.item]), uniform(g.ext[tl.item]), tl.m0, tl.n0, tl.ks & KS_MASK, smem);
     }
 }
+
+constexpr int FAR_SHAPE = 7;
+// Tiles of 32 to 96 rows by 32 to 96 columns, 4 waves in 2 x 2, four workgroups per CU: the shape is
+// chosen per item (pick_shape) so that little of a tile lies outside the output, and is carried by each tile.
+template <bool TA, bool TB>
+__global__ __launch_bounds__(G_THREADS, 4) void k_gemm_f64(GemmArgs g)
+{
+    extern __shared__ __attribute__((aligned(16))) double smem[];
+    const TileRange tr = my_tiles(g);
+    for(int t = tr.begin; t < tr.end; t += tr.stride) {
+        const Tile tl = uniform(g.tiles[t]);
+        const xh_gemm_item it = uniform(g.items[tl.item]);
+        const ItemExt ex = uniform(g.ext[tl.item]);
+        const int ks = tl.ks & KS_MASK;
+        switch(tl.ks >> KS_BITS) {
+        case 1: tile_f64<1, 1, 2, 2, TA, TB>(g, it, ex, tl.m0, tl.n0, ks, smem); break;
+        case 2: tile_f64<2, 1, 2, 2, TA, TB>(g, it, ex, tl.m0, tl.n0, ks, smem); break;
+        case 3: tile_f64<1, 2, 2, 2, TA, TB>(g, it, ex, tl.m0, tl.n0, ks, smem); break;
+        case 4: tile_f64<2, 3, 2, 2, TA, TB>(g, it, ex, tl.m0, tl.n0, ks, smem); break;
+        case 5: tile_f64<3, 2, 2, 2, TA, TB>(g, it, ex, tl.m0, tl.n0, ks, smem); break;
+        case FAR_SHAPE: tile_f64_far(g, it, ex, tl, ks, smem); break;
+        default: tile_f64<2, 2, 2, 2, TA, TB>(g, it, ex, tl.m0, tl.n0, ks, smem); break;
+        }
+    }
+}
+constexpr int SHAPE_M[] = {64, 32, 64, 32, 64, 96, 0, 64}, SHAPE_N[] = {64, 32, 32, 64, 96, 64, 0, 64};
+constexpr int NSHAPE = 6;
+
+// whether a 128-row tile of an operand, or 16 columns of one, spans 2 GiB
+bool far_item(const xh_gemm_item& it, bool ta, bool tb)
+{
+    const int64_t a = ta ? int64_t(BM2) * it.k : int64_t(BK) * it.m, b = tb ? int64_t(BK) * it.n : int64_t(BN2) * it.k;
+    return std::max(a, b) >= (int64_t(1) << 28);
+}
+
+// LDS bytes of two stages of a tile shape
+constexpr size_t tile_lds(bool ta, bool tb, int tm, int tn) { return 2 * sizeof(double) * size_t(lds_doubles(ta, tm) + lds_doubles(!tb, tn)); }
 
 // ---------------------------------------------------------------- FP64, skinny items
 // Items whose output has one short side (S = min(m, n) <= SK_MAX) and a short K (<= SK_KMAX) are
@@ -524,79 +720,6 @@ __global__ __launch_bounds__(SK_THREADS, SCATTER ? 1 : 4) void k_gemm_skinny_gat
     }
 }
 
-// ---------------------------------------------------------------- FP64, 128 x 128 tiles
-// For items with both output sides >= 192: 8 waves in 2 x 4, each owning 64 x 32 (4 x 2 MFMA
-// blocks, 8 accumulators, so two or three waves share a SIMD), K steps of 16 staged in LDS, and
-// the next K step's operands fetched into registers while the matrix cores work on the current
-// one.  (A 4-wave variant with 64 x 64 per wave ran at one wave per SIMD and was 25-30 % slower.)
-constexpr int BM2 = 128, BN2 = 128;
-constexpr int BIG_MIN = 192;
-
-constexpr int G8_THREADS = 512;
-__global__ __launch_bounds__(G8_THREADS, 4) void k_gemm_f64_128(GemmArgs g)
-{
-    constexpr int BK = 16;
-    __shared__ double sA[BK][BM2 + 1];
-    __shared__ double sB[BK][BN2 + 1];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave & 1, wn = wave >> 1;  // wn in 0..3
-    const TileRange tr = my_tiles(g);
-    for(int t = tr.begin; t < tr.end; t += tr.stride) {
-        const Tile tl = g.tiles[t];
-        const xh_gemm_item it = g.items[tl.item];
-        const ItemExt ex = g.ext[tl.item];
-        const int kbeg = tl.ks * ex.kc, kend = min(it.k, kbeg + ex.kc);
-        d4 acc[4][2];
-        for(int a = 0; a < 4; ++a)
-            for(int b = 0; b < 2; ++b) acc[a][b] = d4{0, 0, 0, 0};
-        double ra[4], rb[4];
-        auto fetch = [&](int k0) {
-            for(int r = 0; r < 4; ++r) {
-                const int idx = tid + G8_THREADS * r;
-                const int i = g.ta ? idx >> 4 : idx & 127, kk = g.ta ? idx & 15 : idx >> 7;
-                ra[r] = load_a(g, it, tl.m0 + i, k0 + kk, kend);
-                const int kb = g.tb ? idx >> 7 : idx & 15, j = g.tb ? idx & 127 : idx >> 4;
-                rb[r] = load_b(g, it, k0 + kb, tl.n0 + j, kend);
-            }
-        };
-        if(kbeg < kend) fetch(kbeg);
-        for(int k0 = kbeg; k0 < kend; k0 += BK) {
-            __syncthreads();
-            for(int r = 0; r < 4; ++r) {
-                const int idx = tid + G8_THREADS * r;
-                const int i = g.ta ? idx >> 4 : idx & 127, kk = g.ta ? idx & 15 : idx >> 7;
-                sA[kk][i] = ra[r];
-                const int kb = g.tb ? idx >> 7 : idx & 15, j = g.tb ? idx & 127 : idx >> 4;
-                sB[kb][j] = rb[r];
-            }
-            __syncthreads();
-            if(k0 + BK < kend) fetch(k0 + BK);
-            for(int kq = 0; kq < BK; kq += 4) {
-                const int kr = kq + (lane >> 4);
-                double av[4], bv[2];
-                for(int mi = 0; mi < 4; ++mi) av[mi] = sA[kr][wm * 64 + mi * 16 + (lane & 15)];
-                for(int ni = 0; ni < 2; ++ni) bv[ni] = sB[kr][wn * 32 + ni * 16 + (lane & 15)];
-                for(int mi = 0; mi < 4; ++mi)
-                    for(int ni = 0; ni < 2; ++ni) acc[mi][ni] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[mi], bv[ni], acc[mi][ni], 0, 0, 0);
-            }
-        }
-        const bool part = ex.split > 1;
-        double* base = part ? g.ws + ex.ws_off + int64_t(tl.ks) * it.m * it.n : g.C + it.c_off;
-        const double alpha = part ? 1.0 : g.alpha, beta = part ? 0.0 : g.beta;
-        for(int mi = 0; mi < 4; ++mi)
-            for(int ni = 0; ni < 2; ++ni)
-                for(int r = 0; r < 4; ++r) {
-                    const int row = tl.m0 + wm * 64 + mi * 16 + (lane >> 4) + 4 * r;
-                    const int col = tl.n0 + wn * 32 + ni * 16 + (lane & 15);
-                    if(row < it.m && col < it.n) {
-                        double* p = base + int64_t(col) * it.m + row;
-                        const double v = acc[mi][ni][r];
-                        *p = (beta == 0.0) ? alpha * v : alpha * v + beta * *p;
-                    }
-                }
-    }
-}
-
 // ---------------------------------------------------------------- FP64 through int8 slices
 // Ozaki, Ogita, Oishi and Rump, Numer. Algorithms 59 (2012) 95-118 (error-free splitting of a
 // matrix product), with int8 slices as in Ootomo, Ozaki and Yokota, IJHPCA (2024).  Row i of A is
@@ -876,7 +999,8 @@ __global__ __launch_bounds__(G_THREADS) void k_gemm_f32(GemmArgs g)
     const int wm = wave & 1, wn = wave >> 1;
     const TileRange tr = my_tiles(g);
     for(int t = tr.begin; t < tr.end; t += tr.stride) {
-        const Tile tl = g.tiles[t];
+        Tile tl = g.tiles[t];
+        tl.ks &= KS_MASK;
         const xh_gemm_item it = g.items[tl.item];
         const ItemExt ex = g.ext[tl.item];
         const int kbeg = tl.ks * ex.kc, kend = min(it.k, kbeg + ex.kc);
@@ -927,7 +1051,8 @@ __global__ __launch_bounds__(G_THREADS) void k_gemm_bf16x3(GemmArgs g)
     const int wm = wave & 1, wn = wave >> 1;
     const TileRange tr = my_tiles(g);
     for(int t = tr.begin; t < tr.end; t += tr.stride) {
-        const Tile tl = g.tiles[t];
+        Tile tl = g.tiles[t];
+        tl.ks &= KS_MASK;
         const xh_gemm_item it = g.items[tl.item];
         const ItemExt ex = g.ext[tl.item];
         const int kbeg = tl.ks * ex.kc, kend = min(it.k, kbeg + ex.kc);
@@ -994,10 +1119,13 @@ struct xh_gemm_plan : xh::PlanLife {
     ItemExt* d_ext = nullptr;
     RedItem* d_red = nullptr;
     TileList all64;           // every item in 64 x 64 tiles (FP32 / BF16x3 modes), built on first use
-    TileList big128, rest64;  // FP64: items with both sides >= BIG_MIN in 128 x 128 tiles, the others in 64 x 64
+    TileList big128, rest64;  // FP64: items with large output sides in 128 x 128 tiles (is_big), the others in k_gemm_f64's shapes
+    size_t lds64 = 0;         // LDS bytes of rest64's largest tile
     TileList skinny;          // FP64: blocks of 256 long-side indices of the skinny items (Tile.m0 = first index)
     int sk_ms = 8;            // register width of the skinny kernel: 8, 16 or 32 >= every skinny item's short side
     bool all64_built = false, any_tiles = false;
+    bool skinny_kernel = false;  // skinny-shaped items run in the skinny kernel (use_skinny)
+    bool is_skinny(const xh_gemm_item& it) const;
     xh::PackedUpload up_all;
     // XH_OZAKI, built on first use: the slice layout of the items that take the int8 path, their
     // tiles and slicing jobs, and the 64 x 64 FP64 tiles of the other non-skinny items
@@ -1035,9 +1163,51 @@ void cut_parts(const std::vector<double>& work, int32_t part[NPART + 1])
     for(; x <= NPART; ++x) part[x] = static_cast<int32_t>(work.size());
 }
 
-bool is_big(const xh_gemm_item& it) { return it.m >= BIG_MIN && it.n >= BIG_MIN; }
-bool is_skinny(const xh_gemm_item& it) { return std::min(it.m, it.n) <= SK_MAX && it.k <= SK_KMAX; }
+// output elements of the tiles that cover m x n
+double padded(const xh_gemm_item& it, int tm, int tn) { return double((it.m + tm - 1) / tm) * tm * ((it.n + tn - 1) / tn) * tn; }
+// The shape of k_gemm_f64's tiles for an item: the least padded output, weighted with the operand
+// loads per product (1 / tm + 1 / tn; the factor is one load against 8 products).  A sketch panel
+// of 1900 x 74 takes 64 x 96 tiles (23 % of them outside) instead of 64 x 64 (42 %).
+int pick_shape(const xh_gemm_item& it, bool ta, bool tb)
+{
+    if(far_item(it, ta, tb)) return FAR_SHAPE;
+    int best = 0;
+    double least = 0.0;
+    for(int c = 0; c < NSHAPE; ++c) {
+        const double cost = padded(it, SHAPE_M[c], SHAPE_N[c]) * (1.0 + 8.0 / SHAPE_M[c] + 8.0 / SHAPE_N[c]);
+        if(c == 0 || cost < least) {
+            best = c;
+            least = cost;
+        }
+    }
+    return best;
+}
+// 128 x 128 tiles unless their padding costs more than the larger tile gains (192 x 192 fills 56 %)
+bool is_big(const xh_gemm_item& it, bool ta, bool tb)
+{
+    return !far_item(it, ta, tb) && it.m >= BIG_MIN && it.n >= BIG_MIN && padded(it, BM2, BN2) <= 1.4 * padded(it, BM, BN);
+}
+bool fits_skinny(const xh_gemm_item& it) { return std::min(it.m, it.n) <= SK_MAX && it.k <= SK_KMAX; }
+// Whether a call's skinny-shaped items take the skinny kernel: where every item is one, or where
+// they fill the chip by themselves (256 indices of the long side a workgroup).  A few of them beside
+// other items are tiles of the launch that runs anyway: alone they are a launch of 6 to 14 us, the
+// latency of one index's sums (projector SVD at chi 256: 54 launches).
+bool use_skinny(const std::vector<xh_gemm_item>& v, int num_cu)
+{
+    int64_t blocks = 0;
+    bool all = true;
+    for(const auto& it : v) {
+        if(it.m == 0 || it.n == 0) continue;
+        if(fits_skinny(it))
+            blocks += (std::max(it.m, it.n) + SK_THREADS - 1) / SK_THREADS;
+        else
+            all = false;
+    }
+    return all || blocks >= 2 * num_cu;
+}
 }  // namespace
+
+bool xh_gemm_plan::is_skinny(const xh_gemm_item& it) const { return skinny_kernel && fits_skinny(it); }
 
 extern "C" int xh_gemm_plan_create(xh_ctx* ctx, const xh_gemm_item* items, int64_t nitems, int trans_a, int trans_b, xh_gemm_plan** out)
 {
@@ -1050,12 +1220,16 @@ extern "C" int xh_gemm_plan_create(xh_ctx* ctx, const xh_gemm_item* items, int64
         std::vector<int> order(v.size());
         for(size_t i = 0; i < v.size(); ++i) order[i] = static_cast<int>(i);
         std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return double(v[a].m) * v[a].n * v[a].k > double(v[b].m) * v[b].n * v[b].k; });
+        plan->skinny_kernel = use_skinny(v, std::max(ctx->num_cu, 1));
+        auto is_skinny = [&](const xh_gemm_item& it) { return plan->skinny_kernel && fits_skinny(it); };
         int64_t base_tiles = 0;  // output tiles of the FP64 launch
         for(const auto& it : v) {
             if(it.m < 0 || it.n < 0 || it.k < 0) throw xh::Error(XH_EINVAL, "gemm plan: negative extent");
             if(it.a_off < 0 || it.b_off < 0 || it.c_off < 0) throw xh::Error(XH_EINVAL, "gemm plan: negative offset");
             if(it.m == 0 || it.n == 0 || is_skinny(it)) continue;
-            const int tm = is_big(it) ? BM2 : BM, tn = is_big(it) ? BN2 : BN;
+            const bool big = is_big(it, trans_a != 0, trans_b != 0);
+            const int sh = pick_shape(it, trans_a != 0, trans_b != 0);
+            const int tm = big ? BM2 : SHAPE_M[sh], tn = big ? BN2 : SHAPE_N[sh];
             base_tiles += int64_t((it.m + tm - 1) / tm) * ((it.n + tn - 1) / tn);
         }
         // K split: aim at 4 tiles per CU, chunks of at least 128
@@ -1089,7 +1263,10 @@ extern "C" int xh_gemm_plan_create(xh_ctx* ctx, const xh_gemm_item* items, int64
                     plan->max_red_mn = std::max(plan->max_red_mn, mn);
                 }
             }
-            const bool big = is_big(it);
+            const bool big = is_big(it, trans_a != 0, trans_b != 0);
+            const int sh = pick_shape(it, trans_a != 0, trans_b != 0), tm = SHAPE_M[sh], tn = SHAPE_N[sh];
+            if(e.split > KS_MASK) throw xh::Error(XH_EINVAL, "gemm plan: too many K chunks");
+            if(!big) plan->lds64 = std::max(plan->lds64, tile_lds(trans_a != 0, trans_b != 0, tm, tn));
             for(int ks = 0; ks < e.split; ++ks) {
                 const double kw = std::min(it.k - ks * e.kc, e.kc) + 8.0;  // + per-tile overhead
                 plan->any_tiles = true;
@@ -1100,10 +1277,10 @@ extern "C" int xh_gemm_plan_create(xh_ctx* ctx, const xh_gemm_item* items, int64
                             w_big.push_back(4.0 * kw);
                         }
                 } else {
-                    for(int n0 = 0; n0 < it.n; n0 += BN)
-                        for(int m0 = 0; m0 < it.m; m0 += BM) {
-                            t_rest.push_back(Tile{id, m0, n0, ks});
-                            w_rest.push_back(kw);
+                    for(int n0 = 0; n0 < it.n; n0 += tn)
+                        for(int m0 = 0; m0 < it.m; m0 += tm) {
+                            t_rest.push_back(Tile{id, m0, n0, ks | (sh << KS_BITS)});
+                            w_rest.push_back(kw * (tm * tn) / double(BM * BN));
                         }
                 }
             }
@@ -1214,11 +1391,12 @@ void build_all64(xh_ctx* ctx, xh_gemm_plan* plan)
         const xh_gemm_item& it = plan->h_items[id];
         if(it.m == 0 || it.n == 0) continue;
         const ItemExt& e = plan->h_ext[id];
+        const int far = far_item(it, plan->ta != 0, plan->tb != 0) ? FAR_SHAPE << KS_BITS : 0;
         for(int ks = 0; ks < e.split; ++ks) {
             const double kw = std::min(it.k - ks * e.kc, e.kc) + 8.0;
             for(int n0 = 0; n0 < it.n; n0 += BN)
                 for(int m0 = 0; m0 < it.m; m0 += BM) {
-                    t.push_back(Tile{id, m0, n0, ks});
+                    t.push_back(Tile{id, m0, n0, ks | far});
                     w.push_back(kw);
                 }
         }
@@ -1272,14 +1450,15 @@ void build_oz(xh_ctx* ctx, xh_gemm_plan* plan)
     std::vector<double> w_oz, w_rest;
     for(int id : plan->h_order) {
         const xh_gemm_item& it = plan->h_items[id];
-        if(it.m == 0 || it.n == 0 || is_skinny(it)) continue;
+        if(it.m == 0 || it.n == 0 || plan->is_skinny(it)) continue;
         const ItemExt& e = plan->h_ext[id];
         const bool oz = oz_item(it);
+        const int far = far_item(it, plan->ta != 0, plan->tb != 0) ? FAR_SHAPE << KS_BITS : 0;
         for(int ks = 0; ks < e.split; ++ks) {
             const double kw = std::min(it.k - ks * e.kc, e.kc) + 8.0;
             for(int n0 = 0; n0 < it.n; n0 += BN)
                 for(int m0 = 0; m0 < it.m; m0 += BM) {
-                    (oz ? t_oz : t_rest).push_back(Tile{id, m0, n0, ks});
+                    (oz ? t_oz : t_rest).push_back(Tile{id, m0, n0, oz ? ks : ks | far});
                     (oz ? w_oz : w_rest).push_back(kw);
                 }
         }
@@ -1372,15 +1551,20 @@ void gemm_run(xh_ctx* ctx, const xh_gemm_plan* cplan, const double* A, const dou
         xh::pin_for_capture(ctx, plan, gemm_plan_release);
         GemmArgs g{plan->d_items, plan->d_ext, nullptr, {}, plan->ta, plan->tb, A, B, C, ws, alpha, beta};
         // a multiple of NPART workgroups, at most per_cu per CU
-        auto launch = [&](const TileList& L, void (*kernel)(GemmArgs), int per_cu, int threads, const char* name) {
+        auto launch = [&](const TileList& L, void (*kernel)(GemmArgs), int per_cu, int threads, size_t lds, const char* name) {
             if(L.ntiles == 0) return;
             g.tiles = L.d_tiles;
             for(int x = 0; x <= NPART; ++x) g.part[x] = L.part[x];
             int grid = std::min<int>(L.ntiles, ctx->num_cu * per_cu);
             grid = (grid + NPART - 1) / NPART * NPART;
-            hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), 0, ctx->stream, g);
+            if(lds > 64 * 1024) check(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)), "hipFuncSetAttribute");
+            hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), lds, ctx->stream, g);
             xh::launch_check(name);
         };
+        const bool fta = plan->ta != 0, ftb = plan->tb != 0;
+        auto* f64_128 = fta ? (ftb ? k_gemm_f64_128<true, true> : k_gemm_f64_128<true, false>) : (ftb ? k_gemm_f64_128<false, true> : k_gemm_f64_128<false, false>);
+        auto* f64_64 = fta ? (ftb ? k_gemm_f64<true, true> : k_gemm_f64<true, false>) : (ftb ? k_gemm_f64<false, true> : k_gemm_f64<false, false>);
+        const size_t lds128 = tile_lds(fta, ftb, BM2, BN2), lds64 = tile_lds(fta, ftb, BM, BN);
         // tiles: 0 = FP64 128x128 tiles for the large items and 64x64 for the rest, 1 = 64x64 only
         auto run = [&](int tiles) {
             if(precision == XH_FP64 && tiles == 0) {
@@ -1390,10 +1574,10 @@ void gemm_run(xh_ctx* ctx, const xh_gemm_plan* cplan, const double* A, const dou
                     hipLaunchKernelGGL(kern, dim3(grid), dim3(SK_THREADS), 0, ctx->stream, g, plan->skinny.d_tiles, plan->skinny.ntiles);
                     xh::launch_check("k_gemm_skinny");
                 }
-                launch(plan->big128, k_gemm_f64_128, 2, G8_THREADS, "k_gemm_f64_128");
-                launch(plan->rest64, k_gemm_f64p<64, 64, 16, 2, 2>, 8, G_THREADS, "k_gemm_f64");
+                launch(plan->big128, f64_128, 2, G8_THREADS, lds128, "k_gemm_f64_128");
+                launch(plan->rest64, f64_64, 8, G_THREADS, plan->lds64, "k_gemm_f64");
             } else if(precision == XH_FP64) {
-                launch(plan->all64, k_gemm_f64p<64, 64, 16, 2, 2>, 8, G_THREADS, "k_gemm_f64");
+                launch(plan->all64, f64_64, 8, G_THREADS, lds64, "k_gemm_f64");
             } else if(precision == XH_OZAKI) {
                 if(!plan->oz_built) build_oz(ctx, plan);
                 if(plan->skinny.ntiles > 0) {
@@ -1402,7 +1586,7 @@ void gemm_run(xh_ctx* ctx, const xh_gemm_plan* cplan, const double* A, const dou
                     hipLaunchKernelGGL(kern, dim3(grid), dim3(SK_THREADS), 0, ctx->stream, g, plan->skinny.d_tiles, plan->skinny.ntiles);
                     xh::launch_check("k_gemm_skinny");
                 }
-                launch(plan->oz_rest, k_gemm_f64p<64, 64, 16, 2, 2>, 8, G_THREADS, "k_gemm_f64");
+                launch(plan->oz_rest, f64_64, 8, G_THREADS, lds64, "k_gemm_f64");
                 if(plan->oz_tiles.ntiles > 0) {
                     int8_t* sl = nullptr;
                     const size_t ex_off = (size_t(plan->oz_slice_bytes) + 255) / 256 * 256;
@@ -1428,7 +1612,7 @@ void gemm_run(xh_ctx* ctx, const xh_gemm_plan* cplan, const double* A, const dou
                     check(xh::dfree(ctx, sl), "hipFreeAsync(Ozaki slices)");
                 }
             } else {
-                launch(plan->all64, precision == XH_FP32 ? k_gemm_f32 : k_gemm_bf16x3, 8, G_THREADS, "k_gemm");
+                launch(plan->all64, precision == XH_FP32 ? k_gemm_f32 : k_gemm_bf16x3, 8, G_THREADS, 0, "k_gemm");
             }
             if(plan->nred > 0) {
                 const unsigned gx = static_cast<unsigned>(std::min<int64_t>((plan->max_red_mn + 1023) / 1024, 256));
@@ -1556,7 +1740,7 @@ bool gather_eligible(const xh_gemm_plan* plan)
 {
     if(plan->ta != 0 || plan->skinny.ntiles == 0) return false;
     for(const auto& it : plan->h_items)
-        if(it.m > 0 && it.n > 0 && !(is_skinny(it) && it.m > it.n)) return false;
+        if(it.m > 0 && it.n > 0 && !(plan->is_skinny(it) && it.m > it.n)) return false;
     return true;
 }
 
