@@ -433,144 +433,167 @@ constexpr size_t tile_lds(bool ta, bool tb, int tm, int tn) { return 2 * sizeof(
 // Items whose output has one short side (S = min(m, n) <= SK_MAX) and a short K (<= SK_KMAX) are
 // bound by the bytes of the long operand and of C, not by arithmetic: a 16 x 16 matrix-core tile
 // would waste most of its work on them.  One thread per index of the long side (256 per
-// workgroup) reads that index's K entries of the long operand once, keeps the S sums in registers
-// with the small operand staged in LDS (read as broadcasts), and writes its S outputs.
+// workgroup) reads that index's K entries of the long operand into registers and writes its S
+// outputs, each a sum over kk in order.  The small operand is the same for every lane, so its
+// entries come through scalar loads and are the scalar operands of the multiply-adds.  (Staged in
+// LDS and read as broadcasts it was bound by them: a 16-byte broadcast keeps the LDS of a CU busy
+// for 8 cycles and feeds two multiply-adds, of which the four SIMDs do one a cycle.)  KM: 16 or 32
+// >= K, for the registers (48 and 88).
 constexpr int SK_MAX = 32, SK_KMAX = 32, SK_THREADS = 256;
 
-// The S <= MS sums of one long-side index against the small operand in LDS (sS, [kk][s]) and
-// hands output s to store(s, sum), in passes of at most 16 outputs: the K loaded
-// elements stay in registers and only 16 accumulators are live (the gather kernel: 145 instead of
-// 169 VGPRs at MS = 32, three waves per SIMD instead of two).  Every sum runs over kk in order, as
-// one pass would.
-template <int MS, class Store>
-__device__ __forceinline__ void skinny_sums(const double* __restrict__ sS, const double (&x)[SK_KMAX], int K, int S, Store&& store)
+// Read-only memory whose loads at uniform addresses go through the scalar cache.
+using ConstDoubles = const double __attribute__((address_space(4)))*;
+
+// The S sums of one long-side index over kk < K of x[kk] and entry (kk, s) of the small operand,
+// at b[s ld + kk] (KC) or b[kk ld + s]; output s goes to store(s, sum).  K lies in the last of NCH
+// chunks of 4; entries past K are a zero times a zero.  NS sums at a time, whose operands (at most
+// 72 scalar registers) are loaded together, as the wait for them is what a pass costs.
+template <int NCH, int NS, bool KC, int KM, class Store>
+__device__ __forceinline__ void skinny_passes(ConstDoubles b, int K, int S, int64_t ld, const double (&x)[KM], Store&& store)
 {
-    constexpr int MH = MS > 16 ? 16 : MS;
+    for(int s = 0; s < S; s += NS) {
+        // the last pass without KC repeats sums of the one before: NS neighbours load together
+        const int s0 = KC ? s : min(s, S - NS);
+        ConstDoubles p = b + s0;
+        double acc[NS];
 #pragma unroll
-    for(int h = 0; h < MS; h += MH) {
-        if(h >= S) break;
-        double acc[MH];
+        for(int j = 0; j < NS; ++j) acc[j] = 0.0;
 #pragma unroll
-        for(int c = 0; c < MH; ++c) acc[c] = 0.0;
+        for(int kk = 0; kk < 4 * NCH; ++kk) {
+            const bool in = kk < 4 * (NCH - 1) || kk < K;
 #pragma unroll
-        for(int kk = 0; kk < SK_KMAX; ++kk)
-            if(kk < K)
+            for(int j = 0; j < NS; ++j) {
+                const double v = KC ? b[int64_t(min(s + j, S - 1)) * ld + (in ? kk : 0)] : p[j];
+                acc[j] = __builtin_fma(in ? v : 0.0, x[kk], acc[j]);
+            }
+            p += kk < K - 1 ? ld : 0;
+            if(!KC && NS * (kk % 32 + 1) % 32 == 0) __builtin_amdgcn_sched_barrier(0);
+        }
 #pragma unroll
-                for(int c = 0; c < MH; ++c) acc[c] = __builtin_fma(sS[kk * MS + h + c], x[kk], acc[c]);
+        for(int j = 0; j < NS; ++j) asm volatile("" : "+v"(acc[j]));  // summed here, not under the stores' conditions
 #pragma unroll
-        for(int c = 0; c < MH; ++c)
-            if(h + c < S) store(h + c, acc[c]);
+        for(int j = 0; j < NS; ++j)
+            if(KC ? s + j < S : s0 + j >= s) store(s0 + j, acc[j]);
     }
 }
-
-template <int MS, int R>
-__global__ __launch_bounds__(SK_THREADS) void k_gemm_skinny(GemmArgs g, const Tile* __restrict__ blocks, int nblocks)
+template <int NCH, bool KC, int KM, class Store>
+__device__ __forceinline__ void skinny_chunks(ConstDoubles b, int K, int S, int64_t ld, const double (&x)[KM], Store&& store)
 {
-    __shared__ double sS[SK_KMAX * MS];  // the small operand, [kk][s]
-    for(int b = blockIdx.x; b < nblocks; b += gridDim.x) {
-        const Tile tl = blocks[b];
-        const xh_gemm_item it = g.items[tl.item];
-        const bool wide = it.m <= it.n;  // wide: A is the small operand (C has S rows); else B
-        const int S = wide ? it.m : it.n, K = it.k, Lng = wide ? it.n : it.m;
-        __syncthreads();  // the previous block's reads of sS are done
-        for(int e = threadIdx.x; e < K * MS; e += SK_THREADS) {
-            const int sx = e % MS, kk = e / MS;
-            double v = 0.0;
-            if(sx < S) {
-                if(wide)
-                    v = g.ta ? g.A[it.a_off + int64_t(sx) * K + kk] : g.A[it.a_off + int64_t(kk) * it.m + sx];
-                else
-                    v = g.tb ? g.B[it.b_off + int64_t(kk) * it.n + sx] : g.B[it.b_off + int64_t(sx) * K + kk];
+    if constexpr(KC) {
+        skinny_passes<NCH, NCH <= 1 ? 8 : NCH == 2 ? 4 : NCH == 3 ? 3 : NCH == 4 ? 2 : 1, KC>(b, K, S, ld, x, store);
+    } else if(S >= 4) {
+        skinny_passes<NCH, 4, KC>(b, K, S, ld, x, store);
+    } else {
+        skinny_passes<NCH, 1, KC>(b, K, S, ld, x, store);
+    }
+}
+template <bool KC, int KM, class Store>
+__device__ __forceinline__ void skinny_sums(ConstDoubles b, int K, int S, int64_t ld, const double (&x)[KM], Store&& store)
+{
+    static_assert(KM == 16 || KM == 32);
+    switch((K + 3) / 4) {
+    case 0:
+        for(int s = 0; s < S; ++s) store(s, 0.0);
+        break;
+    case 1: skinny_chunks<1, KC>(b, K, S, ld, x, store); break;
+    case 2: skinny_chunks<2, KC>(b, K, S, ld, x, store); break;
+    case 3: skinny_chunks<3, KC>(b, K, S, ld, x, store); break;
+    case 4: skinny_chunks<4, KC>(b, K, S, ld, x, store); break;
+    default:
+        if constexpr(KM == 32) {
+            switch((K + 3) / 4) {
+            case 5: skinny_chunks<5, KC>(b, K, S, ld, x, store); break;
+            case 6: skinny_chunks<6, KC>(b, K, S, ld, x, store); break;
+            case 7: skinny_chunks<7, KC>(b, K, S, ld, x, store); break;
+            default: skinny_chunks<8, KC>(b, K, S, ld, x, store);
             }
-            sS[kk * MS + sx] = v;
-        }
-        __syncthreads();
-        // R long indices per thread, SK_THREADS apart, so that consecutive lanes stay consecutive; all
-        // K loads of a thread are issued before the first product, to keep many loads in flight
-#pragma unroll
-        for(int r = 0; r < R; ++r) {
-            const int L = tl.m0 + threadIdx.x + r * SK_THREADS;
-            if(L >= Lng) break;
-            double x[SK_KMAX];
-#pragma unroll
-            for(int kk = 0; kk < SK_KMAX; ++kk) {
-                x[kk] = 0.0;
-                if(kk < K) {
-                    if(wide)
-                        x[kk] = g.tb ? g.B[it.b_off + int64_t(kk) * it.n + L] : g.B[it.b_off + int64_t(L) * K + kk];
-                    else
-                        x[kk] = g.ta ? g.A[it.a_off + int64_t(L) * K + kk] : g.A[it.a_off + int64_t(kk) * it.m + L];
-                }
-            }
-            double acc[MS];
-#pragma unroll
-            for(int sx = 0; sx < MS; ++sx) acc[sx] = 0.0;
-#pragma unroll
-            for(int kk = 0; kk < SK_KMAX; ++kk)
-                if(kk < K)
-#pragma unroll
-                    for(int sx = 0; sx < MS; ++sx) acc[sx] = __builtin_fma(sS[kk * MS + sx], x[kk], acc[sx]);
-#pragma unroll
-            for(int sx = 0; sx < MS; ++sx)
-                if(sx < S) {
-                    double* p = g.C + it.c_off + (wide ? int64_t(L) * it.m + sx : int64_t(sx) * it.m + L);
-                    *p = (g.beta == 0.0) ? g.alpha * acc[sx] : g.alpha * acc[sx] + g.beta * *p;
-                }
         }
     }
 }
 
-// long-side indices per thread of the skinny kernel: one.  (Two or four, processed one after the
-// other, halved the workgroups without adding loads in flight: on single items of 262144 x 20 x 20
-// and 65536 x 20 x 20 one index per thread took 28.8 and 13.3 us against 30.5 and 21.0 us.)
-constexpr int sk_rows(int) { return 1; }
+template <int KM>
+__global__ __launch_bounds__(SK_THREADS) void k_gemm_skinny(GemmArgs g, const Tile* __restrict__ blocks)
+{
+    const Tile tl = uniform(blocks[blockIdx.x]);
+    const xh_gemm_item it = uniform(g.items[tl.item]);
+    const bool wide = it.m <= it.n;  // wide: A is the small operand (C has S rows); else B
+    const int S = wide ? it.m : it.n, K = it.k, Lng = wide ? it.n : it.m;
+    const int L = tl.m0 + threadIdx.x;
+    if(L >= Lng) return;
+    // all K loads of a thread are issued before the first product, to keep many in flight
+    const bool lk = wide ? g.tb == 0 : g.ta != 0;  // the long operand's K entries of one index are contiguous
+    const double* xl = (wide ? g.B + it.b_off : g.A + it.a_off) + (lk ? int64_t(L) * K : int64_t(L));
+    const int64_t xs = lk ? 1 : Lng;
+    double x[KM];
+#pragma unroll
+    for(int kk = 0; kk < KM; ++kk) {
+        x[kk] = 0.0;
+        if(kk < K) x[kk] = xl[kk * xs];
+    }
+    double* c = g.C + it.c_off + (wide ? int64_t(L) * it.m : int64_t(L));
+    const int64_t cs = wide ? 1 : it.m;
+    auto store = [&](int sx, double a) {
+        double* q = c + sx * cs;
+        *q = (g.beta == 0.0) ? g.alpha * a : g.alpha * a + g.beta * *q;
+    };
+    const ConstDoubles sm = (ConstDoubles)(wide ? g.A + it.a_off : g.B + it.b_off);
+    if(wide ? g.ta != 0 : g.tb == 0)
+        skinny_sums<true>(sm, K, S, K, x, store);
+    else
+        skinny_sums<false>(sm, K, S, S, x, store);
+}
 
 // ---------------------------------------------------------------- FP64, skinny items, A through a permute
 // The skinny kernel with its long operand A read through a single-source permute of src, instead
 // of from the materialised permuted tensor (xh_gemm_gather).  Row r of an item's A block lies in
 // domain tree a and column kk in codomain tree b; the element is entry (r - start_a, kk - start_b)
-// of permute task task_base + a * ncod + b, and its source offset is
-//   src_off(t) + sum over legs of (leg index) * (leg stride in the source, times src_ld for a
-//   source column leg),
-// the domain legs' indices peeled off the row, the codomain legs' off the column.  The plan cuts
-// every item's rows into blocks of at most 256 rows that meet at most GA_SEG domain trees.  Per
-// (block tree, column) the block tabulates in LDS everything but the domain legs' terms (the
-// column's offset) and the domain legs' strides; a thread then adds (index x stride) over its
-// row's domain legs per column.  Coefficients are +1 or -1, so the operand is the source element,
-// negated for -1: the value the permute writes, up to the sign of a zero, which sums that start
-// from +0 do not see.  The sums run in the skinny kernel's order, so the product equals
-// permute + xh_gemm bit for bit.
+// of permute task (a, b), and its source offset is the offset of (a, kk) at row 0 (columns' terms
+// included) plus the row's indices along the domain legs times their source strides in (a, b).  The
+// plan tabulates both per domain tree, with the domain legs of extent 1 dropped and those that
+// lie behind one another in the source in every task of the tree joined.  It cuts every item's rows
+// into blocks of at most 256 rows that meet at most GA_SEG domain trees; a block copies its trees'
+// tables to LDS, one wavefront per tree, and a thread sums its row's terms once per codomain tree
+// and adds a column's offset per element.  One workgroup per block: a persistent loop waits for the
+// stores of a block before the loads of the next (187 and 189 us below).
+// Bound by the bytes, in columns that start at any element, and by the chain block, tables,
+// elements, operands: 22.7 M elements read and 44.2 M written (corner, chi 256) 155 us, 44.2 M read
+// and 22.7 M written 153, 3.5 TB/s.  (With the columns' offsets decoded by every block, a term
+// per domain leg and element from 64-bit strides, and the small operand in LDS: 197 and 192.)
+// Coefficients are +1 or -1, so the operand is the source element, negated for -1: the value the
+// permute writes, up to the sign of a zero, which sums that start from +0 do not see.  The sums
+// run in the skinny kernel's order, so the product equals permute + xh_gemm bit for bit.
 constexpr int GA_MAXR = 8;  // domain legs of a gather plan's permuted tensor (checked at plan creation)
-constexpr int GA_SEG = 4;   // domain trees one block may meet
+constexpr int GA_SEG = SK_THREADS / 64;  // domain trees one block may meet
+constexpr int GA_RUN = 16;  // consecutive blocks that run on one XCD (1: 157 and 160 us above; whole eighths differ in work: 225)
 struct GatherBlock {
-    int32_t item, row0, nrows, nseg;
-    int32_t a[GA_SEG];      // domain tree of each segment
-    int32_t start[GA_SEG];  // first row of that tree (segments ascend)
+    int64_t b_off, c_off;    // the item's
+    int64_t trees;           // its first domain tree in legs and neg
+    int64_t offs, strides;   // tables of its domain tree a at offs + a k and strides + a ncod nl
+    int32_t item, m, n, k, ncod;
+    uint32_t first;          // bit kk: column kk is the first of its codomain tree
+    int32_t row0, nrows, nseg;
+    int32_t a[GA_SEG];       // domain tree of each segment
+    int32_t start[GA_SEG];   // first row of that tree (segments ascend)
 };
-struct GatherItem {
-    int32_t task_base, ncod;
-    int64_t cols_off;  // per column kk < K: codomain tree b | (column inside it << 16)
-};
-struct GatherSrc {
-    int64_t off, ld;   // source subblock offset and leading dimension
-    int32_t neg, pad;  // 1: coefficient -1
+struct RowLeg {
+    uint32_t ext, magic, shift, pad;  // one of a domain tree's joined legs
 };
 struct GatherDev {
     const GatherBlock* blocks;
-    const GatherItem* items;  // per GEMM item
-    const int32_t* cols;
-    const xh::LegInfo* legs;  // ntasks * nlegs
-    const GatherSrc* src;     // per task
-    int32_t nlegs, new_rank, nblocks;
+    const int64_t* offs;        // per domain tree and column: source offset at row 0
+    const uint32_t* strides;    // per task and joined leg: source stride, low half
+    const uint32_t* strides_hi;  // high half; null where all are 0
+    const RowLeg* legs;         // per domain tree: nl joined legs
+    const uint32_t* neg;        // per domain tree: bit kk for a column whose task has coefficient -1
+    int32_t nl, new_rank, nblocks;
 };
 
 // The permute of the product folded into the stores (SCATTER): every product subblock (domain tree
 // a, codomain tree c) is the single source of one task of that permute, which fixes its place in
 // the output.  Per (block tree, product column) the block tabulates the column's destination
-// offset and the destination strides of the product's domain legs, which are the permuted left
-// operand's domain legs, so the row's indices are the ones decoded for the gather.
+// offset and the destination strides of the product's domain legs.
 struct ScatterItem {
-    int64_t grid_off, cols_off;  // product subblock (a, c) -> task grid[grid_off + a * ncod + c]; columns as GatherItem's
+    int64_t grid_off, cols_off;  // product subblock (a, c) -> task grid[grid_off + a * ncod + c]; columns at cols[cols_off ..]
     int32_t ncod, pad;
 };
 struct ScatterDev {
@@ -583,140 +606,150 @@ struct ScatterDev {
     int32_t nlegs;             // product legs (its domain legs first)
 };
 
-template <int MS, bool SCATTER>
-__global__ __launch_bounds__(SK_THREADS, SCATTER ? 1 : 4) void k_gemm_skinny_gather(GemmArgs g, GatherDev gd, const double* __restrict__ src, ScatterDev sd)
+template <int KM, bool SCATTER>
+__global__ __launch_bounds__(SK_THREADS, SCATTER ? 1 : (KM == 16 ? 6 : 4)) void k_gemm_skinny_gather(GemmArgs g, GatherDev gd, const double* __restrict__ src, ScatterDev sd)
 {
     constexpr int DS = SCATTER ? GA_SEG : 1, DC = SCATTER ? SK_MAX : 1, DR = SCATTER ? GA_MAXR : 1;
     __shared__ int64_t s_doff[DS][DC];      // per tree and product column: destination offset of the column
     __shared__ int64_t s_drs[DS][DC][DR];   // per tree and product column: destination strides of the domain legs
+    __shared__ xh::LegInfo s_dleg[DS][DR];  // per tree: its domain legs (extents, divisions)
     __shared__ uint32_t s_dneg[DS];         // bit c: the column's task has coefficient -1
-    __shared__ double sS[SK_KMAX * MS];                     // B, [kk][s]
-    __shared__ int64_t s_off[GA_SEG][SK_KMAX];              // per tree and column: the column's offset
-    __shared__ int64_t s_rs[GA_SEG][SK_KMAX][GA_MAXR];      // per tree and column: the domain legs' strides
-    __shared__ xh::LegInfo s_rleg[GA_SEG][GA_MAXR];         // per tree: its domain legs (extents, divisions)
-    __shared__ uint32_t s_neg[GA_SEG];                      // bit kk: the column's task has coefficient -1
-    const int R = gd.new_rank, NL = gd.nlegs;
-    for(int blk = blockIdx.x; blk < gd.nblocks; blk += gridDim.x) {
-        const GatherBlock bl = gd.blocks[blk];
-        const xh_gemm_item it = g.items[bl.item];
-        const GatherItem gi = gd.items[bl.item];
-        const int S = it.n, K = it.k;
-        __syncthreads();  // the previous block's reads of the shared tables are done
-        for(int e = threadIdx.x; e < K * MS; e += SK_THREADS) {
-            const int sx = e % MS, kk = e / MS;
-            double v = 0.0;
-            if(sx < S) v = g.tb ? g.B[it.b_off + int64_t(kk) * it.n + sx] : g.B[it.b_off + int64_t(sx) * K + kk];
-            sS[kk * MS + sx] = v;
+    __shared__ int64_t s_off[GA_SEG][KM];   // per tree: its tables
+    __shared__ uint32_t s_rs[GA_SEG][KM * GA_MAXR], s_rh[GA_SEG][KM * GA_MAXR];
+    __shared__ RowLeg s_rleg[GA_SEG][GA_MAXR];
+    __shared__ uint32_t s_neg[GA_SEG];
+    const int R = gd.new_rank, nl = gd.nl, lane = threadIdx.x & 63, wave = uniform(int(threadIdx.x >> 6));
+    const bool far = gd.strides_hi != nullptr;
+    // workgroup i runs on XCD i mod 8: each XCD takes runs of GA_RUN blocks, whose rows share cache lines
+    const int j = blockIdx.x / NPART, blk = ((j / GA_RUN) * NPART + blockIdx.x % NPART) * GA_RUN + j % GA_RUN;
+    if(blk >= gd.nblocks) return;
+    const GatherBlock bl = gd.blocks[blk];
+    const int S = bl.n, K = bl.k, ncod = bl.ncod, nseg = bl.nseg;
+    const uint32_t first = bl.first;
+    if(wave < nseg) {
+        const int64_t a = gd.blocks[blk].a[wave], tree = bl.trees + a;
+        if(lane < K) s_off[wave][lane] = gd.offs[bl.offs + a * K + lane];
+        const int64_t rs = bl.strides + a * ncod * nl;
+        for(int e = lane; e < ncod * nl; e += 64) {  // at most one codomain tree per column: ncod <= K
+            s_rs[wave][e] = gd.strides[rs + e];
+            if(far) s_rh[wave][e] = gd.strides_hi[rs + e];
         }
-        if(int(threadIdx.x) < GA_SEG) s_neg[threadIdx.x] = 0;
-        if constexpr(SCATTER)
-            if(int(threadIdx.x) < GA_SEG) s_dneg[threadIdx.x] = 0;
+        if(lane < nl) s_rleg[wave][lane] = gd.legs[tree * nl + lane];
+        if(lane == 0) s_neg[wave] = gd.neg[tree];
+    }
+    if constexpr(SCATTER) {
+        if(int(threadIdx.x) < GA_SEG) s_dneg[threadIdx.x] = 0;
         __syncthreads();
-        for(int e = threadIdx.x; e < bl.nseg * K; e += SK_THREADS) {
-            const int sg = e / K, kk = e % K;
-            const int32_t cb = gd.cols[gi.cols_off + kk];
-            const int t = gi.task_base + gd.blocks[blk].a[sg] * gi.ncod + (cb & 0xffff);
-            const GatherSrc so = gd.src[t];
-            const xh::LegInfo* Lg = gd.legs + int64_t(t) * NL;
-            // the codomain legs' terms of column kk (its index inside tree b peeled leg by leg)
+        const ScatterItem si = sd.items[bl.item];
+        const int NP = sd.nlegs;
+        for(int e = threadIdx.x; e < nseg * S; e += SK_THREADS) {
+            const int sg = e / S, c = e % S;
+            const int32_t cb = sd.cols[si.cols_off + c];
+            const int t = sd.grid[si.grid_off + int64_t(gd.blocks[blk].a[sg]) * si.ncod + (cb & 0xffff)];
+            const xh::LegInfo* Lg = sd.legs + int64_t(t) * NP;
             uint32_t x = static_cast<uint32_t>(cb >> 16);
-            int64_t off = so.off;
-            for(int k = R; k < NL; ++k) {
+            int64_t off = sd.dst_off[t];
+            for(int k = R; k < NP; ++k) {
                 const xh::LegInfo li = Lg[k];
                 const uint32_t q = xh::fdiv(x, li.magic, xh::leg_shift(li));
-                const uint32_t j = x - q * li.ext;
+                off += int64_t(x - q * li.ext) * li.stride;
                 x = q;
-                off += (li.flags & 256u) ? int64_t(j) * li.stride * so.ld : int64_t(j) * li.stride;
             }
-            s_off[sg][kk] = off;
+            s_doff[sg][c] = off;
             for(int k = 0; k < R; ++k) {
                 const xh::LegInfo li = Lg[k];
-                s_rs[sg][kk][k] = (li.flags & 256u) ? int64_t(li.stride) * so.ld : int64_t(li.stride);
-                if(kk == 0) s_rleg[sg][k] = li;
+                s_drs[sg][c][k] = li.stride;
+                if(c == 0) s_dleg[sg][k] = li;
             }
-            if(so.neg) atomicOr(&s_neg[sg], 1u << kk);
+            if(sd.neg[t]) atomicOr(&s_dneg[sg], 1u << c);
         }
-        if constexpr(SCATTER) {
-            const ScatterItem si = sd.items[bl.item];
-            const int NP = sd.nlegs;
-            for(int e = threadIdx.x; e < bl.nseg * S; e += SK_THREADS) {
-                const int sg = e / S, c = e % S;
-                const int32_t cb = sd.cols[si.cols_off + c];
-                const int t = sd.grid[si.grid_off + int64_t(gd.blocks[blk].a[sg]) * si.ncod + (cb & 0xffff)];
-                const xh::LegInfo* Lg = sd.legs + int64_t(t) * NP;
-                uint32_t x = static_cast<uint32_t>(cb >> 16);
-                int64_t off = sd.dst_off[t];
-                for(int k = R; k < NP; ++k) {
-                    const xh::LegInfo li = Lg[k];
-                    const uint32_t q = xh::fdiv(x, li.magic, xh::leg_shift(li));
-                    off += int64_t(x - q * li.ext) * li.stride;
-                    x = q;
-                }
-                s_doff[sg][c] = off;
-                for(int k = 0; k < R; ++k) s_drs[sg][c][k] = Lg[k].stride;
-                if(sd.neg[t]) atomicOr(&s_dneg[sg], 1u << c);
-            }
-        }
-        __syncthreads();
-        if(int(threadIdx.x) >= bl.nrows) continue;  // no barrier follows before the next block's first one
-        const int L = bl.row0 + threadIdx.x;
-        int sg = 0, first = bl.start[0];
+    }
+    __syncthreads();
+    if(int(threadIdx.x) >= bl.nrows) return;
+    const int L = bl.row0 + threadIdx.x;
+    int sg = 0, begin = bl.start[0];
 #pragma unroll
-        for(int q = 1; q < GA_SEG; ++q)
-            if(q < bl.nseg && bl.start[q] <= L) {
-                sg = q;
-                first = bl.start[q];
+    for(int q = 1; q < GA_SEG; ++q)
+        if(q < nseg && bl.start[q] <= L) {
+            sg = q;
+            begin = bl.start[q];
+        }
+    // the row's indices along the joined legs of its tree
+    const uint32_t in_tree = static_cast<uint32_t>(L - begin);
+    uint32_t x = in_tree, dig[GA_MAXR];
+#pragma unroll
+    for(int k = 0; k < GA_MAXR; ++k) {
+        dig[k] = 0;
+        if(k < nl) {
+            const RowLeg li = s_rleg[sg][k];
+            const uint32_t q = xh::fdiv(x, li.magic, li.shift);
+            dig[k] = x - q * li.ext;
+            x = q;
+        }
+    }
+    double xv[KM];
+    int64_t row = 0;
+    int tree = 0;  // nl times the codomain tree after the current one
+#pragma unroll
+    for(int kk = 0; kk < KM; ++kk) {
+        xv[kk] = 0.0;
+        if(kk < K) {
+            if((first >> kk) & 1u) {
+                row = 0;
+#pragma unroll
+                for(int k = 0; k < GA_MAXR; ++k)
+                    if(k < nl) {
+                        row += uint64_t(dig[k]) * s_rs[sg][tree + k];
+                        if(far) row += int64_t(uint64_t(dig[k]) * s_rh[sg][tree + k] << 32);
+                    }
+                tree += nl;
             }
-        // the row's domain-leg indices inside its tree
-        uint32_t x = static_cast<uint32_t>(L - first);
-        uint32_t dig[GA_MAXR];
+            xv[kk] = src[s_off[sg][kk] + row];
+        }
+    }
+    const uint32_t negm = s_neg[sg];
+    if(__any(negm != 0))
+#pragma unroll
+        for(int kk = 0; kk < KM; ++kk)
+            if((negm >> kk) & 1u) xv[kk] = -xv[kk];
+    const ConstDoubles sm = (ConstDoubles)(g.B + bl.b_off);
+    auto sums = [&](auto&& store) {
+        if(g.tb)
+            skinny_sums<false>(sm, K, S, S, xv, store);
+        else
+            skinny_sums<true>(sm, K, S, K, xv, store);
+    };
+    if constexpr(!SCATTER) {
+        double* base = g.C + bl.c_off + L;
+        const int64_t ld = bl.m;
+        sums([&](int c, double a) {
+            double* p = base + int64_t(c) * ld;
+            *p = (g.beta == 0.0) ? g.alpha * a : g.alpha * a + g.beta * *p;
+        });
+    } else {
+        // each output straight to its place in the permuted product: the column's offset plus
+        // (domain-leg index x destination stride) over the row's legs; 0 + c v with c = +-1,
+        // as the permute writes it (beta is 0)
+        const uint32_t dneg = s_dneg[sg];
+        uint32_t y = in_tree, dd[GA_MAXR];
 #pragma unroll
         for(int k = 0; k < GA_MAXR; ++k) {
-            dig[k] = 0;
+            dd[k] = 0;
             if(k < R) {
-                const xh::LegInfo li = s_rleg[sg][k];
-                const uint32_t q = xh::fdiv(x, li.magic, xh::leg_shift(li));
-                dig[k] = x - q * li.ext;
-                x = q;
+                const xh::LegInfo li = s_dleg[sg][k];
+                const uint32_t q = xh::fdiv(y, li.magic, xh::leg_shift(li));
+                dd[k] = y - q * li.ext;
+                y = q;
             }
         }
-        double xv[SK_KMAX];
+        sums([&](int c, double a) {
+            int64_t off = s_doff[sg][c];
 #pragma unroll
-        for(int kk = 0; kk < SK_KMAX; ++kk) {
-            xv[kk] = 0.0;
-            if(kk < K) {
-                int64_t off = s_off[sg][kk];
-#pragma unroll
-                for(int k = 0; k < GA_MAXR; ++k)
-                    if(k < R) off += int64_t(dig[k]) * s_rs[sg][kk][k];
-                xv[kk] = src[off];
-            }
-        }
-        const uint32_t negm = s_neg[sg];
-#pragma unroll
-        for(int kk = 0; kk < SK_KMAX; ++kk)
-            if((negm >> kk) & 1u) xv[kk] = -xv[kk];
-        if constexpr(!SCATTER) {
-            double* base = g.C + it.c_off + L;
-            const int64_t ld = it.m;
-            skinny_sums<MS>(sS, xv, K, S, [&](int c, double a) {
-                double* p = base + int64_t(c) * ld;
-                *p = (g.beta == 0.0) ? g.alpha * a : g.alpha * a + g.beta * *p;
-            });
-        } else {
-            // each output straight to its place in the permuted product: the column's offset plus
-            // (domain-leg index x destination stride) over the row's legs; 0 + c v with c = +-1,
-            // as the permute writes it (beta is 0)
-            const uint32_t dneg = s_dneg[sg];
-            skinny_sums<MS>(sS, xv, K, S, [&](int c, double a) {
-                int64_t off = s_doff[sg][c];
-#pragma unroll
-                for(int k = 0; k < GA_MAXR; ++k)
-                    if(k < R) off += int64_t(dig[k]) * s_drs[sg][c][k];
-                const double v = g.alpha * a;
-                g.C[off] = ((dneg >> c) & 1u) ? 0.0 - v : 0.0 + v;
-            });
-        }
+            for(int k = 0; k < GA_MAXR; ++k)
+                if(k < R) off += int64_t(dd[k]) * s_drs[sg][c][k];
+            const double v = g.alpha * a;
+            g.C[off] = ((dneg >> c) & 1u) ? 0.0 - v : 0.0 + v;
+        });
     }
 }
 
@@ -1122,7 +1155,7 @@ struct xh_gemm_plan : xh::PlanLife {
     TileList big128, rest64;  // FP64: items with large output sides in 128 x 128 tiles (is_big), the others in k_gemm_f64's shapes
     size_t lds64 = 0;         // LDS bytes of rest64's largest tile
     TileList skinny;          // FP64: blocks of 256 long-side indices of the skinny items (Tile.m0 = first index)
-    int sk_ms = 8;            // register width of the skinny kernel: 8, 16 or 32 >= every skinny item's short side
+    int sk_km = 16;           // register width of the skinny kernels: 16 or 32 >= every skinny item's K
     bool all64_built = false, any_tiles = false;
     bool skinny_kernel = false;  // skinny-shaped items run in the skinny kernel (use_skinny)
     bool is_skinny(const xh_gemm_item& it) const;
@@ -1285,15 +1318,14 @@ extern "C" int xh_gemm_plan_create(xh_ctx* ctx, const xh_gemm_item* items, int64
                 }
             }
         }
-        // skinny items: blocks of SK_THREADS * rows-per-thread long-side indices
+        // skinny items: blocks of SK_THREADS long-side indices
         for(const auto& it : v)
             if(it.m > 0 && it.n > 0 && is_skinny(it))
-                while(plan->sk_ms < std::min(it.m, it.n)) plan->sk_ms *= 2;
+                while(plan->sk_km < it.k) plan->sk_km *= 2;
         for(int id : order) {
             const xh_gemm_item& it = v[id];
             if(it.m == 0 || it.n == 0 || !is_skinny(it)) continue;
-            const int step = SK_THREADS * sk_rows(plan->sk_ms);
-            for(int l0 = 0; l0 < std::max(it.m, it.n); l0 += step) t_sk.push_back(Tile{id, l0, 0, 0});
+            for(int l0 = 0; l0 < std::max(it.m, it.n); l0 += SK_THREADS) t_sk.push_back(Tile{id, l0, 0, 0});
         }
         if(t_big.size() + t_rest.size() + t_sk.size() > 0x7fffffff) throw xh::Error(XH_EINVAL, "gemm plan: too many tiles");
         plan->skinny.ntiles = static_cast<int32_t>(t_sk.size());
@@ -1569,9 +1601,8 @@ void gemm_run(xh_ctx* ctx, const xh_gemm_plan* cplan, const double* A, const dou
         auto run = [&](int tiles) {
             if(precision == XH_FP64 && tiles == 0) {
                 if(plan->skinny.ntiles > 0) {
-                    auto* kern = plan->sk_ms <= 8 ? k_gemm_skinny<8, sk_rows(8)> : plan->sk_ms <= 16 ? k_gemm_skinny<16, sk_rows(16)> : k_gemm_skinny<32, sk_rows(32)>;
-                    const int grid = std::min<int>(plan->skinny.ntiles, ctx->num_cu * 8);
-                    hipLaunchKernelGGL(kern, dim3(grid), dim3(SK_THREADS), 0, ctx->stream, g, plan->skinny.d_tiles, plan->skinny.ntiles);
+                    auto* kern = plan->sk_km <= 16 ? k_gemm_skinny<16> : k_gemm_skinny<32>;
+                    hipLaunchKernelGGL(kern, dim3(unsigned(plan->skinny.ntiles)), dim3(SK_THREADS), 0, ctx->stream, g, plan->skinny.d_tiles);
                     xh::launch_check("k_gemm_skinny");
                 }
                 launch(plan->big128, f64_128, 2, G8_THREADS, lds128, "k_gemm_f64_128");
@@ -1581,9 +1612,8 @@ void gemm_run(xh_ctx* ctx, const xh_gemm_plan* cplan, const double* A, const dou
             } else if(precision == XH_OZAKI) {
                 if(!plan->oz_built) build_oz(ctx, plan);
                 if(plan->skinny.ntiles > 0) {
-                    auto* kern = plan->sk_ms <= 8 ? k_gemm_skinny<8, sk_rows(8)> : plan->sk_ms <= 16 ? k_gemm_skinny<16, sk_rows(16)> : k_gemm_skinny<32, sk_rows(32)>;
-                    const int grid = std::min<int>(plan->skinny.ntiles, ctx->num_cu * 8);
-                    hipLaunchKernelGGL(kern, dim3(grid), dim3(SK_THREADS), 0, ctx->stream, g, plan->skinny.d_tiles, plan->skinny.ntiles);
+                    auto* kern = plan->sk_km <= 16 ? k_gemm_skinny<16> : k_gemm_skinny<32>;
+                    hipLaunchKernelGGL(kern, dim3(unsigned(plan->skinny.ntiles)), dim3(SK_THREADS), 0, ctx->stream, g, plan->skinny.d_tiles);
                     xh::launch_check("k_gemm_skinny");
                 }
                 launch(plan->oz_rest, f64_64, 8, G_THREADS, lds64, "k_gemm_f64");
@@ -1744,6 +1774,9 @@ bool gather_eligible(const xh_gemm_plan* plan)
     return true;
 }
 
+// workgroups of a gather product: whole runs of GA_RUN blocks on every XCD
+unsigned gather_grid(int nblocks) { return unsigned((nblocks + NPART * GA_RUN - 1) / (NPART * GA_RUN)) * (NPART * GA_RUN); }
+
 void gather_plan_release(xh_ctx* ctx, xh::PlanLife* p)
 {
     auto* plan = static_cast<xh_gather_plan*>(p);
@@ -1834,22 +1867,33 @@ extern "C" int xh_gather_plan_create(xh_ctx* ctx, const xh_gemm_plan* gemm, cons
                 for(int k = 0; k < NR; ++k) plan->h_dext.push_back(pd.tasks[g.task_base + int64_t(a) * g.ncod].ext[k]);
         }
         // blocks of at most SK_THREADS rows meeting at most GA_SEG domain trees, in the GEMM plan's
-        // item order; per item the codomain tree and in-tree column of every column
+        // item order, and the places of the items' tables
+        struct TreeAt {
+            int64_t item;
+            int32_t a, nl = 0;
+            int32_t leg[GA_MAXR] = {};  // first domain leg of each joined leg
+            uint32_t ext[GA_MAXR] = {};
+            bool far = false;
+        };
         std::vector<GatherBlock> blocks;
-        std::vector<GatherItem> items(size_t(d->nitems), GatherItem{0, 0, 0});
-        std::vector<int32_t> cols;
+        std::vector<GatherBlock> items(size_t(d->nitems));  // an item's part of its blocks
+        std::vector<TreeAt> trees;
+        int64_t noffs = 0, npairs = 0;
         for(int64_t j = 0; j < d->nitems; ++j) {
             const xh_gemm_item& it = gemm->h_items[j];
             const xh_gather_item& g = d->items[j];
             if(it.m == 0 || it.n == 0) continue;
             const int32_t* ds = d->starts + g.starts_off;
             const int32_t* cs = ds + g.ndom + 1;
-            items[j] = GatherItem{g.task_base, g.ncod, int64_t(cols.size())};
-            for(int b = 0; b < g.ncod; ++b)
-                for(int c = cs[b]; c < cs[b + 1]; ++c) cols.push_back(b | ((c - cs[b]) << 16));
+            items[j] = GatherBlock{it.b_off, it.c_off, int64_t(trees.size()), noffs, npairs, int32_t(j), it.m, it.n, it.k, g.ncod, 0, 0, 0, 0, {}, {}};
+            for(int b = 0; b < g.ncod; ++b) items[j].first |= 1u << cs[b];
+            noffs += int64_t(g.ndom) * it.k;
+            npairs += int64_t(g.ndom) * g.ncod;
+            for(int a = 0; a < g.ndom; ++a) trees.push_back(TreeAt{j, a});
             int a = 0;
             for(int r = 0; r < it.m;) {
-                GatherBlock bl{int32_t(j), r, 0, 0, {}, {}};
+                GatherBlock bl = items[j];
+                bl.row0 = r;
                 const int end = std::min(it.m, r + SK_THREADS);
                 while(r < end && bl.nseg < GA_SEG) {
                     while(ds[a + 1] <= r) ++a;
@@ -1862,10 +1906,48 @@ extern "C" int xh_gather_plan_create(xh_ctx* ctx, const xh_gemm_plan* gemm, cons
                 blocks.push_back(bl);
             }
         }
-        if(blocks.size() > 0x7fffffff) throw xh::Error(XH_EINVAL, "gather plan: too many blocks");
+        if(blocks.size() > 0x7fffffff - NPART * GA_RUN) throw xh::Error(XH_EINVAL, "gather plan: too many blocks");
+        auto task_of = [&](const TreeAt& tr, int b) -> const xh_permute_task& {
+            const xh_gather_item& g = d->items[tr.item];
+            return pd.tasks[g.task_base + int64_t(tr.a) * g.ncod + b];
+        };
+        auto stride_of = [&](const xh_permute_task& tk, int k) { return tk.is_col[k] ? tk.sstride[k] * pd.sources[tk.src_begin].src_ld : tk.sstride[k]; };
+        // per domain tree: its joined legs
+        xp::parallel_ranges(trees.size(), 256, [&](size_t i0, size_t i1) {
+            for(size_t i = i0; i < i1; ++i) {
+                TreeAt& tr = trees[i];
+                const int ncod = d->items[tr.item].ncod;
+                const xh_permute_task& t0 = task_of(tr, 0);
+                for(int k = 0; k < NR; ++k) {
+                    if(t0.ext[k] == 1) continue;
+                    bool join = tr.nl > 0;
+                    for(int b = 0; b < ncod; ++b) {
+                        const xh_permute_task& tk = task_of(tr, b);
+                        const int64_t st = stride_of(tk, k);
+                        if(st >= (int64_t(1) << 32)) tr.far = true;
+                        if(join && st != stride_of(tk, tr.leg[tr.nl - 1]) * tr.ext[tr.nl - 1]) join = false;
+                    }
+                    if(join) {
+                        tr.ext[tr.nl - 1] *= t0.ext[k];
+                    } else {
+                        tr.leg[tr.nl] = k;
+                        tr.ext[tr.nl++] = t0.ext[k];
+                    }
+                }
+            }
+        });
+        int nl = 0;
+        bool far = false;
+        for(const TreeAt& tr : trees) {
+            nl = std::max(nl, int(tr.nl));
+            far = far || tr.far;
+        }
+        for(GatherBlock& bl : items) bl.strides *= nl;
+        for(GatherBlock& bl : blocks) bl.strides *= nl;
         xh::PackedUpload& up = plan->up;
-        const size_t bytes = xh::PackedUpload::packed_bytes({blocks.size() * sizeof(GatherBlock), items.size() * sizeof(GatherItem), cols.size() * sizeof(int32_t),
-                                                             size_t(NT * NL) * sizeof(xh::LegInfo), size_t(NT) * sizeof(GatherSrc)});
+        const size_t ntrees = trees.size(), nst = size_t(npairs * nl), nhi = far ? nst : 0;
+        const size_t bytes = xh::PackedUpload::packed_bytes({blocks.size() * sizeof(GatherBlock), size_t(noffs) * sizeof(int64_t),
+                                                             nst * sizeof(uint32_t), nhi * sizeof(uint32_t), ntrees * nl * sizeof(RowLeg), ntrees * sizeof(uint32_t)});
         if(bytes >= (size_t(1) << 18)) up.begin_pinned(ctx, bytes);
         auto put = [&up](const auto& vec) {
             using T = typename std::decay_t<decltype(vec)>::value_type;
@@ -1873,21 +1955,50 @@ extern "C" int xh_gather_plan_create(xh_ctx* ctx, const xh_gemm_plan* gemm, cons
             if(!vec.empty()) std::memcpy(up.host_ptr<T>(o), vec.data(), vec.size() * sizeof(T));
             return o;
         };
-        const size_t o_bl = put(blocks), o_it = put(items), o_co = put(cols);
-        const size_t o_lg = up.reserve<xh::LegInfo>(NT * NL), o_src = up.reserve<GatherSrc>(NT);
-        xh::LegInfo* lg = up.host_ptr<xh::LegInfo>(o_lg);
-        GatherSrc* gs = up.host_ptr<GatherSrc>(o_src);
-        xp::parallel_ranges(size_t(NT), 4096, [&](size_t t0, size_t t1) {
-            for(size_t t = t0; t < t1; ++t) {
-                const xh_permute_task& tk = pd.tasks[t];
-                for(int k = 0; k < NL; ++k) lg[t * NL + k] = xh::make_leg(tk.ext[k], tk.sstride[k], tk.is_col[k] != 0);
-                const xh_permute_source& so = pd.sources[tk.src_begin];
-                gs[t] = GatherSrc{so.src_off, so.src_ld, so.coeff < 0.0 ? 1 : 0, 0};
+        const size_t o_bl = put(blocks);
+        const size_t o_of = up.reserve<int64_t>(noffs), o_st = up.reserve<uint32_t>(int64_t(nst)), o_hi = up.reserve<uint32_t>(int64_t(nhi)),
+                     o_lg = up.reserve<RowLeg>(int64_t(ntrees * nl)), o_ng = up.reserve<uint32_t>(int64_t(ntrees));
+        int64_t* h_of = up.host_ptr<int64_t>(o_of);
+        uint32_t *h_st = up.host_ptr<uint32_t>(o_st), *h_hi = up.host_ptr<uint32_t>(o_hi), *h_ng = up.host_ptr<uint32_t>(o_ng);
+        RowLeg* h_lg = up.host_ptr<RowLeg>(o_lg);
+        xp::parallel_ranges(ntrees, 256, [&](size_t i0, size_t i1) {
+            for(size_t i = i0; i < i1; ++i) {
+                const TreeAt& tr = trees[i];
+                const GatherBlock& gi = items[tr.item];
+                for(int q = 0; q < nl; ++q) {
+                    const uint32_t ext = q < tr.nl ? tr.ext[q] : 1u;
+                    const xh::FastDiv fd = xh::make_fastdiv(ext);
+                    h_lg[i * nl + q] = RowLeg{ext, fd.magic, fd.shift, 0};
+                }
+                int64_t* off = h_of + gi.offs + int64_t(tr.a) * gemm->h_items[tr.item].k;
+                uint32_t neg = 0;
+                int kk = 0;
+                for(int b = 0; b < gi.ncod; ++b) {
+                    const xh_permute_task& tk = task_of(tr, b);
+                    const xh_permute_source& so = pd.sources[tk.src_begin];
+                    for(int q = 0; q < nl; ++q) {
+                        const uint64_t st = q < tr.nl ? uint64_t(stride_of(tk, tr.leg[q])) : 0;
+                        const int64_t at = gi.strides + (int64_t(tr.a) * gi.ncod + b) * nl + q;
+                        h_st[at] = uint32_t(st);
+                        if(far) h_hi[at] = uint32_t(st >> 32);
+                    }
+                    for(int64_t c = 0; c < tk.cols; ++c, ++kk) {  // column kk: its index along the codomain legs
+                        int64_t x = c, o = so.src_off;
+                        for(int k = NR; k < NL; ++k) {
+                            if(tk.ext[k] == 1) continue;
+                            o += (x % tk.ext[k]) * stride_of(tk, k);
+                            x /= tk.ext[k];
+                        }
+                        off[kk] = o;
+                        if(so.coeff < 0.0) neg |= 1u << kk;
+                    }
+                }
+                h_ng[i] = neg;
             }
         });
         up.upload(ctx);
-        plan->dev = GatherDev{up.ptr<GatherBlock>(o_bl), up.ptr<GatherItem>(o_it), up.ptr<int32_t>(o_co), up.ptr<xh::LegInfo>(o_lg), up.ptr<GatherSrc>(o_src),
-                              NL, NR, static_cast<int32_t>(blocks.size())};
+        plan->dev = GatherDev{up.ptr<GatherBlock>(o_bl), up.ptr<int64_t>(o_of), up.ptr<uint32_t>(o_st),
+                              far ? up.ptr<uint32_t>(o_hi) : nullptr, up.ptr<RowLeg>(o_lg), up.ptr<uint32_t>(o_ng), nl, NR, static_cast<int32_t>(blocks.size())};
         plan->gemm = gemm;
         plan->src_elems = d->src_elems;
     });
@@ -1926,8 +2037,8 @@ extern "C" int xh_gemm_gather(xh_ctx* ctx, const xh_gemm_plan* plan, const xh_ga
         const bool timed = ctx->gemm_timing;
         if(timed) xh::gemm_timer_begin(ctx);
         GemmArgs g{plan->d_items, plan->d_ext, nullptr, {}, plan->ta, plan->tb, nullptr, B, C, nullptr, alpha, beta};
-        auto* kern = plan->sk_ms <= 8 ? k_gemm_skinny_gather<8, false> : plan->sk_ms <= 16 ? k_gemm_skinny_gather<16, false> : k_gemm_skinny_gather<32, false>;
-        const int grid = std::min<int>(gp->dev.nblocks, ctx->num_cu * 8);
+        auto* kern = plan->sk_km <= 16 ? k_gemm_skinny_gather<16, false> : k_gemm_skinny_gather<32, false>;
+        const unsigned grid = gather_grid(gp->dev.nblocks);
         if(grid > 0) hipLaunchKernelGGL(kern, dim3(grid), dim3(SK_THREADS), 0, ctx->stream, g, gp->dev, src, ScatterDev{});
         xh::launch_check("k_gemm_skinny_gather");
         if(timed) xh::gemm_timer_end(ctx, plan->flops, launch_items(ctx, plan));
@@ -2086,8 +2197,8 @@ extern "C" int xh_gemm_gather_scatter(xh_ctx* ctx, const xh_gemm_plan* plan, con
         const bool timed = ctx->gemm_timing;
         if(timed) xh::gemm_timer_begin(ctx);
         GemmArgs g{plan->d_items, plan->d_ext, nullptr, {}, plan->ta, plan->tb, nullptr, B, dst, nullptr, alpha, 0.0};
-        auto* kern = plan->sk_ms <= 8 ? k_gemm_skinny_gather<8, true> : plan->sk_ms <= 16 ? k_gemm_skinny_gather<16, true> : k_gemm_skinny_gather<32, true>;
-        const int grid = std::min<int>(gp->dev.nblocks, ctx->num_cu * 8);
+        auto* kern = plan->sk_km <= 16 ? k_gemm_skinny_gather<16, true> : k_gemm_skinny_gather<32, true>;
+        const unsigned grid = gather_grid(gp->dev.nblocks);
         if(grid > 0) hipLaunchKernelGGL(kern, dim3(grid), dim3(SK_THREADS), 0, ctx->stream, g, gp->dev, src, sp->dev);
         xh::launch_check("k_gemm_skinny_gather");
         if(timed) xh::gemm_timer_end(ctx, plan->flops, launch_items(ctx, plan));
