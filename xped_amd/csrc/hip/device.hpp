@@ -369,12 +369,21 @@ inline void* slab_take(xh_ctx* ctx, size_t bytes)
     return static_cast<char*>(ctx->slab.p) + off;
 }
 
+// A few KB of host memory to the device as the arguments of a small kernel (ctx.hip), in stream order:
+// they are copied at the launch, so src may go as soon as this returns.
+constexpr size_t PUT_MAX = 3584;
+void put_small(xh_ctx* ctx, void* dst, const void* src, size_t bytes);
+
 // Asynchronous copy of host memory to the device, ordered on the context stream; the caller may
 // reuse or free src as soon as this returns.  Not for a stream under graph capture (the graph
 // would copy from the staging memory again at every replay).
 inline void upload_async(xh_ctx* ctx, void* dst, const void* src, size_t bytes)
 {
     if(bytes == 0) return;
+    if(bytes <= PUT_MAX) {
+        put_small(ctx, dst, src, bytes);
+        return;
+    }
     if(bytes <= SLAB_BYTES / 4) {
         void* s = slab_take(ctx, bytes);
         std::memcpy(s, src, bytes);
