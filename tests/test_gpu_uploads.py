@@ -48,3 +48,33 @@ def test_ranges(rt, n):
     assert L.xh_range_sumsq(ctx, off.ctypes.data_as(i64), ln.ctypes.data_as(i64), n, p, out.ctypes.data_as(C.POINTER(C.c_double))) == 0
     L.xh_free(ctx, p)
     assert np.array_equal(out, [np.sum(x[o:o + k] ** 2) for o, k in zip(off, ln)])
+
+
+@pytest.mark.parametrize("transpose", [0, 1])
+@pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 70])
+def test_rectangles(rt, n, transpose):
+    """Up to 16 rectangles are kernel arguments, more are uploaded."""
+    L, ctx = lib(), rt.ctx()
+    r = np.random.default_rng(n)
+
+    class Rect(C.Structure):
+        _fields_ = [("src_off", C.c_int64), ("src_ld", C.c_int64), ("dst_off", C.c_int64), ("dst_ld", C.c_int64), ("rows", C.c_int32), ("cols", C.c_int32),
+                    ("factor", C.c_double), ("transpose", C.c_int32)]
+
+    src, rects, at = r.uniform(-1, 1, 5000), [], 0
+    for q in range(n):
+        m, k = int(r.integers(0, 40)), int(r.integers(1, 40))
+        rects.append(Rect(int(r.integers(0, 1000)), (k if transpose else m) + q % 3, at, m + q % 2, m, k, 1.0 if q % 2 else -2.0, transpose))
+        at += (m + q % 2) * k
+    out = np.full(max(at, 1), 7.0)
+    exp, a, b = out.copy(), _on_device(rt, src), _on_device(rt, out)
+    copy = L.xh_copy_rects
+    copy.argtypes = [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int64]
+    assert copy(ctx, a, b, C.addressof((Rect * n)(*rects)), n) == 0
+    L.xh_download(ctx, out.ctypes.data, b, out.nbytes)
+    L.xh_free(ctx, a)
+    L.xh_free(ctx, b)
+    for x in rects:
+        i, j = np.meshgrid(np.arange(x.rows), np.arange(x.cols), indexing="ij")
+        exp[x.dst_off + i + j * x.dst_ld] = x.factor * src[x.src_off + (j + i * x.src_ld if transpose else i + j * x.src_ld)]
+    assert np.array_equal(out, exp)
