@@ -342,7 +342,7 @@ def run_c4(args):
                               "flops_per_step": fast["gemm_timed_flops"], "kernel_ms_per_step": round(fast["gemm_kernel_ms"], 3),
                               "randomized_svd_products": {"achieved": round(sk_fl / (sk_ms * 1e-3) / 1e12, 4) if sk_ms > 0 else 0.0, "launches": sk_n,
                                                           "flops": sk_fl, "kernel_ms": round(sk_ms, 3)}},
-        "permute_roofline": {"bound": "hbm", "kernel": "k_permute_gather + k_permute_transpose",
+        "permute_roofline": {"bound": "hbm", "kernel": "k_permute_compact + k_permute_gather + k_permute_transpose",
                              "achieved": round(fast["permute_bytes"] / (fast["permute_ms"] * 1e-3) / 1e9, 1) if fast["permute_ms"] > 0 else 0.0,
                              "peak": 8000.0, "unit": "GB/s",
                              "frac": round(fast["permute_bytes"] / (fast["permute_ms"] * 1e-3) / 1e9 / 8000.0, 4) if fast["permute_ms"] > 0 else 0.0,
