@@ -155,3 +155,19 @@ def test_block_chol_inv_across_kernel_edges(rt):
     x = x.reshape(n, n).T
     g = b + 0.5 * np.trace(b) / n * np.eye(n)
     assert np.linalg.norm(x.T @ g @ x - np.eye(n)) <= 4.0 * n * EPS * np.linalg.cond(g)
+
+
+@pytest.mark.parametrize("n", [16, 17, 32, 33, 100, 192, 193, 300])
+def test_block_chol_inv_exact(rt, n):
+    """R = D (I + N) with powers of two on D and N = +-1 from even rows to odd columns, so N N = 0 and
+    R^-1 = (I - N) D^-1.  Every intermediate is a small dyadic number, so the result has to be exact:
+    one element of a tile read before the lane that updates it has stored it would show."""
+    r = np.random.default_rng(n)
+    N = np.triu(r.choice([-1.0, 0.0, 1.0], (n, n)), 1)
+    N[1::2], N[:, ::2] = 0.0, 0.0
+    d = r.choice([0.5, 1.0, 2.0], n)
+    R = d[:, None] * (np.eye(n) + N)
+    G = R.T @ R
+    shift = (C.c_double * 1)(0.0)
+    x, = _run(rt, lambda ctx, arr, k, dA, dX: lib().xh_block_chol_inv(ctx, arr, k, dA, dX, shift), [G], (n * n,), [_lib.xh_factor_item(0, 0, 0, 0, n, n)])
+    assert np.array_equal(x.reshape(n, n).T, (np.eye(n) - N) / d[None, :])

@@ -730,6 +730,10 @@ __global__ __launch_bounds__(CI_THREADS) void k_chol_inv(FactorArgs fa)
         __syncthreads();
         if(wave == 0) {
             update(p, p + 1, p + 1);
+            // factor's lanes read elements that other lanes of this wave have just stored
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
             factor(p + 1);
         } else {
             int left = wave;  // tiles of the trailing triangle by columns; number 0 is wave 0's
