@@ -1,8 +1,9 @@
 """Skinny FP64 products (short side and K at most 32) and the gather product at their edges (needs an
 MI355X), against numpy within k u |A| |B| elementwise (Higham, Accuracy and Stability of Numerical
 Algorithms, 2nd ed., section 3.5), doubled for the reference's own: K around the multiples of 4,
-short sides around the sums of one pass, all transposes, non-finite entries, domain legs that drop
-out, join and do not, several domain trees per workgroup, source strides past 32 bits."""
+short sides around the sums of one pass, calls whose short sides are all at most 8 (scalar operands)
+and others (operands from LDS), all transposes, non-finite entries, domain legs that drop out, join
+and do not, several domain trees per workgroup, source strides past 32 bits."""
 import ctypes as C
 
 import numpy as np
@@ -19,12 +20,13 @@ SHORT = [1, 2, 3, 4, 5, 8, 9, 17, 31, 32]
 
 
 @pytest.mark.parametrize("ta,tb", [(0, 0), (1, 0), (0, 1), (1, 1)])
+@pytest.mark.parametrize("short", [SHORT, [1, 2, 3, 4, 5, 7, 8]], ids=["s32", "s8"])
 @pytest.mark.parametrize("ks", [(1, 3, 4, 5, 8, 9, 11, 12, 13, 16), (17, 20, 21, 24, 25, 28, 29, 31, 32)], ids=["k16", "k32"])
-def test_skinny_products(rt, ta, tb, ks):
+def test_skinny_products(rt, ta, tb, ks, short):
     r = np.random.default_rng(5)
     mats = []
     for i, k in enumerate(ks):
-        for j, s in enumerate(SHORT):
+        for j, s in enumerate(short):
             long = (33, 256, 257, 700)[(i + j) % 4]
             m, n = (s, long) if (i + j // 2) % 2 else (long, s)
             A, B = r.uniform(-1, 1, (m, k)), r.uniform(-1, 1, (k, n))
@@ -38,6 +40,19 @@ def test_skinny_products(rt, ta, tb, ks):
         assert not np.isfinite(c[~rows]).any() and not np.isfinite(c[:, ~cols]).any()
 
 
+@pytest.mark.parametrize("ta,tb", [(0, 0), (1, 0), (0, 1), (1, 1)])
+@pytest.mark.parametrize("k", [7, 16, 23, 32])
+def test_skinny_variants_same_bits(rt, ta, tb, k):
+    """The variant follows the largest short side and K of the call; an item's sums do not."""
+    r = np.random.default_rng(k)
+    mats = [(r.uniform(-1, 1, (m, k)), r.uniform(-1, 1, (k, n))) for m, n in ((500, 8), (3, 300), (700, 1), (6, 257))]
+    wide = [(r.uniform(-1, 1, (400, kw)), r.uniform(-1, 1, (kw, 32))) for kw in (k, 32)]
+    alone = _products(rt, mats, ta, tb)
+    for w in wide:
+        for a, b in zip(alone, _products(rt, mats + [w], ta, tb)):
+            assert np.array_equal(a, b)
+
+
 class _GatherItem(C.Structure):
     _fields_ = [("task_base", C.c_int32), ("ndom", C.c_int32), ("ncod", C.c_int32), ("pad", C.c_int32), ("starts_off", C.c_int64)]
 
@@ -48,8 +63,9 @@ class _GatherDesc(C.Structure):
 
 
 @pytest.mark.parametrize("far", [0, 1 << 32], ids=["near", "far"])
+@pytest.mark.parametrize("ns", [(1, 3, 8, 11), (1, 5, 8), (17, 32)], ids=["n11", "n8", "n32"])
 @pytest.mark.parametrize("kmax", [12, 32])
-def test_gather_product(rt, kmax, far):
+def test_gather_product(rt, kmax, ns, far):
     """far: one domain leg of extent 2 whose source entries lie 2^32 elements apart (a 34 GB source)."""
     r = np.random.default_rng(kmax)
     L, ctx = lib(), rt.ctx()
@@ -57,7 +73,7 @@ def test_gather_product(rt, kmax, far):
     src = r.uniform(-1, 1, W)
     tasks, sources, starts, gitems, gemms, ops = [], [], [], [], [], []
     bo = co = 0
-    for n in (1, 3, 8, 11):
+    for n in ns:
         dom = [[int(x) for x in (r.choice([1, 2, 45]), r.choice([1, 3]), 2 if far else r.choice([1, 2, 7]))] for _ in range(40)]
         cod = []
         while sum(a * b for a, b in cod) < kmax - 4:

@@ -434,12 +434,27 @@ constexpr size_t tile_lds(bool ta, bool tb, int tm, int tn) { return 2 * sizeof(
 // bound by the bytes of the long operand and of C, not by arithmetic: a 16 x 16 matrix-core tile
 // would waste most of its work on them.  One thread per index of the long side (256 per
 // workgroup) reads that index's K entries of the long operand into registers and writes its S
-// outputs, each a sum over kk in order.  The small operand is the same for every lane, so its
-// entries come through scalar loads and are the scalar operands of the multiply-adds.  (Staged in
-// LDS and read as broadcasts it was bound by them: a 16-byte broadcast keeps the LDS of a CU busy
-// for 8 cycles and feeds two multiply-adds, of which the four SIMDs do one a cycle.)  KM: 16 or 32
-// >= K, for the registers (48 and 88).
+// outputs, each a sum over kk in order.  The small operand is the same for every lane and comes
+// either way, with the same sums:
+//  * staged in LDS and read as broadcasts, MH sums at a time (skinny_sums_lds);
+//  * through scalar loads, as the scalar operands of the multiply-adds (skinny_sums): nothing is
+//    staged, but the scalar registers hold the operands of 1 to 8 sums only, and every pass of so
+//    many waits for its own.
+// KM: 16 or 32 >= K, for the registers.
 constexpr int SK_MAX = 32, SK_KMAX = 32, SK_THREADS = 256;
+// The largest short side of a call with scalar operands.  Times of a call of one item in us, LDS with a
+// workgroup looping over blocks | scalar operands | as here:
+//   long side 262144, K 16, S  8                     12.2 | 10.7 | 10.7  (scalar)
+//   long side 262144, K 20, S 16, all transposed     32.7 | 67   | 32.0  (each pass stores a part of every
+//                                                                  line of C, which is long gone from L2)
+//   long side 262144, K  8, S 32                     19.6 | 20.0 | 15.2
+//   long side   3000, K 16, S 32                      9.3 | 11.8 |  7.9
+//   long side     40, K  2, S 32                      5.1 |  6.7 |  4.2
+// With K above 16 scalar operands also lose at S <= 8 where the long operand is contiguous along K
+// (long side 65536, K 32, S 8: 10.3 | 13.1 | 10.8), so the plain product uses LDS there as well, 8 sums
+// at a time.  The gather product with S <= 8 is faster with scalar operands up to K 32 (262144 rows, K 16:
+// S 8 16.1 | 15.5 | 15.5, S 32 23.8 | 32.4 | 22.6).
+constexpr int SK_SCALAR = 8;
 
 // Read-only memory whose loads at uniform addresses go through the scalar cache.
 using ConstDoubles = const double __attribute__((address_space(4)))*;
@@ -511,13 +526,49 @@ __device__ __forceinline__ void skinny_sums(ConstDoubles b, int K, int S, int64_
     }
 }
 
-template <int KM>
+// The same sums with the small operand in LDS, entry (kk, s) at sS[kk SK_MAX + s], MH at a time.
+template <int MH, int KM, class Store>
+__device__ __forceinline__ void skinny_sums_lds(const double* __restrict__ sS, int K, int S, const double (&x)[KM], Store&& store)
+{
+    for(int s = 0; s < S; s += MH) {
+        double acc[MH];
+#pragma unroll
+        for(int j = 0; j < MH; ++j) acc[j] = 0.0;
+#pragma unroll
+        for(int kk = 0; kk < KM; ++kk)
+            if(kk < K)
+#pragma unroll
+                for(int j = 0; j < MH; ++j) acc[j] = __builtin_fma(sS[kk * SK_MAX + s + j], x[kk], acc[j]);
+#pragma unroll
+        for(int j = 0; j < MH; ++j)
+            if(s + j < S) store(s + j, acc[j]);
+    }
+}
+// Entry (kk, s) of the small operand, at b[s ld + kk] (kc) or b[kk ld + s], to LDS; what lies past S
+// only reaches sums that are not stored.
+__device__ __forceinline__ void stage_small(double* __restrict__ sS, const double* __restrict__ b, int K, int S, int64_t ld, bool kc)
+{
+    for(int e = threadIdx.x; e < K * SK_MAX; e += SK_THREADS) {
+        const int s = e % SK_MAX, kk = e / SK_MAX;
+        if(s < S) sS[e] = kc ? b[s * ld + kk] : b[kk * ld + s];
+    }
+}
+
+// MH: sums at a time from LDS, 0: scalar operands
+template <int KM, int MH>
 __global__ __launch_bounds__(SK_THREADS) void k_gemm_skinny(GemmArgs g, const Tile* __restrict__ blocks)
 {
+    __shared__ double sS[MH > 0 ? KM * SK_MAX : 1];
     const Tile tl = uniform(blocks[blockIdx.x]);
     const xh_gemm_item it = uniform(g.items[tl.item]);
     const bool wide = it.m <= it.n;  // wide: A is the small operand (C has S rows); else B
     const int S = wide ? it.m : it.n, K = it.k, Lng = wide ? it.n : it.m;
+    const bool kc = wide ? g.ta != 0 : g.tb == 0;  // the small operand's K entries of one output are contiguous
+    const double* small = wide ? g.A + it.a_off : g.B + it.b_off;
+    if constexpr(MH > 0) {
+        stage_small(sS, small, K, S, kc ? K : S, kc);
+        __syncthreads();
+    }
     const int L = tl.m0 + threadIdx.x;
     if(L >= Lng) return;
     // all K loads of a thread are issued before the first product, to keep many in flight
@@ -536,11 +587,12 @@ __global__ __launch_bounds__(SK_THREADS) void k_gemm_skinny(GemmArgs g, const Ti
         double* q = c + sx * cs;
         *q = (g.beta == 0.0) ? g.alpha * a : g.alpha * a + g.beta * *q;
     };
-    const ConstDoubles sm = (ConstDoubles)(wide ? g.A + it.a_off : g.B + it.b_off);
-    if(wide ? g.ta != 0 : g.tb == 0)
-        skinny_sums<true>(sm, K, S, K, x, store);
+    if constexpr(MH > 0)
+        skinny_sums_lds<MH>(sS, K, S, x, store);
+    else if(kc)
+        skinny_sums<true>((ConstDoubles)small, K, S, K, x, store);
     else
-        skinny_sums<false>(sm, K, S, S, x, store);
+        skinny_sums<false>((ConstDoubles)small, K, S, S, x, store);
 }
 
 // ---------------------------------------------------------------- FP64, skinny items, A through a permute
@@ -554,17 +606,17 @@ __global__ __launch_bounds__(SK_THREADS) void k_gemm_skinny(GemmArgs g, const Ti
 // into blocks of at most 256 rows that meet at most GA_SEG domain trees; a block copies its trees'
 // tables to LDS, one wavefront per tree, and a thread sums its row's terms once per codomain tree
 // and adds a column's offset per element.  One workgroup per block: a persistent loop waits for the
-// stores of a block before the loads of the next (187 and 189 us below).
+// stores of a block before the loads of the next (30 us more on each of the products below).
 // Bound by the bytes, in columns that start at any element, and by the chain block, tables,
-// elements, operands: 22.7 M elements read and 44.2 M written (corner, chi 256) 155 us, 44.2 M read
-// and 22.7 M written 153, 3.5 TB/s.  (With the columns' offsets decoded by every block, a term
-// per domain leg and element from 64-bit strides, and the small operand in LDS: 197 and 192.)
+// elements, operands: 22.7 M elements read and 44.2 M written (corner, chi 256) 146 us, 44.2 M read
+// and 22.7 M written 163, 3.5 TB/s.  (With the columns' offsets decoded by every block, a term
+// per domain leg and element from 64-bit strides, and a persistent loop: 197 and 192.)
 // Coefficients are +1 or -1, so the operand is the source element, negated for -1: the value the
 // permute writes, up to the sign of a zero, which sums that start from +0 do not see.  The sums
 // run in the skinny kernel's order, so the product equals permute + xh_gemm bit for bit.
 constexpr int GA_MAXR = 8;  // domain legs of a gather plan's permuted tensor (checked at plan creation)
 constexpr int GA_SEG = SK_THREADS / 64;  // domain trees one block may meet
-constexpr int GA_RUN = 16;  // consecutive blocks that run on one XCD (1: 157 and 160 us above; whole eighths differ in work: 225)
+constexpr int GA_RUN = 16;  // consecutive blocks that run on one XCD (with scalar operands: 155 and 153 us above, runs of 1 157 and 160, whole eighths 225, as they differ in work)
 struct GatherBlock {
     int64_t b_off, c_off;    // the item's
     int64_t trees;           // its first domain tree in legs and neg
@@ -606,8 +658,8 @@ struct ScatterDev {
     int32_t nlegs;             // product legs (its domain legs first)
 };
 
-template <int KM, bool SCATTER>
-__global__ __launch_bounds__(SK_THREADS, SCATTER ? 1 : (KM == 16 ? 6 : 4)) void k_gemm_skinny_gather(GemmArgs g, GatherDev gd, const double* __restrict__ src, ScatterDev sd)
+template <int KM, int MH, bool SCATTER>
+__global__ __launch_bounds__(SK_THREADS, SCATTER ? 1 : (KM == 16 && MH == 0 ? 6 : 4)) void k_gemm_skinny_gather(GemmArgs g, GatherDev gd, const double* __restrict__ src, ScatterDev sd)
 {
     constexpr int DS = SCATTER ? GA_SEG : 1, DC = SCATTER ? SK_MAX : 1, DR = SCATTER ? GA_MAXR : 1;
     __shared__ int64_t s_doff[DS][DC];      // per tree and product column: destination offset of the column
@@ -618,6 +670,7 @@ __global__ __launch_bounds__(SK_THREADS, SCATTER ? 1 : (KM == 16 ? 6 : 4)) void 
     __shared__ uint32_t s_rs[GA_SEG][KM * GA_MAXR], s_rh[GA_SEG][KM * GA_MAXR];
     __shared__ RowLeg s_rleg[GA_SEG][GA_MAXR];
     __shared__ uint32_t s_neg[GA_SEG];
+    __shared__ double sS[MH > 0 ? KM * SK_MAX : 1];
     const int R = gd.new_rank, nl = gd.nl, lane = threadIdx.x & 63, wave = uniform(int(threadIdx.x >> 6));
     const bool far = gd.strides_hi != nullptr;
     // workgroup i runs on XCD i mod 8: each XCD takes runs of GA_RUN blocks, whose rows share cache lines
@@ -637,6 +690,7 @@ __global__ __launch_bounds__(SK_THREADS, SCATTER ? 1 : (KM == 16 ? 6 : 4)) void 
         if(lane < nl) s_rleg[wave][lane] = gd.legs[tree * nl + lane];
         if(lane == 0) s_neg[wave] = gd.neg[tree];
     }
+    if constexpr(MH > 0) stage_small(sS, g.B + bl.b_off, K, S, g.tb ? S : K, g.tb == 0);
     if constexpr(SCATTER) {
         if(int(threadIdx.x) < GA_SEG) s_dneg[threadIdx.x] = 0;
         __syncthreads();
@@ -714,7 +768,9 @@ __global__ __launch_bounds__(SK_THREADS, SCATTER ? 1 : (KM == 16 ? 6 : 4)) void 
             if((negm >> kk) & 1u) xv[kk] = -xv[kk];
     const ConstDoubles sm = (ConstDoubles)(g.B + bl.b_off);
     auto sums = [&](auto&& store) {
-        if(g.tb)
+        if constexpr(MH > 0)
+            skinny_sums_lds<MH>(sS, K, S, xv, store);
+        else if(g.tb)
             skinny_sums<false>(sm, K, S, S, xv, store);
         else
             skinny_sums<true>(sm, K, S, K, xv, store);
@@ -1156,6 +1212,7 @@ struct xh_gemm_plan : xh::PlanLife {
     size_t lds64 = 0;         // LDS bytes of rest64's largest tile
     TileList skinny;          // FP64: blocks of 256 long-side indices of the skinny items (Tile.m0 = first index)
     int sk_km = 16;           // register width of the skinny kernels: 16 or 32 >= every skinny item's K
+    int sk_short = 0;         // the largest short side of the skinny items
     bool all64_built = false, any_tiles = false;
     bool skinny_kernel = false;  // skinny-shaped items run in the skinny kernel (use_skinny)
     bool is_skinny(const xh_gemm_item& it) const;
@@ -1320,8 +1377,10 @@ extern "C" int xh_gemm_plan_create(xh_ctx* ctx, const xh_gemm_item* items, int64
         }
         // skinny items: blocks of SK_THREADS long-side indices
         for(const auto& it : v)
-            if(it.m > 0 && it.n > 0 && is_skinny(it))
+            if(it.m > 0 && it.n > 0 && is_skinny(it)) {
                 while(plan->sk_km < it.k) plan->sk_km *= 2;
+                plan->sk_short = std::max(plan->sk_short, std::min(it.m, it.n));
+            }
         for(int id : order) {
             const xh_gemm_item& it = v[id];
             if(it.m == 0 || it.n == 0 || !is_skinny(it)) continue;
@@ -1597,25 +1656,24 @@ void gemm_run(xh_ctx* ctx, const xh_gemm_plan* cplan, const double* A, const dou
         auto* f64_128 = fta ? (ftb ? k_gemm_f64_128<true, true> : k_gemm_f64_128<true, false>) : (ftb ? k_gemm_f64_128<false, true> : k_gemm_f64_128<false, false>);
         auto* f64_64 = fta ? (ftb ? k_gemm_f64<true, true> : k_gemm_f64<true, false>) : (ftb ? k_gemm_f64<false, true> : k_gemm_f64<false, false>);
         const size_t lds128 = tile_lds(fta, ftb, BM2, BN2), lds64 = tile_lds(fta, ftb, BM, BN);
+        auto launch_skinny = [&] {
+            if(plan->skinny.ntiles == 0) return;
+            auto* kern = plan->sk_short > SK_SCALAR ? (plan->sk_km <= 16 ? k_gemm_skinny<16, 16> : k_gemm_skinny<32, 16>)
+                                                    : (plan->sk_km <= 16 ? k_gemm_skinny<16, 0> : k_gemm_skinny<32, 8>);
+            hipLaunchKernelGGL(kern, dim3(unsigned(plan->skinny.ntiles)), dim3(SK_THREADS), 0, ctx->stream, g, plan->skinny.d_tiles);
+            xh::launch_check("k_gemm_skinny");
+        };
         // tiles: 0 = FP64 128x128 tiles for the large items and 64x64 for the rest, 1 = 64x64 only
         auto run = [&](int tiles) {
             if(precision == XH_FP64 && tiles == 0) {
-                if(plan->skinny.ntiles > 0) {
-                    auto* kern = plan->sk_km <= 16 ? k_gemm_skinny<16> : k_gemm_skinny<32>;
-                    hipLaunchKernelGGL(kern, dim3(unsigned(plan->skinny.ntiles)), dim3(SK_THREADS), 0, ctx->stream, g, plan->skinny.d_tiles);
-                    xh::launch_check("k_gemm_skinny");
-                }
+                launch_skinny();
                 launch(plan->big128, f64_128, 2, G8_THREADS, lds128, "k_gemm_f64_128");
                 launch(plan->rest64, f64_64, 8, G_THREADS, plan->lds64, "k_gemm_f64");
             } else if(precision == XH_FP64) {
                 launch(plan->all64, f64_64, 8, G_THREADS, lds64, "k_gemm_f64");
             } else if(precision == XH_OZAKI) {
                 if(!plan->oz_built) build_oz(ctx, plan);
-                if(plan->skinny.ntiles > 0) {
-                    auto* kern = plan->sk_km <= 16 ? k_gemm_skinny<16> : k_gemm_skinny<32>;
-                    hipLaunchKernelGGL(kern, dim3(unsigned(plan->skinny.ntiles)), dim3(SK_THREADS), 0, ctx->stream, g, plan->skinny.d_tiles);
-                    xh::launch_check("k_gemm_skinny");
-                }
+                launch_skinny();
                 launch(plan->oz_rest, f64_64, 8, G_THREADS, lds64, "k_gemm_f64");
                 if(plan->oz_tiles.ntiles > 0) {
                     int8_t* sl = nullptr;
@@ -1772,6 +1830,13 @@ bool gather_eligible(const xh_gemm_plan* plan)
     for(const auto& it : plan->h_items)
         if(it.m > 0 && it.n > 0 && !(plan->is_skinny(it) && it.m > it.n)) return false;
     return true;
+}
+
+template <bool SCATTER>
+auto gather_kernel(const xh_gemm_plan* plan)
+{
+    return plan->sk_short > SK_SCALAR ? (plan->sk_km <= 16 ? k_gemm_skinny_gather<16, 16, SCATTER> : k_gemm_skinny_gather<32, 16, SCATTER>)
+                                      : (plan->sk_km <= 16 ? k_gemm_skinny_gather<16, 0, SCATTER> : k_gemm_skinny_gather<32, 0, SCATTER>);
 }
 
 // workgroups of a gather product: whole runs of GA_RUN blocks on every XCD
@@ -2037,7 +2102,7 @@ extern "C" int xh_gemm_gather(xh_ctx* ctx, const xh_gemm_plan* plan, const xh_ga
         const bool timed = ctx->gemm_timing;
         if(timed) xh::gemm_timer_begin(ctx);
         GemmArgs g{plan->d_items, plan->d_ext, nullptr, {}, plan->ta, plan->tb, nullptr, B, C, nullptr, alpha, beta};
-        auto* kern = plan->sk_km <= 16 ? k_gemm_skinny_gather<16, false> : k_gemm_skinny_gather<32, false>;
+        auto* kern = gather_kernel<false>(plan);
         const unsigned grid = gather_grid(gp->dev.nblocks);
         if(grid > 0) hipLaunchKernelGGL(kern, dim3(grid), dim3(SK_THREADS), 0, ctx->stream, g, gp->dev, src, ScatterDev{});
         xh::launch_check("k_gemm_skinny_gather");
@@ -2197,7 +2262,7 @@ extern "C" int xh_gemm_gather_scatter(xh_ctx* ctx, const xh_gemm_plan* plan, con
         const bool timed = ctx->gemm_timing;
         if(timed) xh::gemm_timer_begin(ctx);
         GemmArgs g{plan->d_items, plan->d_ext, nullptr, {}, plan->ta, plan->tb, nullptr, B, dst, nullptr, alpha, 0.0};
-        auto* kern = plan->sk_km <= 16 ? k_gemm_skinny_gather<16, true> : k_gemm_skinny_gather<32, true>;
+        auto* kern = gather_kernel<true>(plan);
         const unsigned grid = gather_grid(gp->dev.nblocks);
         if(grid > 0) hipLaunchKernelGGL(kern, dim3(grid), dim3(SK_THREADS), 0, ctx->stream, g, gp->dev, src, sp->dev);
         xh::launch_check("k_gemm_skinny_gather");
