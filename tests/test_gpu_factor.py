@@ -80,7 +80,7 @@ def _svd_blocks():
     r = np.random.default_rng(8)
     out = [r.uniform(-1, 1, s) for s in
            [(1, 1), (1, 9), (9, 1), (2, 2), (31, 32), (33, 32), (65, 31), (64, 64), (63, 64), (130, 33), (129, 64), (66, 65), (97, 97), (98, 98), (99, 99), (100, 96),
-            (300, 20), (1500, 9), (40, 400)]]
+            (300, 20), (1500, 9), (40, 400), (256, 7), (257, 7), (257, 32), (257, 33), (2000, 8), (9, 1800), (9000, 2), (19000, 1)]]
     out.append(np.zeros((7, 5)))
     out.append(np.ones((20, 20)))  # rank one, equal columns
     out.append(np.diag(np.arange(12.0)))

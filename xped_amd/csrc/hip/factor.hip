@@ -64,8 +64,9 @@ __device__ __forceinline__ double* work_base(double* smem, const FactorArgs& fa)
 // (nn), order (nn ints).
 //
 // The kernel is a serial chain of (nn - 1) steps per sweep, each the latency of one rotation: the
-// columns of a pair read from LDS, an inner product, the angle, the update, a barrier.  So 16
-// lanes own a pair (two rows each per 16-byte LDS access) and reduce by DPP; the columns of W stay
+// columns of a pair read from LDS, an inner product, the angle, the update, a barrier.  So G = 16
+// lanes own a pair (two rows each per 16-byte LDS access; 64 lanes in tall blocks, SVD_TALL) and
+// reduce by DPP; the columns of W stay
 // in registers between the inner product and the update (RM > 0: rows <= 32 RM; RM = 0: any
 // number, read twice); V is read only when the pair rotates.  Squared column norms are kept beside
 // W, moved with each rotation, summed afresh where a rotation takes most of a
@@ -89,7 +90,7 @@ constexpr double SVD_TINY = 1e-135;  // squared norm of a column taken as zero (
 
 constexpr double SVD_NEAR = 1e-14;    // squared cosine below which a sweep counts as nearly converged
 
-template <int RM, int VM>
+template <int RM, int VM, int G = 16>
 __global__ __launch_bounds__(SVD_THREADS) void k_svd_jacobi(FactorArgs fa)
 {
     extern __shared__ __attribute__((aligned(16))) double smem[];
@@ -105,7 +106,7 @@ __global__ __launch_bounds__(SVD_THREADS) void k_svd_jacobi(FactorArgs fa)
     double* V = W + int64_t(ldw) * nn;
     double* sig = V + int64_t(ldv) * nn;
     int* ord = reinterpret_cast<int*>(sig + nn);
-    constexpr int G = 16, RR = RM > 0 ? RM : 1;
+    constexpr int RR = RM > 0 ? RM : 1;
     const int tid = threadIdx.x, gl = tid % G, grp = tid / G, ngroups = blockDim.x / G;
     double mx = 0.0;
     for(int j = grp; j < nn; j += ngroups) {
@@ -970,6 +971,12 @@ void run_factor(xh_ctx* ctx, void (*kern_lds)(FactorArgs), void (*kern_global)(F
 // anyway, but 1.4 ms by itself), and only those that do not fit LDS in a call of smaller blocks
 // (15 sectors of up to 74 columns: 0.46 ms by themselves, 1.07 ms with block Jacobi and its products).
 constexpr int BJ_MIN_COLS = 64, BJ_MIN_COLS_ALONE = 98;
+// Rows from which a call's pairs of up to 32 columns are worked on by 64 lanes instead of 16, which
+// then read a column four times as fast: 2000 x 8 429 us with 16 lanes, 165 with 64 (296 with three
+// reductions through ds_bpermute and IEEE divisions), 300 x 32 456 and 423, 20000 x 1 418 and 126.  Below,
+// the longer reduction and the fewer blocks per CU cost more: 140 x 32 320 and 372, 300 blocks of
+// 200 x 30 481 and 689.
+constexpr int SVD_TALL = 257;
 
 namespace {
 // The single-workgroup Jacobi kernel on blocks whose working set fits LDS: one launch, in the
@@ -987,7 +994,11 @@ void small_svd(xh_ctx* ctx, const std::vector<xh_factor_item>& v, const double* 
         maxd = std::max(maxd, svd_work_doubles(a, b));
     }
     void (*kern)(FactorArgs) = nullptr;
-    if(nn <= 32)
+    int G = 16;  // lanes per pair of columns
+    if(nn <= 32 && mm >= SVD_TALL) {
+        kern = k_svd_jacobi<0, 1, 64>;
+        G = 64;
+    } else if(nn <= 32)
         kern = mm <= 32 ? k_svd_jacobi<1, 1> : mm <= 64 ? k_svd_jacobi<2, 1> : mm <= 128 ? k_svd_jacobi<4, 1> : k_svd_jacobi<0, 1>;
     else if(nn <= 64)
         kern = mm <= 64 ? k_svd_jacobi<2, 2> : mm <= 128 ? k_svd_jacobi<4, 2> : k_svd_jacobi<0, 2>;
@@ -995,7 +1006,7 @@ void small_svd(xh_ctx* ctx, const std::vector<xh_factor_item>& v, const double* 
         kern = mm <= 128 ? k_svd_jacobi<4, 4> : k_svd_jacobi<0, 4>;
     static_assert(BJ_MIN_COLS_ALONE <= 128, "k_svd_jacobi's V rows");
     const int npairs = (nn + 1) / 2;
-    const int threads = std::min(SVD_THREADS, (npairs * 16 + 63) / 64 * 64);
+    const int threads = std::min(SVD_THREADS, (npairs * G + 63) / 64 * 64);
     int* d_status = nullptr;
     check(xh::dmalloc(ctx, reinterpret_cast<void**>(&d_status), sizeof(int)), "hipMallocAsync");
     check(hipMemsetAsync(d_status, 0, sizeof(int), ctx->stream), "hipMemsetAsync");
