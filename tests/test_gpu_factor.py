@@ -171,3 +171,39 @@ def test_block_chol_inv_exact(rt, n):
     shift = (C.c_double * 1)(0.0)
     x, = _run(rt, lambda ctx, arr, k, dA, dX: lib().xh_block_chol_inv(ctx, arr, k, dA, dX, shift), [G], (n * n,), [_lib.xh_factor_item(0, 0, 0, 0, n, n)])
     assert np.array_equal(x.reshape(n, n).T, (np.eye(n) - N) / d[None, :])
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf, 1e170], ids=["nan", "inf", "overflow"])
+@pytest.mark.parametrize("shape,beside", [((65, 65), None), ((98, 98), None), ((70, 150), None), ((150, 70), None), ((99, 99), None), ((70, 70), (20, 20)),
+                                          ((70, 70), (120, 120))])
+def test_block_svd_refuses_non_finite_blocks(rt, shape, beside, bad):
+    """Blocks of more than 64 columns whose sum of squares is not finite: XH_EINVAL, whichever kernel
+    they are for; the context works on afterwards."""
+    r = np.random.default_rng(2)
+    blocks = [r.uniform(-1, 1, s) for s in (shape, beside) if s]
+    blocks[0][shape[0] // 2, shape[1] - 1] = bad
+    items, ao, uo, so, vo = [], 0, 0, 0, 0
+    for b in blocks:
+        (m, n), k = b.shape, min(b.shape)
+        items.append(_lib.xh_factor_item(ao, uo, so, vo, m, n))
+        ao, uo, so, vo = ao + m * n, uo + m * k, so + k, vo + k * n
+    codes = []
+
+    def call(ctx, arr, n, *bufs):
+        codes.append(lib().xh_block_svd(ctx, arr, n, *bufs))
+        return 0
+
+    _run(rt, call, blocks, (uo, so, vo), items)
+    assert codes == [_lib.XH_EINVAL] and b"non-finite" in lib().xh_last_error(rt.ctx())
+    blocks[0][shape[0] // 2, shape[1] - 1] = 0.5
+    _, S, _ = _run(rt, call, blocks, (uo, so, vo), items)
+    assert codes[1] == 0 and np.isfinite(S).all()
+
+
+def test_block_svd_passes_small_non_finite_blocks(rt):
+    """Up to 64 columns nothing is refused: the values of the columns that hold no NaN come out, the NaN last."""
+    r = np.random.default_rng(3)
+    b = np.diag(r.uniform(1, 2, 64))
+    b[5, 5] = np.nan
+    _, S, _ = _run(rt, lib().xh_block_svd, [b], (64 * 64, 64, 64 * 64), [_lib.xh_factor_item(0, 0, 0, 0, 64, 64)])
+    assert np.isnan(S[63]) and np.array_equal(S[:63], np.sort(np.delete(np.diag(b), 5))[::-1])

@@ -1,8 +1,10 @@
 // Batched per-sector factorisations in FP64: SVD (one-sided Jacobi), QR (Householder, with the
-// reflector convention of Eigen::HouseholderQR) and symmetric eigen (parallel cyclic Jacobi).
+// reflector convention of Eigen::HouseholderQR), inverse Cholesky factors and symmetric eigen
+// (parallel cyclic Jacobi).
 //
 // One workgroup owns one sector block.  Blocks that fit the LDS budget are factorised entirely in
-// LDS; larger blocks use a global-memory working copy with the same algorithm.
+// LDS; larger ones use a global-memory working copy with the same algorithm, except for the SVD,
+// whose larger blocks go to block Jacobi (bjsvd.hip).
 //
 // The reference calls Eigen per sector (PlainInterface::svd, PlainInterface_Eigen_impl.cpp:116-127;
 // MatrixInterface::qr, MatrixInterface_Eigen_impl.cpp:249-255; MatrixInterface::eigh,
@@ -66,17 +68,23 @@ __device__ __forceinline__ double* work_base(double* smem, const FactorArgs& fa)
 // The kernel is a serial chain of (nn - 1) steps per sweep, each the latency of one rotation: the
 // columns of a pair read from LDS, an inner product, the angle, the update, a barrier.  So G = 16
 // lanes own a pair (two rows each per 16-byte LDS access; 64 lanes in tall blocks, SVD_TALL) and
-// reduce by DPP; the columns of W stay
-// in registers between the inner product and the update (RM > 0: rows <= 32 RM; RM = 0: any
-// number, read twice); V is read only when the pair rotates.  Squared column norms are kept beside
-// W, moved with each rotation, summed afresh where a rotation takes most of a
-// column away and for every column before each sweep, so the last sweep, which finds every pair
-// orthogonal, judges by fresh norms.  The block is scaled by a power of two to a largest entry of
-// [1/2, 1), so that squares and their products stay in range.
+// reduce by DPP; the columns of W stay in registers between the inner product and the update (RM > 0:
+// rows <= 32 RM; RM = 0: any number, read twice); V is read only when the pair rotates.  Squared
+// column norms are kept beside W, moved with each rotation, summed afresh where a rotation takes
+// most of a column away and for every column before each sweep, so the last sweep, which finds
+// every pair orthogonal, judges by fresh norms.  The block is scaled by a power of two to a largest
+// entry of [1/2, 1), so that squares and their products stay in range.  A block of more than
+// BJ_MIN_COLS columns with a non-finite sum of squares is refused, as block Jacobi refuses it.
 // (64 to 8 lanes per pair, three reductions through ds_bpermute, IEEE divisions and square roots
 // took 542 us for the 9 blocks, 32 x 32 the largest, of a two-site tensor at bond 64; three DPP
 // reductions and refined quotients 220 us; this takes 184 us.)
 constexpr int SVD_THREADS = 1024;
+
+// Blocks with more columns than this (after transposition) use the block Jacobi path: any block of
+// a call where some block has to (a block of 65 to 98 columns then adds nothing to steps that run
+// anyway, but 1.4 ms by itself), and only those that do not fit LDS in a call of smaller blocks
+// (15 sectors of up to 74 columns: 0.46 ms by themselves, 1.07 ms with block Jacobi and its products).
+constexpr int BJ_MIN_COLS = 64, BJ_MIN_COLS_ALONE = 98;
 
 __host__ __device__ inline int svd_ld(int rows) { return (rows + 1) & ~1; }
 __host__ __device__ inline int64_t svd_work_doubles(int64_t mm, int64_t nn)
@@ -95,7 +103,7 @@ __global__ __launch_bounds__(SVD_THREADS) void k_svd_jacobi(FactorArgs fa)
 {
     extern __shared__ __attribute__((aligned(16))) double smem[];
     __shared__ int rotated, far;  // a pair was rotated this sweep; one by more than SVD_NEAR
-    __shared__ double s_max[SVD_THREADS / 64];
+    __shared__ double s_max[SVD_THREADS / 64], s_sq[SVD_THREADS / 64];
     const xh_factor_item it = fa.items[blockIdx.x];
     const int m = it.m, n = it.n;
     if(m == 0 || n == 0) return;
@@ -107,21 +115,37 @@ __global__ __launch_bounds__(SVD_THREADS) void k_svd_jacobi(FactorArgs fa)
     double* sig = V + int64_t(ldv) * nn;
     int* ord = reinterpret_cast<int*>(sig + nn);
     constexpr int RR = RM > 0 ? RM : 1;
+    constexpr bool WIDE = 32 * VM > BJ_MIN_COLS;  // may hold blocks that are refused where not finite
     const int tid = threadIdx.x, gl = tid % G, grp = tid / G, ngroups = blockDim.x / G;
-    double mx = 0.0;
+    double mx = 0.0, sq = 0.0;
     for(int j = grp; j < nn; j += ngroups) {
         for(int i = gl; i < ldw; i += G) {
             const double v = i >= mm ? 0.0 : tr ? fa.A[it.a_off + j + int64_t(i) * m] : fa.A[it.a_off + i + int64_t(j) * m];
             W[j * ldw + i] = v;
             mx = fmax(mx, fabs(v));
+            sq = fma(v, v, sq);
         }
         for(int i = gl; i < ldv; i += G) V[j * ldv + i] = i == j ? 1.0 : 0.0;
     }
-    for(int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o));
-    if((tid & 63) == 0) s_max[tid >> 6] = mx;
+    for(int o = 32; o > 0; o >>= 1) {
+        mx = fmax(mx, __shfl_xor(mx, o));
+        if constexpr(WIDE) sq += __shfl_xor(sq, o);
+    }
+    if((tid & 63) == 0) {
+        s_max[tid >> 6] = mx;
+        if constexpr(WIDE) s_sq[tid >> 6] = sq;
+    }
     __syncthreads();
+    sq = 0.0;
+    for(int w = 0; w < int(blockDim.x >> 6); ++w) {
+        mx = fmax(mx, s_max[w]);
+        if constexpr(WIDE) sq += s_sq[w];
+    }
+    if(WIDE && nn > BJ_MIN_COLS && !isfinite(sq)) {  // the same in every thread
+        if(tid == 0) atomicOr(fa.status, XH_EINVAL);
+        return;
+    }
     int ex = 0;
-    for(int w = 0; w < int(blockDim.x >> 6); ++w) mx = fmax(mx, s_max[w]);
     if(mx > 0.0 && mx <= DBL_MAX) frexp(mx, &ex);
 
     const int n2 = nn + (nn & 1);
@@ -267,7 +291,7 @@ __global__ __launch_bounds__(SVD_THREADS) void k_svd_jacobi(FactorArgs fa)
             }
         }
     }
-    if(sweep >= MAX_SWEEPS && tid == 0) atomicExch(fa.status, XH_ENOTCONV);
+    if(sweep >= MAX_SWEEPS && tid == 0) atomicOr(fa.status, XH_ENOTCONV);
     // column norms
     for(int j = grp; j < nn; j += ngroups) {
         const double* wj = W + j * ldw;
@@ -966,11 +990,6 @@ void run_factor(xh_ctx* ctx, void (*kern_lds)(FactorArgs), void (*kern_global)(F
 
 }  // namespace
 
-// Blocks with more columns than this (after transposition) use the block Jacobi path: any block of
-// a call where some block has to (a block of 65 to 98 columns then adds nothing to steps that run
-// anyway, but 1.4 ms by itself), and only those that do not fit LDS in a call of smaller blocks
-// (15 sectors of up to 74 columns: 0.46 ms by themselves, 1.07 ms with block Jacobi and its products).
-constexpr int BJ_MIN_COLS = 64, BJ_MIN_COLS_ALONE = 98;
 // Rows from which a call's pairs of up to 32 columns are worked on by 64 lanes instead of 16, which
 // then read a column four times as fast: 2000 x 8 429 us with 16 lanes, 165 with 64 (296 with three
 // reductions through ds_bpermute and IEEE divisions), 300 x 32 456 and 423, 20000 x 1 418 and 126.  Below,
@@ -1022,6 +1041,8 @@ void small_svd(xh_ctx* ctx, const std::vector<xh_factor_item>& v, const double* 
     check(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
     xh::dev_free(ctx, d_items);
     xh::dev_free(ctx, d_status);
+    static_assert((XH_EINVAL & XH_ENOTCONV) == 0, "status bits");
+    if(status & XH_EINVAL) throw xh::Error(XH_EINVAL, "block SVD: non-finite input block");
     if(status != 0) throw xh::Error(XH_ENOTCONV, "Jacobi iteration did not converge within the sweep limit");
 }
 }  // namespace
