@@ -228,7 +228,13 @@ int xh_trace_marker(xh_ctx* ctx, int id);
  * (Tensor.cpp:757-780) over MatrixInterface::qr, and Tensor::teigh (Tensor.cpp:782-803) over
  * MatrixInterface::eigh.  Block g is m x n column-major at a_off; outputs are thin:
  * U (m x r) at u_off, S (r) at s_off, Vt (r x n) at vt_off with r = min(m, n); singular values
- * descending.  eigh: square blocks, eigenvalues ascending, eigenvectors in columns. */
+ * descending.  eigh: square blocks, eigenvalues ascending, eigenvectors in columns.
+ * SVD: a block whose short side exceeds 64 and whose sum of squares is not finite fails with
+ * XH_EINVAL; a smaller one passes, its NaN values last.  Columns (rows of a wide block) are made
+ * orthogonal whatever their size down to 2e-214 of the block's largest entry where the block is
+ * factorised by one workgroup (short side up to 64, and up to 98 in a call without larger blocks),
+ * and down to max(m, n) eps of the block's norm otherwise; the vectors of smaller ones are only
+ * normalised. */
 typedef struct {
     int64_t a_off, u_off, s_off, vt_off;
     int32_t m, n;

@@ -207,3 +207,36 @@ def test_block_svd_passes_small_non_finite_blocks(rt):
     b[5, 5] = np.nan
     _, S, _ = _run(rt, lib().xh_block_svd, [b], (64 * 64, 64, 64 * 64), [_lib.xh_factor_item(0, 0, 0, 0, 64, 64)])
     assert np.isnan(S[63]) and np.array_equal(S[:63], np.sort(np.delete(np.diag(b), 5))[::-1])
+
+
+@pytest.mark.parametrize("scale", [1.0, 1e-150, 1e60])
+@pytest.mark.parametrize("shape", [(8, 6), (30, 30), (64, 64), (98, 98), (100, 9), (300, 12), (20, 300)])
+def test_block_svd_of_graded_blocks(rt, shape, scale):
+    """Columns (rows of a wide block) 1e-75 and 1e-140 of the others: both factors orthonormal, and the
+    values of each group those of its part orthogonal to the larger groups, to the relative accuracy of
+    one-sided Jacobi (Demmel and Veselic, SIAM J. Matrix Anal. Appl. 13 (1992) 1204: eps times the
+    condition of the columns scaled to norm 1, here below 1e4)."""
+    r = np.random.default_rng(shape[0])
+    m, n = max(shape), min(shape)
+    base = r.uniform(-1, 1, (m, n)) + (2.0 * np.eye(m, n) if m == n else 0.0)
+    cut = [0, n // 3, 2 * n // 3, n]
+    grades = [1.0, 1e-75, 1e-140]
+    if scale < 1.0:
+        grades = [1.0, 1e-60, 1e-120]
+    perm = r.permutation(n)
+    b = base * np.repeat(grades, np.diff(cut))[None, :] * scale
+    b = b[:, perm]
+    b = b if shape[0] >= shape[1] else b.T
+    k = n
+    U, S, V = _run(rt, lib().xh_block_svd, [b], (shape[0] * k, k, k * shape[1]), [_lib.xh_factor_item(0, 0, 0, 0, *shape)])
+    u, v = U.reshape(k, shape[0]).T, V.reshape(shape[1], k).T
+    tol = 1e-12 * np.sqrt(k)
+    assert np.abs(u.T @ u - np.eye(k)).max() <= tol and np.abs(v @ v.T - np.eye(k)).max() <= tol
+    assert np.linalg.norm((u * S) @ v - b) <= tol * S[0]
+    for g in range(3):
+        part = base[:, cut[g]:cut[g + 1]]
+        if g:
+            q = np.linalg.qr(base[:, :cut[g]])[0]
+            part = part - q @ (q.T @ part)
+        ref = np.linalg.svd(part, compute_uv=False) * grades[g] * scale
+        assert np.abs(S[cut[g]:cut[g + 1]] / ref - 1).max() <= 1e-10, (g, shape)

@@ -14,6 +14,7 @@
 #include <cfloat>
 #include <cstring>
 #include <iterator>
+#include <type_traits>
 
 #include "device.hpp"
 
@@ -72,9 +73,14 @@ __device__ __forceinline__ double* work_base(double* smem, const FactorArgs& fa)
 // rows <= 32 RM; RM = 0: any number, read twice); V is read only when the pair rotates.  Squared
 // column norms are kept beside W, moved with each rotation, summed afresh where a rotation takes
 // most of a column away and for every column before each sweep, so the last sweep, which finds
-// every pair orthogonal, judges by fresh norms.  The block is scaled by a power of two to a largest
-// entry of [1/2, 1), so that squares and their products stay in range.  A block of more than
-// BJ_MIN_COLS columns with a non-finite sum of squares is refused, as block Jacobi refuses it.
+// every pair orthogonal, judges by fresh norms.  A block of more than BJ_MIN_COLS columns with a
+// non-finite sum of squares is refused, as block Jacobi refuses it.
+//
+// Range: the block is scaled by a power of two to a largest finite entry of [2^229, 2^230).  Squared
+// norms are then at most 2^475, and the products of two of them in range unless both columns are
+// tiny; such a pair is scaled once more for its test and its angle, in a copy of the steps for blocks
+// that have tiny columns (asked for each pair, it took 3 to 6 % more).  Only columns below
+// sqrt(SVD_ZERO), 2e-214 of the largest entry, are left alone.
 // (64 to 8 lanes per pair, three reductions through ds_bpermute, IEEE divisions and square roots
 // took 542 us for the 9 blocks, 32 x 32 the largest, of a two-site tensor at bond 64; three DPP
 // reductions and refined quotients 220 us; this takes 184 us.)
@@ -94,15 +100,29 @@ __host__ __device__ inline int64_t svd_work_doubles(int64_t mm, int64_t nn)
 
 typedef double d2 __attribute__((ext_vector_type(2)));
 
-constexpr double SVD_TINY = 1e-135;  // squared norm of a column taken as zero (largest entry scaled to 1)
+constexpr int SVD_EXP = 230;            // the largest entry is scaled to below 2^SVD_EXP
+constexpr double SVD_ZERO = 0x1p-960;   // squared norm of a column taken as zero
+constexpr double SVD_SMALL = 0x1p-450;  // tiny: two such squared norms have their product scaled
+constexpr double SVD_NEAR = 1e-14;      // squared cosine below which a sweep counts as nearly converged
 
-constexpr double SVD_NEAR = 1e-14;    // squared cosine below which a sweep counts as nearly converged
+// al, be and ga of a pair with al be < SVD_SMALL^2 times a power of two: the larger norm to about 2^400,
+// the smaller one, at least SVD_ZERO, then above 2^-621
+__device__ __forceinline__ void scale_pair(double& al, double& be, double& ga)
+{
+    if(al * be >= SVD_SMALL * SVD_SMALL) return;
+    int e;
+    frexp(fmax(al, be), &e);
+    al = ldexp(al, 400 - e);
+    be = ldexp(be, 400 - e);
+    ga = ldexp(ga, 400 - e);
+}
 
 template <int RM, int VM, int G = 16>
 __global__ __launch_bounds__(SVD_THREADS) void k_svd_jacobi(FactorArgs fa)
 {
     extern __shared__ __attribute__((aligned(16))) double smem[];
     __shared__ int rotated, far;  // a pair was rotated this sweep; one by more than SVD_NEAR
+    __shared__ int s_tiny;        // a column was tiny at the start of a sweep
     __shared__ double s_max[SVD_THREADS / 64], s_sq[SVD_THREADS / 64];
     const xh_factor_item it = fa.items[blockIdx.x];
     const int m = it.m, n = it.n;
@@ -122,7 +142,7 @@ __global__ __launch_bounds__(SVD_THREADS) void k_svd_jacobi(FactorArgs fa)
         for(int i = gl; i < ldw; i += G) {
             const double v = i >= mm ? 0.0 : tr ? fa.A[it.a_off + j + int64_t(i) * m] : fa.A[it.a_off + i + int64_t(j) * m];
             W[j * ldw + i] = v;
-            mx = fmax(mx, fabs(v));
+            mx = fmax(mx, isfinite(v) ? fabs(v) : 0.0);
             sq = fma(v, v, sq);
         }
         for(int i = gl; i < ldv; i += G) V[j * ldv + i] = i == j ? 1.0 : 0.0;
@@ -146,7 +166,8 @@ __global__ __launch_bounds__(SVD_THREADS) void k_svd_jacobi(FactorArgs fa)
         return;
     }
     int ex = 0;
-    if(mx > 0.0 && mx <= DBL_MAX) frexp(mx, &ex);
+    if(mx > 0.0) frexp(mx, &ex);
+    ex -= SVD_EXP;
 
     const int n2 = nn + (nn & 1);
     const int npairs = n2 / 2;
@@ -167,100 +188,115 @@ __global__ __launch_bounds__(SVD_THREADS) void k_svd_jacobi(FactorArgs fa)
     // the pair of positions (grp, n2 - 1 - grp) of the circle: position 0 keeps its column, the
     // others move on by one each step and are back after the n2 - 1 steps of a sweep
     int a = grp, b = n2 - 1 - grp;
+    // the n2 - 1 steps of a sweep
+    auto steps = [&](auto has_tiny) {
+        constexpr bool tiny = decltype(has_tiny)::value;
+        for(int step = 0; step < n2 - 1; ++step) {
+            if(grp < npairs && max(a, b) < nn) {  // a dummy column fills an odd count
+                d2* wi = reinterpret_cast<d2*>(W + __mul24(a, ldw)) + gl;
+                d2* wj = reinterpret_cast<d2*>(W + __mul24(b, ldw)) + gl;
+                const double al = sig[a], be = sig[b];
+                d2 x[RR], y[RR];
+                double ga = 0;
+                if constexpr(RM > 0) {
+#pragma unroll
+                    for(int k = 0; k < RM; ++k) {
+                        x[k] = d2{0.0, 0.0};
+                        y[k] = d2{0.0, 0.0};
+                        if(k * G < nw) {
+                            x[k] = wi[k * G];
+                            y[k] = wj[k * G];
+                        }
+                    }
+#pragma unroll
+                    for(int k = 0; k < RM; ++k) {
+                        ga = fma(x[k][0], y[k][0], ga);
+                        ga = fma(x[k][1], y[k][1], ga);
+                    }
+                } else {
+                    for(int k = 0; k < nw; k += G) {
+                        const d2 p = wi[k], q = wj[k];
+                        ga = fma(p[0], q[0], ga);
+                        ga = fma(p[1], q[1], ga);
+                    }
+                }
+                ga = xh::lanes_sum<G>(ga);
+                double sa = al, sb = be, sg = ga;  // scaled where the products would underflow
+                if constexpr(tiny) scale_pair(sa, sb, sg);
+                if(fmin(al, be) > SVD_ZERO && sg * sg > tol2 * (sa * sb)) {
+                    d2* vi = reinterpret_cast<d2*>(V + __mul24(a, ldv)) + gl;
+                    d2* vj = reinterpret_cast<d2*>(V + __mul24(b, ldv)) + gl;
+                    d2 u[VM], v[VM];
+#pragma unroll
+                    for(int k = 0; k < VM; ++k)
+                        if(k * G < nv) {
+                            u[k] = vi[k * G];
+                            v[k] = vj[k * G];
+                        }
+                    double c, s;
+                    xh::jacobi_rotation(0.5 * (sb - sa), sg, c, s);
+                    if constexpr(RM > 0) {
+#pragma unroll
+                        for(int k = 0; k < RM; ++k) {
+                            const d2 p = x[k];
+                            x[k] = c * p - s * y[k];
+                            y[k] = s * p + c * y[k];
+                            if(k * G < nw) {
+                                wi[k * G] = x[k];
+                                wj[k * G] = y[k];
+                            }
+                        }
+                    } else {
+                        for(int k = 0; k < nw; k += G) {
+                            const d2 p = wi[k], q = wj[k];
+                            wi[k] = c * p - s * q;
+                            wj[k] = s * p + c * q;
+                        }
+                    }
+#pragma unroll
+                    for(int k = 0; k < VM; ++k)
+                        if(k * G < nv) {
+                            vi[k * G] = c * u[k] - s * v[k];
+                            vj[k * G] = s * u[k] + c * v[k];
+                        }
+                    const double g2 = 2.0 * s * c * ga;
+                    double na = fma(c * c, al, fma(s * s, be, -g2)), nb = fma(s * s, al, fma(c * c, be, g2));
+                    if(fmin(na, nb) < 1e-3 * fmin(al, be)) {  // cancellation (rare): sum afresh
+                        na = norm2(a);
+                        nb = norm2(b);
+                    }
+                    if(gl == 0) {
+                        sig[a] = na;
+                        sig[b] = nb;
+                        rotated = 1;
+                        if(sg * sg > SVD_NEAR * (sa * sb)) far = 1;
+                    }
+                }
+            }
+            if(grp != 0) a = a == n2 - 1 ? 1 : a + 1;
+            b = b == n2 - 1 ? 1 : b + 1;
+            __syncthreads();
+        }
+    };
     int sweep = 0;
+    if(tid == 0) s_tiny = 0;
     if(nn > 1) {
         for(sweep = 0; sweep < MAX_SWEEPS; ++sweep) {
             __syncthreads();
             for(int j = grp; j < nn; j += ngroups) {
                 const double s = norm2(j);
-                if(gl == 0) sig[j] = s;
+                if(gl == 0) {
+                    sig[j] = s;
+                    if(s > 0.0 && s < SVD_SMALL) s_tiny = 1;
+                }
             }
             if(tid == 0) rotated = far = 0;
             __syncthreads();
-            for(int step = 0; step < n2 - 1; ++step) {
-                if(grp < npairs && max(a, b) < nn) {  // a dummy column fills an odd count
-                    d2* wi = reinterpret_cast<d2*>(W + __mul24(a, ldw)) + gl;
-                    d2* wj = reinterpret_cast<d2*>(W + __mul24(b, ldw)) + gl;
-                    const double al = sig[a], be = sig[b];
-                    d2 x[RR], y[RR];
-                    double ga = 0;
-                    if constexpr(RM > 0) {
-#pragma unroll
-                        for(int k = 0; k < RM; ++k) {
-                            x[k] = d2{0.0, 0.0};
-                            y[k] = d2{0.0, 0.0};
-                            if(k * G < nw) {
-                                x[k] = wi[k * G];
-                                y[k] = wj[k * G];
-                            }
-                        }
-#pragma unroll
-                        for(int k = 0; k < RM; ++k) {
-                            ga = fma(x[k][0], y[k][0], ga);
-                            ga = fma(x[k][1], y[k][1], ga);
-                        }
-                    } else {
-                        for(int k = 0; k < nw; k += G) {
-                            const d2 p = wi[k], q = wj[k];
-                            ga = fma(p[0], q[0], ga);
-                            ga = fma(p[1], q[1], ga);
-                        }
-                    }
-                    ga = xh::lanes_sum<G>(ga);
-                    if(fmin(al, be) > SVD_TINY && ga * ga > tol2 * (al * be)) {
-                        d2* vi = reinterpret_cast<d2*>(V + __mul24(a, ldv)) + gl;
-                        d2* vj = reinterpret_cast<d2*>(V + __mul24(b, ldv)) + gl;
-                        d2 u[VM], v[VM];
-#pragma unroll
-                        for(int k = 0; k < VM; ++k)
-                            if(k * G < nv) {
-                                u[k] = vi[k * G];
-                                v[k] = vj[k * G];
-                            }
-                        double c, s;
-                        xh::jacobi_rotation(0.5 * (be - al), ga, c, s);
-                        if constexpr(RM > 0) {
-#pragma unroll
-                            for(int k = 0; k < RM; ++k) {
-                                const d2 p = x[k];
-                                x[k] = c * p - s * y[k];
-                                y[k] = s * p + c * y[k];
-                                if(k * G < nw) {
-                                    wi[k * G] = x[k];
-                                    wj[k * G] = y[k];
-                                }
-                            }
-                        } else {
-                            for(int k = 0; k < nw; k += G) {
-                                const d2 p = wi[k], q = wj[k];
-                                wi[k] = c * p - s * q;
-                                wj[k] = s * p + c * q;
-                            }
-                        }
-#pragma unroll
-                        for(int k = 0; k < VM; ++k)
-                            if(k * G < nv) {
-                                vi[k * G] = c * u[k] - s * v[k];
-                                vj[k * G] = s * u[k] + c * v[k];
-                            }
-                        const double g2 = 2.0 * s * c * ga;
-                        double na = fma(c * c, al, fma(s * s, be, -g2)), nb = fma(s * s, al, fma(c * c, be, g2));
-                        if(fmin(na, nb) < 1e-3 * fmin(al, be)) {  // cancellation (rare): sum afresh
-                            na = norm2(a);
-                            nb = norm2(b);
-                        }
-                        if(gl == 0) {
-                            sig[a] = na;
-                            sig[b] = nb;
-                            rotated = 1;
-                            if(ga * ga > SVD_NEAR * (al * be)) far = 1;
-                        }
-                    }
-                }
-                if(grp != 0) a = a == n2 - 1 ? 1 : a + 1;
-                b = b == n2 - 1 ? 1 : b + 1;
-                __syncthreads();
-            }
+            const bool tiny = __builtin_amdgcn_readfirstlane(s_tiny) != 0;
+            if(tiny)
+                steps(std::true_type{});
+            else
+                steps(std::false_type{});
             if(!rotated) break;
             // Every angle of this sweep was small, so the next one will most likely find all pairs
             // orthogonal: test them all at once, without the steps' barriers (same test).
@@ -284,7 +320,10 @@ __global__ __launch_bounds__(SVD_THREADS) void k_svd_jacobi(FactorArgs fa)
                             ga = fma(p[1], q[1], ga);
                         }
                         ga = xh::lanes_sum<G>(ga);
-                        if(gl == 0 && fmin(sig[i], sig[j]) > SVD_TINY && ga * ga > tol2 * (sig[i] * sig[j])) rotated = 1;
+                        double al = sig[i], be = sig[j];
+                        const bool live = fmin(al, be) > SVD_ZERO;
+                        if(tiny) scale_pair(al, be, ga);
+                        if(gl == 0 && live && ga * ga > tol2 * (al * be)) rotated = 1;
                     }
                 __syncthreads();
                 if(!rotated) break;
