@@ -240,3 +240,20 @@ def test_block_svd_of_graded_blocks(rt, shape, scale):
             part = part - q @ (q.T @ part)
         ref = np.linalg.svd(part, compute_uv=False) * grades[g] * scale
         assert np.abs(S[cut[g]:cut[g + 1]] / ref - 1).max() <= 1e-10, (g, shape)
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf, 1e308], ids=["nan", "inf", "overflow"])
+@pytest.mark.parametrize("n", [5, 16, 17, 100, 250])
+def test_block_chol_inv_rejects_every_pivot_of_a_non_finite_trace(rt, n, bad):
+    """The shift is a multiple of the trace (0 of it included), so with a trace that is not finite no
+    pivot exceeds its bound: X is zero."""
+    r = np.random.default_rng(n)
+    y = r.standard_normal((n + 4, n))
+    G = y.T @ y
+    G[n // 2, n // 2] = bad
+    if np.isfinite(bad):
+        G[0, 0] = bad
+    for rel in (0.0, 1e-3):
+        shift = (C.c_double * 1)(rel)
+        x, = _run(rt, lambda ctx, arr, k, dA, dX: lib().xh_block_chol_inv(ctx, arr, k, dA, dX, shift), [G], (n * n,), [_lib.xh_factor_item(0, 0, 0, 0, n, n)])
+        assert not x.any()

@@ -723,7 +723,7 @@ __global__ __launch_bounds__(CI_THREADS) void k_chol_inv(FactorArgs fa)
             const double e = fma(-d * y, y, 1.0);
             const double s = ok ? fma(y * e, fma(e, 0.375, 0.5), y) : 0.0;
             x[k] *= s;
-            if(lane == k) diag = x[k];
+            if(lane == k) diag = ok ? x[k] : 0.0;  // a rejected pivot may be infinite or NaN
 #pragma unroll
             for(int i = k + 1; i < 16; ++i) x[i] = fma(-lane_value(x[k], i), x[k], x[i]);
         }
