@@ -257,3 +257,36 @@ def test_block_chol_inv_rejects_every_pivot_of_a_non_finite_trace(rt, n, bad):
         shift = (C.c_double * 1)(rel)
         x, = _run(rt, lambda ctx, arr, k, dA, dX: lib().xh_block_chol_inv(ctx, arr, k, dA, dX, shift), [G], (n * n,), [_lib.xh_factor_item(0, 0, 0, 0, n, n)])
         assert not x.any()
+
+
+def _qr(rt, b):
+    (m, n), k = b.shape, min(b.shape)
+    Q, R = _run(rt, lib().xh_block_qr, [b], (m * k, k * n), [_lib.xh_factor_item(0, 0, k, 0, m, n)])
+    return Q.reshape(k, m).T, R.reshape(n, k).T
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf], ids=["nan", "inf"])
+@pytest.mark.parametrize("shape", [(1, 5), (6, 6), (40, 30), (64, 64), (130, 60), (60, 130), (190, 100), (250, 40), (300, 10), (100, 600), (30, 900), (1000, 15), (1030, 7)])
+def test_block_qr_keeps_non_finite_values_where_they_belong(rt, shape, bad):
+    m, n = shape
+    k = min(shape)
+    r = np.random.default_rng(m + n)
+    # triangular already: every reflector is the identity, so Q = I and R is the block, bit for bit
+    for i, j in ((0, n - 1), (k // 2, k // 2)):
+        t = np.triu(r.uniform(1, 2, shape))
+        t[i, j] = bad
+        Q, R = _qr(rt, t)
+        assert np.array_equal(Q, np.eye(m, k)) and np.array_equal(R, t[:k], equal_nan=True)
+    # columns before the one that holds the value are those of the QR without it
+    for j in {n - 1, 2 * n // 3}:
+        b = r.uniform(-1, 1, shape)
+        b[m // 2, j] = bad
+        Q, R = _qr(rt, b)
+        lead = min(j, k)
+        if lead == 0:
+            continue
+        tol = EPS * m * max(n, 4)
+        assert np.isfinite(R[:, :j]).all() and np.array_equal(np.tril(R[:, :j], -1), np.zeros((k, j)))
+        assert np.isfinite(Q[:, :lead]).all() and np.linalg.norm(Q[:, :lead].T @ Q[:, :lead] - np.eye(lead)) <= tol * np.sqrt(lead)
+        assert np.linalg.norm(Q[:, :lead] @ R[:lead, :j] - b[:, :j]) <= tol * np.linalg.norm(b[:, :j])
+        assert not np.isfinite(R[:, j]).all()

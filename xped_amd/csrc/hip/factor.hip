@@ -393,7 +393,13 @@ __global__ __launch_bounds__(SVD_THREADS) void k_svd_jacobi(FactorArgs fa)
 // columns with zeros above and a one on the diagonal, padded with zeros to G * RM rows, so that a
 // step reads RM values per lane without conditions for all NC columns.  More than NC columns per
 // group run in panels; a panel first takes all reflectors of the panels before it.
-// k_qr_tall (any number of rows): the working copy is in LDS or global memory.
+// k_qr_tall (any number of rows): the working copy is in LDS or global memory (qr_in_memory).
+//
+// k_qr takes all rows of a column through a reflector, the zeros of v included, and through identities
+// (tau = 0).  An infinity or a NaN would be spread by that to rows that the reflector does not reach,
+// so a block with one is left to qr_in_memory, which touches a reflector's own rows only.  (Both in
+// one set of steps, or a second copy of them, made finite blocks 7 to 8 % slower by their registers;
+// the look at every value costs 2 %.)
 //
 // One thread per trailing column, serial over its rows, took 2864 us for the 9 blocks (132 x 85
 // the largest) of a U(1) matrix product tensor at bond 300; columns kept in LDS by such groups
@@ -418,6 +424,68 @@ __device__ __forceinline__ void make_householder(double c0, double tail, double&
     }
 }
 
+// Q and R of a block with its columns in memory: Wk, m x n of leading dimension ld, is the working copy,
+// tau min(m, n) doubles.  Wk may be R itself (then ld is R's rows).
+__device__ __forceinline__ void qr_in_memory(const FactorArgs& fa, const xh_factor_item& it, double* Wk, int64_t ld, double* tau)
+{
+    const int m = it.m, n = it.n;
+    const int qc = static_cast<int>(it.s_off);
+    constexpr int G = 64, NG = QR_THREADS / G;
+    const int kmax = min(m, n);
+    const int tid = threadIdx.x, lane = tid % G, grp = tid / G;
+    for(int j = grp; j < n; j += NG)
+        for(int r = lane; r < m; r += G) Wk[j * ld + r] = fa.A[it.a_off + int64_t(j) * m + r];
+    auto reflector = [&](int k) {  // from column k, whose rows this group's lanes wrote themselves
+        double* col = Wk + k * ld;
+        double tail = 0.0, c0 = 0.0;
+        for(int r = lane; r < m; r += G) {
+            const double y = col[r];
+            if(r > k) tail = fma(y, y, tail);
+            if(r == k) c0 = y;
+        }
+        tail = xh::lanes_sum<G>(tail);
+        c0 = xh::lanes_sum<G>(c0);
+        double beta, t, inv;
+        make_householder(c0, tail, beta, t, inv);
+        for(int r = lane; r < m; r += G)
+            if(r >= k) col[r] = r == k ? beta : col[r] * inv;
+        if(lane == 0) tau[k] = t;
+    };
+    auto apply = [&](int k, double t, double* c) {  // c -= tau (v^T c) v, v = [1; column k below k]
+        const double* col = Wk + k * ld;
+        double w = 0.0;
+        for(int r = lane; r < m; r += G)
+            if(r >= k) w = fma(r == k ? 1.0 : col[r], c[r], w);
+        w = xh::lanes_sum<G>(w) * t;
+        for(int r = lane; r < m; r += G)
+            if(r >= k) c[r] = fma(-w, r == k ? 1.0 : col[r], c[r]);
+    };
+    if(grp == 0) reflector(0);
+    for(int k = 0; k < kmax; ++k) {
+        __syncthreads();  // reflector k is there
+        const double t = tau[k];
+        const int first = k + 1;
+        for(int j = first + ((grp - first) % NG + NG) % NG; j < n; j += NG) {
+            if(t != 0.0) apply(k, t, Wk + j * ld);
+            if(j == first && first < kmax) reflector(first);
+        }
+    }
+    __syncthreads();
+    for(int c = grp; c < qc; c += NG) {
+        double* qcol = fa.U + it.u_off + int64_t(c) * m;
+        for(int r = lane; r < m; r += G) qcol[r] = (r == c) ? 1.0 : 0.0;
+        if(c < m)
+            for(int k = min(c, kmax - 1); k >= 0; --k)
+                if(tau[k] != 0.0) apply(k, tau[k], qcol);
+    }
+    __syncthreads();
+    // R: qc x n, upper triangle of the working copy (rows beyond min(m, n) are zero)
+    for(int64_t e = tid; e < int64_t(qc) * n; e += QR_THREADS) {
+        const int r = static_cast<int>(e % qc), c = static_cast<int>(e / qc);
+        fa.Vt[it.vt_off + e] = (r < m && r <= c) ? Wk[r + c * ld] : 0.0;
+    }
+}
+
 template <bool LDS, int G, int RM, int NC>
 __global__ __launch_bounds__(QR_THREADS) void k_qr(FactorArgs fa)
 {
@@ -432,6 +500,31 @@ __global__ __launch_bounds__(QR_THREADS) void k_qr(FactorArgs fa)
     double* tau = V + int64_t(LD) * kmax;  // kmax
     const int lane = threadIdx.x % G, grp = threadIdx.x / G;
     double x[NC][RM], v[RM];
+    auto load_panel = [&](int p0) {
+#pragma unroll
+        for(int q = 0; q < NC; ++q) {
+            const int j = p0 + grp + q * NG;
+#pragma unroll
+            for(int i = 0; i < RM; ++i) {
+                const int r = lane + i * G;
+                x[q][i] = j < n && r < m ? fa.A[it.a_off + int64_t(j) * m + r] : 0.0;
+            }
+        }
+    };
+    load_panel(0);
+    bool ok = true;
+#pragma unroll
+    for(int q = 0; q < NC; ++q)
+#pragma unroll
+        for(int i = 0; i < RM; ++i) ok = ok && isfinite(x[q][i]);
+    for(int64_t e = int64_t(PC) * m + threadIdx.x; e < int64_t(m) * n; e += QR_THREADS) ok = ok && isfinite(fa.A[it.a_off + e]);
+    if(!__syncthreads_and(ok)) {
+        if(n <= m)
+            qr_in_memory(fa, it, V, m, V + m * n);  // (m + 1) n doubles, as k_qr's work area has
+        else
+            qr_in_memory(fa, it, fa.Vt + it.vt_off, qc, tau);
+        return;
+    }
     auto load_v = [&](int k) {
         const double* col = V + int64_t(k) * LD + lane;
 #pragma unroll
@@ -477,15 +570,7 @@ __global__ __launch_bounds__(QR_THREADS) void k_qr(FactorArgs fa)
         if(lane == 0) tau[k] = t;
     };
     for(int p0 = 0; p0 < n; p0 += PC) {
-#pragma unroll
-        for(int q = 0; q < NC; ++q) {
-            const int j = p0 + grp + q * NG;
-#pragma unroll
-            for(int i = 0; i < RM; ++i) {
-                const int r = lane + i * G;
-                x[q][i] = j < n && r < m ? fa.A[it.a_off + int64_t(j) * m + r] : 0.0;
-            }
-        }
+        if(p0 > 0) load_panel(p0);
         for(int k = 0; k < min(p0, kmax); ++k) {
             load_v(k);
             apply(tau[k], p0 + grp, -1);
@@ -550,64 +635,9 @@ __global__ __launch_bounds__(QR_THREADS) void k_qr_tall(FactorArgs fa)
 {
     extern __shared__ double smem[];
     const xh_factor_item it = fa.items[blockIdx.x];
-    const int m = it.m, n = it.n;
-    const int qc = static_cast<int>(it.s_off);
-    if(m == 0 || n == 0) return;
-    constexpr int G = 64, NG = QR_THREADS / G;
-    const int kmax = min(m, n);
-    double* Wk = work_base<LDS>(smem, fa);  // m x n working copy
-    double* tau = Wk + int64_t(m) * n;      // kmax
-    const int tid = threadIdx.x, lane = tid % G, grp = tid / G;
-    for(int j = grp; j < n; j += NG)
-        for(int r = lane; r < m; r += G) Wk[int64_t(j) * m + r] = fa.A[it.a_off + int64_t(j) * m + r];
-    auto reflector = [&](int k) {  // from column k, whose rows this group's lanes wrote themselves
-        double* col = Wk + int64_t(k) * m;
-        double tail = 0.0, c0 = 0.0;
-        for(int r = lane; r < m; r += G) {
-            const double y = col[r];
-            if(r > k) tail = fma(y, y, tail);
-            if(r == k) c0 = y;
-        }
-        tail = xh::lanes_sum<G>(tail);
-        c0 = xh::lanes_sum<G>(c0);
-        double beta, t, inv;
-        make_householder(c0, tail, beta, t, inv);
-        for(int r = lane; r < m; r += G)
-            if(r >= k) col[r] = r == k ? beta : col[r] * inv;
-        if(lane == 0) tau[k] = t;
-    };
-    auto apply = [&](int k, double t, double* c) {  // c -= tau (v^T c) v, v = [1; column k below k]
-        const double* col = Wk + int64_t(k) * m;
-        double w = 0.0;
-        for(int r = lane; r < m; r += G)
-            if(r >= k) w = fma(r == k ? 1.0 : col[r], c[r], w);
-        w = xh::lanes_sum<G>(w) * t;
-        for(int r = lane; r < m; r += G)
-            if(r >= k) c[r] = fma(-w, r == k ? 1.0 : col[r], c[r]);
-    };
-    if(grp == 0) reflector(0);
-    for(int k = 0; k < kmax; ++k) {
-        __syncthreads();  // reflector k is there
-        const double t = tau[k];
-        const int first = k + 1;
-        for(int j = first + ((grp - first) % NG + NG) % NG; j < n; j += NG) {
-            if(t != 0.0) apply(k, t, Wk + int64_t(j) * m);
-            if(j == first && first < kmax) reflector(first);
-        }
-    }
-    __syncthreads();
-    // R: qc x n, upper triangle of the working copy (rows beyond min(m, n) are zero)
-    for(int64_t e = tid; e < int64_t(qc) * n; e += QR_THREADS) {
-        const int r = static_cast<int>(e % qc), c = static_cast<int>(e / qc);
-        fa.Vt[it.vt_off + e] = (r < m && r <= c) ? Wk[r + int64_t(c) * m] : 0.0;
-    }
-    for(int c = grp; c < qc; c += NG) {
-        double* qcol = fa.U + it.u_off + int64_t(c) * m;
-        for(int r = lane; r < m; r += G) qcol[r] = (r == c) ? 1.0 : 0.0;
-        if(c < m)
-            for(int k = min(c, kmax - 1); k >= 0; --k)
-                if(tau[k] != 0.0) apply(k, tau[k], qcol);
-    }
+    if(it.m == 0 || it.n == 0) return;
+    double* Wk = work_base<LDS>(smem, fa);
+    qr_in_memory(fa, it, Wk, it.m, Wk + int64_t(it.m) * it.n);
 }
 
 // Inverse of the upper Cholesky factor of a Gram block G + shift * trace(G) * I (the building
