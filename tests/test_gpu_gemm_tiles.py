@@ -83,3 +83,22 @@ def test_operands_beyond_32_bit_tile_offsets(rt):
     A, B = r.uniform(-1, 1, (3, k)), r.uniform(-1, 1, (k, 2))
     c, = _products(rt, [(A, B)], 1, 0)
     assert np.all(np.abs(c - A @ B) <= 2 * k * U * (np.abs(A) @ np.abs(B)))
+
+
+@pytest.mark.parametrize("shape", [(74, 74, 3000), (500, 500, 500)])
+def test_short_items_do_not_take_the_k_split_from_long_ones(rt, shape):
+    """The partial products of a call (its split along K) are those of its long items alone, however many
+    items of 256 x 16 x 16 run as tiles beside them."""
+    L, ctx = lib(), rt.ctx()
+    m, n, k = shape
+
+    def workspace(short):
+        items = [_lib.xh_gemm_item(0, 0, 0, m, n, k)] + [_lib.xh_gemm_item(0, 0, m * n + 4096 * i, 256, 16, 16) for i in range(short)]
+        plan, b = C.c_void_p(), C.c_int64()
+        assert L.xh_gemm_plan_create(ctx, (_lib.xh_gemm_item * len(items))(*items), len(items), 0, 0, C.byref(plan)) == 0
+        assert L.xh_gemm_plan_workspace(plan, C.byref(b)) == 0
+        L.xh_gemm_plan_destroy(ctx, plan)
+        return b.value
+
+    alone = workspace(0)
+    assert alone > 0 and [workspace(s) for s in (1, 100, 400, 2000)] == [alone] * 4

@@ -71,10 +71,11 @@ extern "C" int xh_destroy(xh_ctx* ctx)
 
 extern "C" const char* xh_last_error(const xh_ctx* ctx) { return ctx ? ctx->err.c_str() : "no context"; }
 
-// Item lists, rectangles and plan tables of a few KB go up as kernel arguments: 1.8 us on the device
-// against 3.6 for a copy command, and less work on the host (an MPS sweep step of QRs at chi 300 took
-// 200 us with the copies, 175 with this; a simple-update step's 336 small uploads 1.2 ms of kernel time,
-// now 0.6).  Two sizes, as every launch copies its whole argument block.
+// Item lists, rectangles and plan tables of a few KB go up as kernel arguments, which takes the host less
+// than a copy command through pinned memory.  A call of small QRs, copy | this: items of 40 bytes in all
+// 11.9 | 10.6 us, 1000 bytes 12.6 | 11.4, 1800 bytes 13.9 | 12.0, 2400 bytes 12.1 | 12.2, 3560 bytes 12.9 |
+// 12.5 (a step of QRs at chi 300: 200 | 175).  On the device the small payload takes 2.0 to 4.4 us, the
+// large one 3.0 to 4.6, a copy 3.3 to 4.0.  Two sizes, as every launch copies its whole argument block.
 namespace {
 template <int BYTES>
 struct Payload {

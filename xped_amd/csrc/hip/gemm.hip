@@ -3,8 +3,8 @@
 // The reference multiplies matched sectors one at a time with Eigen/BLAS
 // (src/Core/TensorBase.cpp:262-279 -> MatrixInterface::prod, MatrixInterface_Eigen_impl.cpp:155-160).
 // Here every (sector, output tile, K chunk) triple of one contraction is an entry of a work list
-// processed by one persistent launch (FP64: sectors with both output sides >= 192 in 128 x 128
-// tiles by one launch, the others in 64 x 64 tiles by a second).  The list is cut into 8 contiguous parts
+// processed by one persistent launch (FP64: large sectors in 128 x 128 tiles by one launch (is_big), the
+// others in tiles of 32 to 96 a side (pick_shape) by a second).  The list is cut into 8 contiguous parts
 // of equal work (sum of K over the tiles), one per XCD: workgroup b serves part b % 8, so the
 // tiles of one sector run on one XCD and share its L2, and uneven sector sizes are balanced.
 // Launches with few output tiles (a sketch's Gram matrix: a small output with a long K) split K
@@ -12,7 +12,7 @@
 // in a fixed order (deterministic) and applies alpha / beta.  Items with one short output side
 // (<= 32) and a short K (<= 32), as the contractions of a site tensor's physical or virtual leg
 // with a large environment tensor give, are memory-bound and run on a third kernel (one thread per
-// index of the long side, FP64 FMA) in the same call.
+// index of the long side, FP64 FMA) where all items of a call are such or enough of them (use_skinny).
 //
 // Precision modes (operands are always FP64 in memory, the output is FP64):
 //   XH_FP64   v_mfma_f64_16x16x4_f64, FP64 accumulation
@@ -393,8 +393,10 @@ __global__ __launch_bounds__(G8_THREADS, 4) void k_gemm_f64_128(GemmArgs g)
 }
 
 constexpr int FAR_SHAPE = 7;
-// Tiles of 32 to 96 rows by 32 to 96 columns, 4 waves in 2 x 2, four workgroups per CU: the shape is
-// chosen per item (pick_shape) so that little of a tile lies outside the output, and is carried by each tile.
+// Tiles of 32 to 96 rows by 32 to 96 columns, 4 waves in 2 x 2: the shape is chosen per item (pick_shape) so
+// that little of a tile lies outside the output, and is carried by each tile.  Four workgroups per CU by
+// their registers and by the 36 KB of LDS of shapes up to 64 x 64; the 46 KB of a 64 x 96 or 96 x 64 tile
+// leave three, and as the launch has the LDS of its largest tile, one such item leaves three for all.
 template <bool TA, bool TB>
 __global__ __launch_bounds__(G_THREADS, 4) void k_gemm_f64(GemmArgs g)
 {
@@ -1272,16 +1274,25 @@ int pick_shape(const xh_gemm_item& it, bool ta, bool tb)
     }
     return best;
 }
-// 128 x 128 tiles unless their padding costs more than the larger tile gains (192 x 192 fills 56 %)
+// 128 x 128 tiles unless they cover more than 1.4 times what 64 x 64 tiles cover (192 x 192: 1.78).  One
+// item in us, 128 | 64: 320 x 320 x 1000 (1.44) 30.6 | 22.5, 400 x 400 x 1000 (1.31) 31.7 | 25.4, 520 x
+// 520 x 1000 (1.23) 34.7 | 33.4, 700 x 700 x 1000 (1.19) 48.4 | 37.6; eight of the last 183 | 160.  So the
+// line lies too high for calls of up to eight items of these sizes.
 bool is_big(const xh_gemm_item& it, bool ta, bool tb)
 {
     return !far_item(it, ta, tb) && it.m >= BIG_MIN && it.n >= BIG_MIN && padded(it, BM2, BN2) <= 1.4 * padded(it, BM, BN);
 }
 bool fits_skinny(const xh_gemm_item& it) { return std::min(it.m, it.n) <= SK_MAX && it.k <= SK_KMAX; }
-// Whether a call's skinny-shaped items take the skinny kernel: where every item is one, or where
-// they fill the chip by themselves (256 indices of the long side a workgroup).  A few of them beside
-// other items are tiles of the launch that runs anyway: alone they are a launch of 6 to 14 us, the
-// latency of one index's sums (projector SVD at chi 256: 54 launches).
+// Whether a call's skinny-shaped items take the skinny kernel.
+//  * Where every item is one: then the call may be made by the gather product, whose sums are the
+//    skinny kernel's, and the two agree bit for bit.  (For its time alone it would be too often: one item
+//    of 3000 x 32 with K = 32 takes 11.9 us in the skinny kernel and 4.6 in tiles, with K = 4 5.1 and 4.4;
+//    20 items of 20000 x 8 with K = 4 10.0 and 22.6.)
+//  * Beside other items where they fill the chip by themselves, from two workgroups of 256 long indices
+//    per CU.  A few of them are tiles of the launch that runs anyway; alone they are a launch of 3 to 11
+//    us, the latency of one index's sums.  Beside one item of 64 x 64 x 64, own launch | tiles: 256
+//    workgroups of S = 4, K = 4 9.8 | 8.4 us, 512 10.5 | 10.9, 1024 12.3 | 15.6; of S = 16, K = 16 12.5 |
+//    8.2, 15.4 | 12.4, 19.9 | 17.8, and 4096 53 | 72.
 bool use_skinny(const std::vector<xh_gemm_item>& v, int num_cu)
 {
     int64_t blocks = 0;
@@ -1312,11 +1323,14 @@ extern "C" int xh_gemm_plan_create(xh_ctx* ctx, const xh_gemm_item* items, int64
         std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return double(v[a].m) * v[a].n * v[a].k > double(v[b].m) * v[b].n * v[b].k; });
         plan->skinny_kernel = use_skinny(v, std::max(ctx->num_cu, 1));
         auto is_skinny = [&](const xh_gemm_item& it) { return plan->skinny_kernel && fits_skinny(it); };
-        int64_t base_tiles = 0;  // output tiles of the FP64 launch
+        // output tiles of the FP64 launch that may be split along K; items with a short K that run as tiles
+        // beside them do not count, or they would take the split away from a long one (74 x 74 x 3000
+        // beside 256 items of 256 x 16 x 16: 17 us split, 86 us not)
+        int64_t base_tiles = 0;
         for(const auto& it : v) {
             if(it.m < 0 || it.n < 0 || it.k < 0) throw xh::Error(XH_EINVAL, "gemm plan: negative extent");
             if(it.a_off < 0 || it.b_off < 0 || it.c_off < 0) throw xh::Error(XH_EINVAL, "gemm plan: negative offset");
-            if(it.m == 0 || it.n == 0 || is_skinny(it)) continue;
+            if(it.m == 0 || it.n == 0 || fits_skinny(it)) continue;
             const bool big = is_big(it, trans_a != 0, trans_b != 0);
             const int sh = pick_shape(it, trans_a != 0, trans_b != 0);
             const int tm = big ? BM2 : SHAPE_M[sh], tn = big ? BN2 : SHAPE_N[sh];
@@ -1502,7 +1516,7 @@ void build_all64(xh_ctx* ctx, xh_gemm_plan* plan)
 }
 
 // XH_OZAKI takes the int8 path for items whose output sides and K are at least OZ_MIN (the matrix
-// cores' tiles are then mostly full); skinny items keep the FP64 skinny kernel and the others the
+// cores' tiles are then mostly full); items of the skinny kernel (use_skinny) keep it and the others the
 // 64 x 64 FP64 tiles, in the same call.  Both are FP64-accurate.
 constexpr int OZ_MIN = 64;
 bool oz_item(const xh_gemm_item& it) { return it.m >= OZ_MIN && it.n >= OZ_MIN && it.k >= OZ_MIN; }
@@ -1663,7 +1677,7 @@ void gemm_run(xh_ctx* ctx, const xh_gemm_plan* cplan, const double* A, const dou
             hipLaunchKernelGGL(kern, dim3(unsigned(plan->skinny.ntiles)), dim3(SK_THREADS), 0, ctx->stream, g, plan->skinny.d_tiles);
             xh::launch_check("k_gemm_skinny");
         };
-        // tiles: 0 = FP64 128x128 tiles for the large items and 64x64 for the rest, 1 = 64x64 only
+        // tiles: 0 = FP64 tiles by size and the skinny kernel (is_big, pick_shape, use_skinny), 1 = 64x64 only
         auto run = [&](int tiles) {
             if(precision == XH_FP64 && tiles == 0) {
                 launch_skinny();
