@@ -1,5 +1,5 @@
-"""Item lists of a call around the sizes at which their way to the device changes (512 and 3584 bytes,
-and lengths that are no multiple of 8), exact results (needs an MI355X)."""
+"""Item lists of a call around the sizes at which their way to the device changes (504 bytes, and lengths
+that are no multiple of 8), exact results (needs an MI355X)."""
 import ctypes as C
 
 import numpy as np

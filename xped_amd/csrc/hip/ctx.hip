@@ -71,41 +71,31 @@ extern "C" int xh_destroy(xh_ctx* ctx)
 
 extern "C" const char* xh_last_error(const xh_ctx* ctx) { return ctx ? ctx->err.c_str() : "no context"; }
 
-// Item lists, rectangles and plan tables of a few KB go up as kernel arguments, which takes the host less
-// than a copy command through pinned memory.  A call of small QRs, copy | this: items of 40 bytes in all
-// 11.9 | 10.6 us, 1000 bytes 12.6 | 11.4, 1800 bytes 13.9 | 12.0, 2400 bytes 12.1 | 12.2, 3560 bytes 12.9 |
-// 12.5 (a step of QRs at chi 300: 200 | 175).  On the device the small payload takes 2.0 to 4.4 us, the
-// large one 3.0 to 4.6, a copy 3.3 to 4.0.  Two sizes, as every launch copies its whole argument block.
+// Item lists of up to PUT_MAX bytes go up as kernel arguments: 2.0 us on the device against 3.3 to 4.0 for
+// a copy command (a call of 1 to 12 QRs of 4 x 4, 40 to 480 bytes: 12.3 -> 11.2 us; a step of QRs at chi
+// 300: 200 -> 178).  It takes the host up to 1 us more than a copy.  With a payload of 3.5 KB that was 1.3
+// to 2 us for an upload of 1 KB (a GEMM plan made and destroyed: 4.7 -> 6.2 us; 33 diagonal blocks inverted:
+// 7.1 -> 9.1), and nothing less on the device, so larger lists are copied.
 namespace {
-template <int BYTES>
+constexpr size_t PUT_BYTES = xh::PUT_MAX + 8;  // the word of a tail of single bytes is inside it
 struct Payload {
-    uint64_t w[BYTES / 8];
+    uint64_t w[PUT_BYTES / 8];
 };
-template <int BYTES>
-__global__ __launch_bounds__(64) void k_put(Payload<BYTES> p, unsigned char* __restrict__ dst, int bytes)
+__global__ __launch_bounds__(64) void k_put(Payload p, unsigned char* __restrict__ dst, int bytes)
 {
     const int words = bytes / 8;
     for(int i = threadIdx.x; i < words; i += 64) reinterpret_cast<uint64_t*>(dst)[i] = p.w[i];
     const int i = words * 8 + threadIdx.x;
     if(i < bytes) dst[i] = static_cast<unsigned char>(p.w[words] >> (8 * threadIdx.x));
 }
-template <int BYTES>
-void put(xh_ctx* ctx, void* dst, const void* src, size_t bytes)
-{
-    Payload<BYTES> p;
-    std::memcpy(&p, src, bytes);
-    std::memset(reinterpret_cast<char*>(&p) + bytes, 0, BYTES - bytes);
-    hipLaunchKernelGGL(k_put<BYTES>, dim3(1), dim3(64), 0, ctx->stream, p, static_cast<unsigned char*>(dst), static_cast<int>(bytes));
-    xh::launch_check("k_put");
-}
 }  // namespace
 void xh::put_small(xh_ctx* ctx, void* dst, const void* src, size_t bytes)
 {
-    // strictly below the payload: the word of a tail of single bytes is inside it
-    if(bytes < 512)
-        put<512>(ctx, dst, src, bytes);
-    else
-        put<PUT_MAX + 8>(ctx, dst, src, bytes);
+    Payload p;
+    std::memcpy(&p, src, bytes);
+    std::memset(reinterpret_cast<char*>(&p) + bytes, 0, PUT_BYTES - bytes);
+    hipLaunchKernelGGL(k_put, dim3(1), dim3(64), 0, ctx->stream, p, static_cast<unsigned char*>(dst), static_cast<int>(bytes));
+    xh::launch_check("k_put");
 }
 
 extern "C" int xh_alloc(xh_ctx* ctx, size_t bytes, void** dptr)

@@ -369,9 +369,9 @@ inline void* slab_take(xh_ctx* ctx, size_t bytes)
     return static_cast<char*>(ctx->slab.p) + off;
 }
 
-// A few KB of host memory to the device as the arguments of a small kernel (ctx.hip), in stream order:
-// they are copied at the launch, so src may go as soon as this returns.
-constexpr size_t PUT_MAX = 3584;
+// Up to PUT_MAX bytes of host memory to the device as the arguments of a small kernel (ctx.hip), in
+// stream order: they are copied at the launch, so src may go as soon as this returns.
+constexpr size_t PUT_MAX = 504;
 void put_small(xh_ctx* ctx, void* dst, const void* src, size_t bytes);
 
 // Asynchronous copy of host memory to the device, ordered on the context stream; the caller may
