@@ -8,6 +8,7 @@ import ctypes as C
 
 import numpy as np
 import pytest
+import torch
 
 from xped_amd import _lib
 from xped_amd._lib import lib
@@ -18,7 +19,17 @@ U = 2.0 ** -53
 SIDES = [1, 31, 32, 33, 64, 65, 95, 96, 97, 128, 129, 191, 193, 200, 257]
 
 
-def _products(rt, mats, ta, tb):
+def _workspace(rt, shapes, ta=0, tb=0):
+    """Device bytes of the split-K partials of a plan."""
+    L, plan, b = lib(), C.c_void_p(), C.c_int64()
+    items = (_lib.xh_gemm_item * len(shapes))(*[_lib.xh_gemm_item(0, 0, 0, *s) for s in shapes])
+    assert L.xh_gemm_plan_create(rt.ctx(), items, len(shapes), ta, tb, C.byref(plan)) == 0
+    assert L.xh_gemm_plan_workspace(plan, C.byref(b)) == 0
+    L.xh_gemm_plan_destroy(rt.ctx(), plan)
+    return b.value
+
+
+def _products(rt, mats, ta, tb, gemm=None):
     """C of every (A, B) in one grouped call; operands stored column-major, transposed where asked."""
     L, ctx = lib(), rt.ctx()
     items, ao, bo, co, fa, fb = [], 0, 0, 0, [], []
@@ -38,7 +49,7 @@ def _products(rt, mats, ta, tb):
     arr = (_lib.xh_gemm_item * len(items))(*items)
     plan = C.c_void_p()
     assert L.xh_gemm_plan_create(ctx, arr, len(items), ta, tb, C.byref(plan)) == 0
-    assert L.xh_gemm(ctx, plan, *bufs, 1.0, 0.0, _lib.XH_FP64) == 0, L.xh_last_error(ctx)
+    assert (gemm or L.xh_gemm)(ctx, plan, *bufs, 1.0, 0.0, _lib.XH_FP64) == 0, L.xh_last_error(ctx)
     out = np.empty(co)
     L.xh_download(ctx, out.ctypes.data, bufs[2], 8 * co)
     L.xh_gemm_plan_destroy(ctx, plan)
@@ -89,16 +100,38 @@ def test_operands_beyond_32_bit_tile_offsets(rt):
 def test_short_items_do_not_take_the_k_split_from_long_ones(rt, shape):
     """The partial products of a call (its split along K) are those of its long items alone, however many
     items of 256 x 16 x 16 run as tiles beside them."""
-    L, ctx = lib(), rt.ctx()
-    m, n, k = shape
+    alone = _workspace(rt, [shape])
+    assert alone > 0 and [_workspace(rt, [shape] + [(256, 16, 16)] * s) for s in (1, 100, 400, 2000)] == [alone] * 4
 
-    def workspace(short):
-        items = [_lib.xh_gemm_item(0, 0, 0, m, n, k)] + [_lib.xh_gemm_item(0, 0, m * n + 4096 * i, 256, 16, 16) for i in range(short)]
-        plan, b = C.c_void_p(), C.c_int64()
-        assert L.xh_gemm_plan_create(ctx, (_lib.xh_gemm_item * len(items))(*items), len(items), 0, 0, C.byref(plan)) == 0
-        assert L.xh_gemm_plan_workspace(plan, C.byref(b)) == 0
-        L.xh_gemm_plan_destroy(ctx, plan)
-        return b.value
 
-    alone = workspace(0)
-    assert alone > 0 and [workspace(s) for s in (1, 100, 400, 2000)] == [alone] * 4
+@pytest.mark.parametrize("ta,tb", [(0, 0), (1, 1)])
+def test_split_has_no_more_chunks_than_plain_tiles_give(rt, ta, tb):
+    """Partials of a plan, whatever its tile shapes, against the split that 64 x 64 tiles (128 x 128 from 192
+    a side) give: chunks for 4 tiles per CU, of at least 128 in multiples of 16."""
+    target = 4 * torch.cuda.get_device_properties(0).multi_processor_count
+
+    def bound(shapes):
+        tiles = sum(-(-m // t) * -(-n // t) for m, n, _ in shapes for t in [128 if min(m, n) >= 192 else 64])
+        chunks = -(-target // tiles) if tiles < target else 1
+        total = 0
+        for m, n, k in shapes:
+            kc = max(128, (-(-k // chunks) + 15) // 16 * 16)
+            if chunks > 1 and k >= 256 and -(-k // kc) > 1:
+                total += 8 * m * n * -(-k // kc)
+        return total
+
+    sides = [33, 65, 74, 96, 97, 130, 192, 200, 260, 390, 700, 1900]
+    for m in sides:
+        for n in sides:
+            for k in (300, 2000, 8000):
+                for count in (1, 5, 18):
+                    assert _workspace(rt, [(m, n, k)] * count, ta, tb) <= bound([(m, n, k)] * count), (m, n, k, count)
+    assert _workspace(rt, [(1900, 74, 500)] * 18, ta, tb) == 0  # not split, so it may be captured
+
+
+def test_noalloc_takes_a_long_sketch_product(rt):
+    """1900 x 74 with K = 8000 has partials below the array's 32 MiB."""
+    r = np.random.default_rng(4)
+    A, B = r.uniform(-1, 1, (1900, 8000)), r.uniform(-1, 1, (8000, 74))
+    c, = _products(rt, [(A, B)], 0, 0, lib().xh_gemm_noalloc)
+    assert np.all(np.abs(c - A @ B) <= 2 * A.shape[1] * U * (np.abs(A) @ np.abs(B)))

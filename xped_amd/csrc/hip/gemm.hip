@@ -1323,22 +1323,33 @@ extern "C" int xh_gemm_plan_create(xh_ctx* ctx, const xh_gemm_item* items, int64
         std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return double(v[a].m) * v[a].n * v[a].k > double(v[b].m) * v[b].n * v[b].k; });
         plan->skinny_kernel = use_skinny(v, std::max(ctx->num_cu, 1));
         auto is_skinny = [&](const xh_gemm_item& it) { return plan->skinny_kernel && fits_skinny(it); };
-        // output tiles of the FP64 launch that may be split along K; items with a short K that run as tiles
+        // the tiles of each item: FP64 128 x 128, or a shape of k_gemm_f64
+        constexpr uint8_t BIG = 255;
+        std::vector<uint8_t> shape(v.size(), 0);
+        // Output tiles of the FP64 launch that may be split along K.  Items with a short K that run as tiles
         // beside them do not count, or they would take the split away from a long one (74 x 74 x 3000
-        // beside 256 items of 256 x 16 x 16: 17 us split, 86 us not)
-        int64_t base_tiles = 0;
-        for(const auto& it : v) {
+        // beside 256 items of 256 x 16 x 16: 17 us split, 86 us not).  plain_tiles: the same with 64 x 64
+        // tiles, and 128 x 128 from BIG_MIN a side.  A split has at most as many chunks as that count
+        // gives, so that whether a plan's partials fit xh_gemm_noalloc's array, and whether it has any
+        // and is refused under capture, does not hang on the tile shapes.
+        int64_t base_tiles = 0, plain_tiles = 0;
+        for(size_t i = 0; i < v.size(); ++i) {
+            const xh_gemm_item& it = v[i];
             if(it.m < 0 || it.n < 0 || it.k < 0) throw xh::Error(XH_EINVAL, "gemm plan: negative extent");
             if(it.a_off < 0 || it.b_off < 0 || it.c_off < 0) throw xh::Error(XH_EINVAL, "gemm plan: negative offset");
-            if(it.m == 0 || it.n == 0 || fits_skinny(it)) continue;
+            if(it.m == 0 || it.n == 0 || is_skinny(it)) continue;
             const bool big = is_big(it, trans_a != 0, trans_b != 0);
-            const int sh = pick_shape(it, trans_a != 0, trans_b != 0);
-            const int tm = big ? BM2 : SHAPE_M[sh], tn = big ? BN2 : SHAPE_N[sh];
+            shape[i] = big ? BIG : static_cast<uint8_t>(pick_shape(it, trans_a != 0, trans_b != 0));
+            if(fits_skinny(it)) continue;
+            const int tm = big ? BM2 : SHAPE_M[shape[i]], tn = big ? BN2 : SHAPE_N[shape[i]];
+            const int tp = it.m >= BIG_MIN && it.n >= BIG_MIN ? BM2 : BM;
             base_tiles += int64_t((it.m + tm - 1) / tm) * ((it.n + tn - 1) / tn);
+            plain_tiles += int64_t((it.m + tp - 1) / tp) * ((it.n + tp - 1) / tp);
         }
         // K split: aim at 4 tiles per CU, chunks of at least 128
         const int64_t target = 4 * int64_t(std::max(ctx->num_cu, 1));
-        const int64_t S = base_tiles > 0 && base_tiles < target ? (target + base_tiles - 1) / base_tiles : 1;
+        const int64_t count = std::max(base_tiles, plain_tiles);
+        const int64_t S = count > 0 && count < target ? (target + count - 1) / count : 1;
         std::vector<ItemExt> ext(v.size(), ItemExt{1, 0, 0});
         std::vector<RedItem> red;
         std::vector<Tile> t_big, t_rest, t_sk;
@@ -1367,8 +1378,8 @@ extern "C" int xh_gemm_plan_create(xh_ctx* ctx, const xh_gemm_item* items, int64
                     plan->max_red_mn = std::max(plan->max_red_mn, mn);
                 }
             }
-            const bool big = is_big(it, trans_a != 0, trans_b != 0);
-            const int sh = pick_shape(it, trans_a != 0, trans_b != 0), tm = SHAPE_M[sh], tn = SHAPE_N[sh];
+            const bool big = shape[id] == BIG;
+            const int sh = big ? 0 : shape[id], tm = SHAPE_M[sh], tn = SHAPE_N[sh];
             if(e.split > KS_MASK) throw xh::Error(XH_EINVAL, "gemm plan: too many K chunks");
             if(!big) plan->lds64 = std::max(plan->lds64, tile_lds(trans_a != 0, trans_b != 0, tm, tn));
             for(int ks = 0; ks < e.split; ++ks) {
