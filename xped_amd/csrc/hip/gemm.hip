@@ -1263,10 +1263,12 @@ double padded(const xh_gemm_item& it, int tm, int tn) { return double((it.m + tm
 int pick_shape(const xh_gemm_item& it, bool ta, bool tb)
 {
     if(far_item(it, ta, tb)) return FAR_SHAPE;
+    const auto covered = [](int x, int t) { return double((x + t - 1) / t) * t; };
+    const double pm[3] = {covered(it.m, 32), covered(it.m, 64), covered(it.m, 96)}, pn[3] = {covered(it.n, 32), covered(it.n, 64), covered(it.n, 96)};
     int best = 0;
     double least = 0.0;
     for(int c = 0; c < NSHAPE; ++c) {
-        const double cost = padded(it, SHAPE_M[c], SHAPE_N[c]) * (1.0 + 8.0 / SHAPE_M[c] + 8.0 / SHAPE_N[c]);
+        const double cost = pm[SHAPE_M[c] / 32 - 1] * pn[SHAPE_N[c] / 32 - 1] * (1.0 + 8.0 / SHAPE_M[c] + 8.0 / SHAPE_N[c]);
         if(c == 0 || cost < least) {
             best = c;
             least = cost;
