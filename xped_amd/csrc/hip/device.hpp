@@ -173,8 +173,7 @@ struct FastDiv {
 inline FastDiv make_fastdiv(uint32_t d)
 {
     FastDiv f{d, 0, 0};
-    uint32_t l = 0;
-    while((uint64_t(1) << l) < d) ++l;
+    const uint32_t l = d > 1 ? 32 - static_cast<uint32_t>(__builtin_clz(d - 1)) : 0;  // the least l with 2^l >= d
     f.shift = l;
     f.magic = static_cast<uint32_t>(((uint64_t(1) << 32) * ((uint64_t(1) << l) - d)) / d + 1);
     return f;

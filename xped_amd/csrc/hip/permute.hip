@@ -130,8 +130,8 @@ struct PermC {
 // PER: 4 (8 was slower: 73 us in the first example below, 143 with several sources, by registers and
 // LDS), or 2 for small tensors, whose time is the latency of one workgroup.
 // Bound by the loads of 8 bytes at L2 line granularity and by the decode: 16.8 M elements of a
-// seven-leg tensor in 46508 tasks 70 us (3.8 TB/s, a copy of the size takes 56), 15.5 M elements from
-// 26.8 M sources of an eight-leg SU(2) tensor 110 us.  (All legs decoded per element from int64
+// seven-leg tensor in 46508 tasks 68 us (3.9 TB/s, a copy of the size takes 56), 15.5 M elements from
+// 26.8 M sources of an eight-leg SU(2) tensor 112 us.  (All legs decoded per element from int64
 // strides, a thread's elements one after the other where they have several sources: 88 and 148.)
 constexpr int MC_CAP = 48;    // tasks of a tile whose records are staged in LDS
 constexpr int MC_LEGS = 8;    // legs of a staged task
@@ -442,27 +442,46 @@ extern "C" int xh_permute_plan_create(xh_ctx* ctx, const xh_permute_desc* desc, 
             int nl1 = 0, nl2 = 0;  // most joined legs of a gather task, with absolute strides and with row / column strides
         };
         // The legs of a task joined (LegC): absolute source strides (abs: one source, its leading
-        // dimension folded in), or source row and column strides.  Calls put(extent, stride, is_col).
-        auto join_legs = [NL](const xh_permute_task& tk, int64_t ld, bool abs, auto&& put) {
-            uint32_t ext = 1;
-            int64_t st = 0;
-            bool col = false;
-            for(int q = 0; q < NL; ++q) {
-                if(tk.ext[q] == 1) continue;
-                const bool c = !abs && tk.is_col[q] != 0;
-                const int64_t sq = tk.sstride[q] * (abs && tk.is_col[q] ? ld : 1);
-                if(ext > 1 && c == col && sq == st * ext) {
-                    ext *= tk.ext[q];
-                    continue;
-                }
-                if(ext > 1) put(ext, st, col);
-                ext = tk.ext[q];
-                st = sq;
-                col = c;
-            }
-            if(ext > 1) put(ext, st, col);
+        // dimension folded in), or source row and column strides.  Leg q joins the one before it (of extent >
+        // 1) if it goes on where that one ends, so that no leg waits for the products of earlier ones, and
+        // there are no branches, which would be guessed wrong for about every leg.  Pass 1 only counts.
+        struct Joined {
+            uint32_t ext;
+            int32_t col;
+            int64_t st;
         };
-        const size_t nchunk = NT >= 16384 ? std::max<size_t>(1, std::min<size_t>(xp::WorkerPool::get().size(), size_t(NT) / 4096)) : 1;
+        auto join_legs = [NL](const xh_permute_task& tk, int64_t ld, bool abs, auto&& leg) {
+            int64_t end = 0;     // where the leg before ends
+            int32_t before = 2;  // its kind: 0 row, 1 column, 2 none
+            for(int q = 0; q < NL; ++q) {
+                const uint32_t e = tk.ext[q];
+                const bool is_col = tk.is_col[q] != 0;
+                const int32_t c = !abs & is_col;
+                const int64_t st = tk.sstride[q] * (abs & is_col ? ld : 1);
+                const bool one = e == 1, joins = (c == before) & (st == end);
+                leg(!one & !joins, e, c, st);  // a new joined leg starts, or the present one is e times longer
+                end = one ? end : st * e;
+                before = one ? before : c;
+            }
+        };
+        auto count_joined = [&join_legs](const xh_permute_task& tk, int64_t ld, bool abs, bool& far) {
+            int n = 0;
+            bool f = false;
+            join_legs(tk, ld, abs, [&](bool fresh, uint32_t, int32_t, int64_t st) {
+                n += fresh;
+                f |= fresh & (uint64_t(st) >= (uint64_t(1) << 31));
+            });
+            far |= f;
+            return n;
+        };
+        auto count_rows_cols = [&count_joined, NL](const xh_permute_task& tk, bool& far) {
+            int64_t reach[2] = {0, 0};  // largest source row and column
+            for(int q = 0; q < NL; ++q) reach[tk.is_col[q] != 0] += (int64_t(tk.ext[q]) - 1) * tk.sstride[q];
+            far |= std::max(reach[0], reach[1]) >= (int64_t(1) << 31);
+            return count_joined(tk, 1, false, far);
+        };
+        // from 2048 tasks on several host threads: 5800 tasks of ten legs 330 us, 870 on one
+        const size_t nchunk = NT >= 2048 ? std::max<size_t>(1, std::min<size_t>(xp::WorkerPool::get().size(), size_t(NT) / 1024)) : 1;
         std::vector<ChunkCount> cc(nchunk);
         auto chunk_lo = [&](size_t c) { return int64_t(size_t(NT) * c / nchunk); };
         auto classify = [&](size_t c) {
@@ -508,20 +527,14 @@ extern "C" int xh_permute_plan_create(xh_ctx* ctx, const xh_permute_desc* desc, 
                     slot[t] = k.ngather;
                     ++k.ngather;
                     k.total += tk.rows * tk.cols;
-                    int n1 = 0, n2 = 0;
-                    int64_t rmax = 0, cmax = 0;
-                    join_legs(tk, 1, false, [&](uint32_t ext, int64_t st, bool col) {
-                        (col ? cmax : rmax) += int64_t(ext - 1) * st;
-                        ++n2;
-                    });
-                    if(std::max(rmax, cmax) >= (int64_t(1) << 31)) k.near = false;
+                    // one source: most likely of every task, so row and column strides are counted only
+                    // if they turn out to be needed
+                    bool far = false;
                     if(tk.nsrc == 1)
-                        join_legs(tk, desc->sources[tk.src_begin].src_ld, true, [&](uint32_t, int64_t st, bool) {
-                            if(st < 0 || st >= (int64_t(1) << 31)) k.near = false;
-                            ++n1;
-                        });
-                    k.nl1 = std::max(k.nl1, n1);
-                    k.nl2 = std::max(k.nl2, n2);
+                        k.nl1 = std::max(k.nl1, count_joined(tk, desc->sources[tk.src_begin].src_ld, true, far));
+                    else
+                        k.nl2 = std::max(k.nl2, count_rows_cols(tk, far));
+                    if(far) k.near = false;
                 }
             }
         };
@@ -546,6 +559,13 @@ extern "C" int xh_permute_plan_create(xh_ctx* ctx, const xh_permute_desc* desc, 
             if(!cc[c].single) plan->single_src = false;
         }
         const bool single = plan->single_src;
+        if(!single)  // tasks with one source among tasks with several
+            for(int64_t t = 0; t < NT; ++t)
+                if(route[t] <= 0 && desc->tasks[t].nsrc == 1) {
+                    bool far = false;
+                    cc[0].nl2 = std::max(cc[0].nl2, count_rows_cols(desc->tasks[t], far));
+                    if(far) cc[0].near = false;
+                }
         int nl = 0;
         bool ordered = true;
         plan->compact = ngather > 0;
@@ -599,18 +619,25 @@ extern "C" int xh_permute_plan_create(xh_ctx* ctx, const xh_permute_desc* desc, 
                     slot[t] += base[c].ngather;
                     prefix[slot[t]] = e;
                     const int64_t e_end = e + tk.rows * tk.cols;
-                    for(int64_t i = (e + tile - 1) / tile; i * tile < e_end; ++i) tile_first[i] = static_cast<int32_t>(slot[t]);
+                    const int64_t i0 = (e + tile - 1) / tile, i1 = (e_end + tile - 1) / tile;
+                    if(i0 < i1) std::fill(tile_first + i0, tile_first + i1, static_cast<int32_t>(slot[t]));
                     e = e_end;
                     if(compact) {
                         const xh_permute_source* so = single ? desc->sources + tk.src_begin : nullptr;
                         const xh::FastDiv fd = xh::make_fastdiv(uint32_t(std::max<int64_t>(tk.rows, 1)));
                         LegC* L = legc + slot[t] * nl;
+                        Joined J[XH_MAXLEGS + 1], j{1, 0, 0};
+                        for(int k = 1; k <= nl; ++k) J[k] = j;
                         uint32_t n = 0;
-                        join_legs(tk, so ? so->src_ld : 1, single, [&](uint32_t ext, int64_t st, bool col) {
-                            const xh::FastDiv d = xh::make_fastdiv(ext);
-                            L[n++] = LegC{ext, d.magic, d.shift | (col ? 256u : 0u), static_cast<uint32_t>(st)};
+                        join_legs(tk, so ? so->src_ld : 1, single, [&](bool fresh, uint32_t e, int32_t col, int64_t st) {
+                            n += fresh;
+                            j = Joined{(fresh ? 1 : j.ext) * e, fresh ? col : j.col, fresh ? st : j.st};
+                            J[n] = j;
                         });
-                        for(int k = static_cast<int>(n); k < nl; ++k) L[k] = LegC{1, 0, 0, 0};
+                        for(int k = 0; k < nl; ++k) {
+                            const xh::FastDiv d = xh::make_fastdiv(J[k + 1].ext);
+                            L[k] = LegC{d.d, d.magic, d.shift | uint32_t(J[k + 1].col << 8), static_cast<uint32_t>(J[k + 1].st)};
+                        }
                         taskc[slot[t]] = TaskC{tk.dst_off, tk.dst_ld, so ? so->src_off : 0, so ? so->coeff : 0.0, uint32_t(tk.rows), fd.magic, fd.shift, n,
                                                tk.nsrc, tk.src_begin};
                         continue;
