@@ -137,6 +137,66 @@ constexpr int MC_CAP = 48;    // tasks of a tile whose records are staged in LDS
 constexpr int MC_LEGS = 8;    // legs of a staged task
 constexpr int SRC_CAP = 192;  // their sources (several per task)
 
+// A tile inside one task: its records are the same for every lane and come through scalar loads, a leg at a
+// time for all elements of a thread.  6 M elements of ten legs that do not join, in 102 tasks: 24 us with one
+// source and 48 with four (from LDS or global memory like the other tiles 46 and 79; before there were
+// compact tasks 33 and 50).
+template <bool SINGLE, int PER>
+__device__ __forceinline__ void one_task(const PermC& p, int t, int64_t e0, int n_here, const double* __restrict__ src, double* __restrict__ dst)
+{
+    const TaskC tk = p.task[t];
+    const LegC* L = p.legs + int64_t(t) * p.nlegs;
+    uint32_t x[PER];
+    int64_t dpos[PER], off[PER];
+    uint32_t row[SINGLE ? 1 : PER], col[SINGLE ? 1 : PER];
+    const int64_t base = e0 - p.prefix[t];
+#pragma unroll
+    for(int i = 0; i < PER; ++i) {
+        const int r = threadIdx.x + i * PT_THREADS;
+        // an element past the end is taken as the first of the tile, and not stored
+        x[i] = static_cast<uint32_t>(base + (r < n_here ? r : 0));
+        const uint32_t c = xh::fdiv(x[i], tk.rmagic, tk.rshift);
+        dpos[i] = tk.dst_off + (x[i] - c * tk.rows) + int64_t(c) * tk.dst_ld;
+        off[i] = tk.src_off;
+        if constexpr(!SINGLE) row[i] = col[i] = 0;
+    }
+    for(uint32_t k = 0; k < tk.nl; ++k) {
+        const LegC l = L[k];
+#pragma unroll
+        for(int i = 0; i < PER; ++i) {
+            const uint32_t q = xh::fdiv(x[i], l.magic, l.shift & 255u), d = x[i] - q * l.ext;
+            if constexpr(SINGLE)
+                off[i] += uint64_t(d) * l.stride;
+            else if(l.shift & 256u)
+                col[i] += d * l.stride;
+            else
+                row[i] += d * l.stride;
+            x[i] = q;
+        }
+    }
+    double val[PER];
+    if constexpr(SINGLE) {
+#pragma unroll
+        for(int i = 0; i < PER; ++i) val[i] = src[off[i]];
+#pragma unroll
+        for(int i = 0; i < PER; ++i) val[i] = __dadd_rn(0.0, __dmul_rn(tk.coeff, val[i]));
+    } else {
+#pragma unroll
+        for(int i = 0; i < PER; ++i) val[i] = 0.0;
+        for(int s = 0; s < tk.nsrc; ++s) {
+            const xh_permute_source so = p.src[tk.src_begin + s];
+            double v[PER];
+#pragma unroll
+            for(int i = 0; i < PER; ++i) v[i] = src[so.src_off + row[i] + int64_t(col[i]) * so.src_ld];
+#pragma unroll
+            for(int i = 0; i < PER; ++i) val[i] = __dadd_rn(val[i], __dmul_rn(so.coeff, v[i]));
+        }
+    }
+#pragma unroll
+    for(int i = 0; i < PER; ++i)
+        if(int(threadIdx.x) + i * PT_THREADS < n_here) dst[dpos[i]] = val[i];
+}
+
 template <bool SINGLE, int PER>
 __global__ __launch_bounds__(PT_THREADS) void k_permute_compact(PermC p, const double* __restrict__ src, double* __restrict__ dst)
 {
@@ -148,6 +208,10 @@ __global__ __launch_bounds__(PT_THREADS) void k_permute_compact(PermC p, const d
     const int64_t e0 = int64_t(blockIdx.x) * TILE;
     const int n_here = static_cast<int>(min(int64_t(TILE), p.total - e0));
     const int t_lo = p.tile_first[blockIdx.x], t_hi = p.tile_first[blockIdx.x + 1];
+    if(t_lo == t_hi) {
+        one_task<SINGLE, PER>(p, __builtin_amdgcn_readfirstlane(t_lo), e0, n_here, src, dst);
+        return;
+    }
     // tasks t_lo .. t_hi intersect the tile; at most TILE + 1 since every task holds an element
     const int nt = t_hi - t_lo + 1, nl_max = p.nlegs;
     const bool staged = nt <= MC_CAP && nl_max <= MC_LEGS;  // uniform over the workgroup
