@@ -231,14 +231,21 @@ def test_ozaki_gemm_error_bound_and_nonfinite_rows(rt, ta, tb):
         assert np.max(err[ok] / scale[ok]) <= 4.0 * max(np.max(np.abs(f64 - ref)[ok] / scale[ok]), 2.0 ** -53)
 
 
+SKINNY = [(16, 5000, 9), (7000, 24, 13), (32, 300, 32), (31, 31, 31), (1, 2000, 1), (3000, 1, 5), (5, 7, 0), (9, 9000, 8)]
+
+
 @pytest.mark.parametrize("ta,tb", [(0, 0), (1, 0), (0, 1), (1, 1)])
-def test_grouped_gemm_skinny_items(rt, ta, tb):
-    # items with a short output side (<= 32) and K <= 32 run on the memory-bound skinny kernel,
-    # mixed in one plan with items on the matrix-core tiles; FP64 to 1e-12
+@pytest.mark.parametrize("beside", [[(200, 150, 40)], [], [(200, 150, 40), (400000, 8, 3)], [s for s in SKINNY if min(s[:2]) > 8]],
+                         ids=["few-beside-another", "alone", "many-beside-another", "alone-short8"])
+def test_grouped_gemm_skinny_items(rt, ta, tb, beside):
+    # items with a short output side (<= 32) and K <= 32, with alpha, beta and K = 0, FP64 to 1e-12.  Alone
+    # in a call, or enough of them to fill the chip (two workgroups of 256 long indices per CU), they run
+    # on the memory-bound skinny kernel, the latter before the tiles of another item; a few beside another
+    # item are tiles themselves.  Of short sides up to 8 alone: the kernel with scalar operands.
     L = lib()
     ctx = rt.ctx()
     r = np.random.default_rng(9)
-    shapes = [(16, 5000, 9), (7000, 24, 13), (32, 300, 32), (31, 31, 31), (1, 2000, 1), (3000, 1, 5), (5, 7, 0), (200, 150, 40), (9, 9000, 8)]
+    shapes = [s for s in SKINNY if s not in beside] if beside and beside[0] in SKINNY else SKINNY[:7] + beside + SKINNY[7:]
     items, ao, bo, co = [], 0, 0, 0
     for m, n, k in shapes:
         items.append({"a": ao, "b": bo, "c": co, "m": m, "n": n, "k": k})

@@ -113,8 +113,8 @@ def test_cholesky_inverse_kernel(rt):
     ctx = rt.ctx()
     r = np.random.default_rng(7)
     blocks = []
-    # n = 199 is the largest block held in LDS (packed upper triangle); n = 200 and 300 run from
-    # a global working copy
+    # n = 192 is the largest block held in LDS (16 x 16 tiles of the upper triangle); n = 199, 200 and
+    # 300 run from a global working copy
     for m, n in [(50, 20), (200, 130), (9, 9), (30, 6), (2, 2), (3, 3), (160, 141), (260, 180), (230, 199), (240, 200), (400, 300)]:
         Y = r.standard_normal((m, n))
         if n > 2:
