@@ -1961,16 +1961,27 @@ extern "C" int xh_gather_plan_create(xh_ctx* ctx, const xh_gemm_plan* gemm, cons
         // blocks of at most SK_THREADS rows meeting at most GA_SEG domain trees, in the GEMM plan's
         // item order, and the places of the items' tables
         struct TreeAt {
-            int64_t item;
-            int32_t a, nl = 0;
-            int32_t leg[GA_MAXR] = {};  // first domain leg of each joined leg
-            uint32_t ext[GA_MAXR] = {};
+            int32_t item, a;
+            int32_t nl = 0;
             bool far = false;
+            uint8_t leg[GA_MAXR] = {};  // first domain leg of each joined leg
+            uint32_t ext[GA_MAXR] = {};
         };
         std::vector<GatherBlock> blocks;
         std::vector<GatherBlock> items(size_t(d->nitems));  // an item's part of its blocks
         std::vector<TreeAt> trees;
         int64_t noffs = 0, npairs = 0;
+        {
+            size_t nt = 0, nb = 0;
+            for(int64_t j = 0; j < d->nitems; ++j) {
+                const xh_gemm_item& it = gemm->h_items[j];
+                if(it.m == 0 || it.n == 0) continue;
+                nt += size_t(d->items[j].ndom);
+                nb += size_t(it.m / SK_THREADS + d->items[j].ndom / GA_SEG + 2);
+            }
+            trees.reserve(nt);
+            blocks.reserve(nb);
+        }
         for(int64_t j = 0; j < d->nitems; ++j) {
             const xh_gemm_item& it = gemm->h_items[j];
             const xh_gather_item& g = d->items[j];
@@ -1981,7 +1992,7 @@ extern "C" int xh_gather_plan_create(xh_ctx* ctx, const xh_gemm_plan* gemm, cons
             for(int b = 0; b < g.ncod; ++b) items[j].first |= 1u << cs[b];
             noffs += int64_t(g.ndom) * it.k;
             npairs += int64_t(g.ndom) * g.ncod;
-            for(int a = 0; a < g.ndom; ++a) trees.push_back(TreeAt{j, a});
+            for(int a = 0; a < g.ndom; ++a) trees.push_back(TreeAt{int32_t(j), a});
             int a = 0;
             for(int r = 0; r < it.m;) {
                 GatherBlock bl = items[j];
@@ -2074,15 +2085,21 @@ extern "C" int xh_gather_plan_create(xh_ctx* ctx, const xh_gemm_plan* gemm, cons
                         h_st[at] = uint32_t(st);
                         if(far) h_hi[at] = uint32_t(st >> 32);
                     }
-                    for(int64_t c = 0; c < tk.cols; ++c, ++kk) {  // column kk: its index along the codomain legs
-                        int64_t x = c, o = so.src_off;
-                        for(int k = NR; k < NL; ++k) {
-                            if(tk.ext[k] == 1) continue;
-                            o += (x % tk.ext[k]) * stride_of(tk, k);
-                            x /= tk.ext[k];
-                        }
+                    // columns kk of the codomain tree, their indices along its legs counted up
+                    uint32_t x[XH_MAXLEGS] = {};
+                    int64_t o = so.src_off;
+                    for(int64_t c = 0; c < tk.cols; ++c, ++kk) {
                         off[kk] = o;
                         if(so.coeff < 0.0) neg |= 1u << kk;
+                        for(int k = NR; k < NL; ++k) {
+                            const int64_t st = stride_of(tk, k);
+                            if(++x[k] < tk.ext[k]) {
+                                o += st;
+                                break;
+                            }
+                            x[k] = 0;
+                            o -= st * (int64_t(tk.ext[k]) - 1);
+                        }
                     }
                 }
                 h_ng[i] = neg;
