@@ -663,14 +663,14 @@ __global__ __launch_bounds__(QR_THREADS) void k_qr_tall(FactorArgs fa)
 // operand R^T, the B operand and the accumulators of v_mfma_f64_16x16x4f64: an accumulator is the
 // B operand of the next product as it is.  A factorised diagonal tile holds R above and X^T = R^-T
 // on and below its diagonal, with R's diagonal in rdiag; X is kept transposed, in LDS in the place
-// of R's block column once that is used up.
+// of R's block column once that is used up, beyond LDS in the output itself.
 // (One barrier per pivot and 16 lanes per dot product of X: 134 us at n = 74, 673 us at n = 190;
 // these tiles 30 and 98 us, 2286 -> 227 us at n = 250.)
 constexpr int CI_THREADS = 1024;
 constexpr int CI_MAX_N = 40000;
 
 __host__ __device__ inline int64_t chol_tiles(int64_t n) { return ((n + 15) / 16) * ((n + 15) / 16 + 1) / 2; }
-__host__ __device__ inline int64_t chol_work_doubles(int64_t n, bool lds) { return chol_tiles(n) * 256 * (lds ? 1 : 2) + 2 * ((n + 15) / 16) * 16; }
+__host__ __device__ inline int64_t chol_work_doubles(int64_t n) { return chol_tiles(n) * 256 + 2 * ((n + 15) / 16) * 16; }
 
 typedef double d4 __attribute__((ext_vector_type(4)));
 
@@ -691,8 +691,7 @@ __global__ __launch_bounds__(CI_THREADS) void k_chol_inv(FactorArgs fa)
     const int nt = (n + 15) / 16;
     const int64_t ntri = chol_tiles(n);
     double* W = work_base<LDS>(smem, fa);
-    double* XT = LDS ? W : W + ntri * 256;          // X's tiles off the diagonal
-    double* rd = W + ntri * (LDS ? 256 : 512);       // shifted original diagonal (dependence threshold)
+    double* rd = W + ntri * 256;                     // shifted original diagonal (dependence threshold)
     double* rdiag = rd + nt * 16;                    // diagonal of R
     constexpr int NW = CI_THREADS / 64;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -805,6 +804,10 @@ __global__ __launch_bounds__(CI_THREADS) void k_chol_inv(FactorArgs fa)
 #pragma unroll
         for(int q = 0; q < 4; ++q) t[o[q]] = c[q];
     };
+    double* X = fa.U + it.u_off;
+    // element q of this lane of tile (i, j), i < j, of X^T outside LDS: rows and columns below n unless j is the
+    // last, which no later column reads
+    auto out_at = [&](int i, int j, int q) -> double* { return X + (16 * i + col) + int64_t(16 * j + row0 + 4 * q) * n; };
     if(wave == 0) factor(0);
     __syncthreads();
     for(int p = 0; p + 1 < nt; ++p) {
@@ -846,12 +849,12 @@ __global__ __launch_bounds__(CI_THREADS) void k_chol_inv(FactorArgs fa)
             for(int i = wave; i < J; i += NW) {
                 c = d4{0, 0, 0, 0};  // S^T = sum_l R_lJ^T X_il^T
                 for(int l = i; l < J; ++l) {
-                    const double *a = tile(l, J), *b = l == i ? tile(i, i) : XT + tri(i, l);
+                    const double *a = tile(l, J), *b = tile(i, l);  // R's diagonal tile holds X^T's
                     double u[4], v[4];
 #pragma unroll
                     for(int q = 0; q < 4; ++q) {
                         u[q] = a[o[q]];
-                        v[q] = b[o[q]];
+                        v[q] = LDS || l == i ? b[o[q]] : *out_at(i, l, q);
                     }
 #pragma unroll
                     for(int q = 0; q < 4; ++q) c = mfma(u[q], l > i || row0 + 4 * q >= col ? v[q] : 0.0, c);
@@ -859,7 +862,8 @@ __global__ __launch_bounds__(CI_THREADS) void k_chol_inv(FactorArgs fa)
                 c = solve(x, r, c, -1.0);
                 if constexpr(!LDS) {
 #pragma unroll
-                    for(int q = 0; q < 4; ++q) XT[tri(i, J) + o[q]] = c[q];
+                    for(int q = 0; q < 4; ++q)
+                        if(16 * J + row0 + 4 * q < n) *out_at(i, J, q) = c[q];
                 }
             }
         }
@@ -867,16 +871,16 @@ __global__ __launch_bounds__(CI_THREADS) void k_chol_inv(FactorArgs fa)
         if constexpr(LDS) {  // at most NW tile rows: one per wave
             if(wave < J) {
 #pragma unroll
-                for(int q = 0; q < 4; ++q) XT[tri(wave, J) + o[q]] = c[q];
+                for(int q = 0; q < 4; ++q) tile(wave, J)[o[q]] = c[q];
             }
             __syncthreads();
         }
     }
     // X to the output, zeros below its diagonal
-    double* X = fa.U + it.u_off;
     for(int t = wave; t < nt * nt; t += NW) {
         const int i = t % nt, j = t / nt;
-        const double* b = i == j ? tile(i, i) : i < j ? XT + tri(i, j) : nullptr;
+        if(!LDS && i < j) continue;  // there already
+        const double* b = i <= j ? tile(i, j) : nullptr;
 #pragma unroll
         for(int q = 0; q < 4; ++q) {
             const int gi = 16 * i + col, gj = 16 * j + row0 + 4 * q;
@@ -1232,12 +1236,12 @@ extern "C" int xh_block_chol_inv(xh_ctx* ctx, const xh_factor_item* items, int64
             if(it.n == 0) continue;
             it.s_off = static_cast<int64_t>(sh.size());
             sh.push_back(shift_rel ? shift_rel[i] : 0.0);
-            if(it.n <= 16 * (CI_THREADS / 64) && size_t(chol_work_doubles(it.n, true)) * sizeof(double) <= budget) {
+            if(it.n <= 16 * (CI_THREADS / 64) && size_t(chol_work_doubles(it.n)) * sizeof(double) <= budget) {
                 small.push_back(it);
-                small_max = std::max(small_max, chol_work_doubles(it.n, true));
+                small_max = std::max(small_max, chol_work_doubles(it.n));
             } else {
                 big.push_back(it);
-                big_max = std::max(big_max, chol_work_doubles(it.n, false));
+                big_max = std::max(big_max, chol_work_doubles(it.n));
             }
         }
         if(sh.empty()) return;
