@@ -192,15 +192,16 @@ int xh_gemm_gather_scatter(xh_ctx* ctx, const xh_gemm_plan* gemm, const xh_gathe
                            int64_t src_elems, const double* B, double* dst, int64_t dst_elems, double alpha);
 /* GEMM tile autotuner (no counterpart in the reference, whose per-block BLAS calls have no tiles
  * to choose): with enable != 0, the first FP64 call of a plan that has 128 x 128 tiles, with
- * beta = 0, runs both tilings (128 x 128 + 64 x 64, and 64 x 64 only), timed with HIP events
+ * beta = 0, runs both tilings (0 and 1 of xh_set_gemm_tiles), timed with HIP events
  * (one host synchronisation), and runs the faster last so that C holds exactly its result; the
  * choice is cached per plan signature (transposes, split-K use, log2 buckets of item count, largest
  * m, n, k and total flops) and reused by later plans of the same signature.  Off by default. */
 int xh_set_gemm_autotune(xh_ctx* ctx, int enable);
 /* autotuner state: cached signatures, tuning runs, cache hits, signatures that chose 64 x 64 only */
 int xh_gemm_autotune_stats(xh_ctx* ctx, int64_t* entries, int64_t* tuned, int64_t* hits, int64_t* chose_64);
-/* FP64 tiling of sectors with both output sides >= 192: 0 = 128 x 128 tiles (default), 1 = 64 x 64
- * tiles like the other sectors.  A tuning switch; no counterpart in the reference. */
+/* FP64 tiling: 0 (default) = 128 x 128 tiles for sectors with both output sides >= 192 that they do
+ * not pad too much, tiles of 32 to 96 a side for the others, the skinny kernel; 1 = 64 x 64 tiles for
+ * every item.  A tuning switch; no counterpart in the reference. */
 int xh_set_gemm_tiles(xh_ctx* ctx, int mode);
 /* HIP-event timing of every xh_gemm launch on the context stream (measurement; no counterpart in
  * the reference): enable (1) / disable (0) / keep (-1); returns the summed kernel time, the flops of

@@ -83,7 +83,7 @@ __device__ __forceinline__ double* work_base(double* smem, const FactorArgs& fa)
 // sqrt(SVD_ZERO), 2e-214 of the largest entry, are left alone.
 // (64 to 8 lanes per pair, three reductions through ds_bpermute, IEEE divisions and square roots
 // took 542 us for the 9 blocks, 32 x 32 the largest, of a two-site tensor at bond 64; three DPP
-// reductions and refined quotients 220 us; this takes 184 us.)
+// reductions and refined quotients 220 us; this takes 180 us.)
 constexpr int SVD_THREADS = 1024;
 
 // Blocks with more columns than this (after transposition) use the block Jacobi path: any block of
@@ -403,7 +403,7 @@ __global__ __launch_bounds__(SVD_THREADS) void k_svd_jacobi(FactorArgs fa)
 //
 // One thread per trailing column, serial over its rows, took 2864 us for the 9 blocks (132 x 85
 // the largest) of a U(1) matrix product tensor at bond 300; columns kept in LDS by such groups
-// 550 us (48 LDS operations per column and reflector); k_qr takes 173 us.
+// 550 us (48 LDS operations per column and reflector); k_qr takes 163 us.
 constexpr int QR_THREADS = 1024;
 
 __host__ __device__ inline int64_t qr_work_doubles(int64_t m, int64_t n, int64_t rows) { return (m < n ? m : n) * (rows + 1) + 1; }
