@@ -101,7 +101,7 @@ def _run(rt, tasks, nlegs, new_rank, shuffled=False, far=0):
 @pytest.mark.parametrize("nlegs,new_rank,exts,ntasks", [
     (0, 0, [1], 3), (1, 1, [1, 5], 700), (4, 2, [1], 1030), (4, 2, [1, 2], 900), (4, 2, [1, 3, 17], 60), (5, 0, [1, 4], 47), (5, 5, [2, 3], 49),
     (7, 3, [1, 2, 5], 200), (20, 9, [1, 1, 2], 40), (12, 5, [2], 5), (3, 1, [40, 70], 30), (3, 2, [90, 110], 2),
-    (10, 4, [3], 2), (9, 3, [2, 4], 3), (2, 1, [1, 2, 3], 5000)])
+    (10, 4, [3], 2), (9, 3, [2, 4], 3), (2, 1, [1, 2, 3], 17000)])
 def test_against_numpy(rt, nlegs, new_rank, exts, ntasks, nsrc):
     r = np.random.default_rng(11)
     for shuffled in (False, True):

@@ -508,60 +508,62 @@ extern "C" int xh_permute_plan_create(xh_ctx* ctx, const xh_permute_desc* desc, 
         // The legs of a task joined (LegC): absolute source strides (abs: one source, its leading
         // dimension folded in), or source row and column strides.  Leg q joins the one before it (of extent >
         // 1) if it goes on where that one ends, so that no leg waits for the products of earlier ones, and
-        // there are no branches, which would be guessed wrong for about every leg.  Pass 1 only counts.
-        struct Joined {
-            uint32_t ext;
-            int32_t col;
-            int64_t st;
-        };
-        auto join_legs = [NL](const xh_permute_task& tk, int64_t ld, bool abs, auto&& leg) {
-            int64_t end = 0;     // where the leg before ends
-            int32_t before = 2;  // its kind: 0 row, 1 column, 2 none
-            for(int q = 0; q < NL; ++q) {
-                const uint32_t e = tk.ext[q];
-                const bool is_col = tk.is_col[q] != 0;
-                const int32_t c = !abs & is_col;
-                const int64_t st = tk.sstride[q] * (abs & is_col ? ld : 1);
-                const bool one = e == 1, joins = (c == before) & (st == end);
-                leg(!one & !joins, e, c, st);  // a new joined leg starts, or the present one is e times longer
+        // there are no branches, which would be guessed wrong for about every leg.  Pass 1 keeps a bit for
+        // each leg that starts a joined one, pass 2 visits these alone.
+        struct LegJoin {
+            int64_t end = 0;       // where the leg before ends
+            uint32_t heads = 0;    // legs that start a joined leg
+            bool col = false;      // kind of the leg before
+            bool far = false;      // a stride of 2^31 or more
+            void add(int q, uint32_t e, int64_t st, bool c)
+            {
+                const bool one = e == 1, head = !one & ((heads == 0) | (st != end) | (c != col));
+                heads |= uint32_t(head) << q;
+                far |= head & (uint64_t(st) >= (uint64_t(1) << 31));
                 end = one ? end : st * e;
-                before = one ? before : c;
+                col = one ? col : c;
             }
         };
-        auto count_joined = [&join_legs](const xh_permute_task& tk, int64_t ld, bool abs, bool& far) {
-            int n = 0;
-            bool f = false;
-            join_legs(tk, ld, abs, [&](bool fresh, uint32_t, int32_t, int64_t st) {
-                n += fresh;
-                f |= fresh & (uint64_t(st) >= (uint64_t(1) << 31));
-            });
-            far |= f;
-            return n;
-        };
-        auto count_rows_cols = [&count_joined, NL](const xh_permute_task& tk, bool& far) {
-            int64_t reach[2] = {0, 0};  // largest source row and column
+        std::vector<uint32_t> heads(static_cast<size_t>(NT));
+        // largest source row and column of a task with row and column strides
+        auto far_reach = [NL](const xh_permute_task& tk) {
+            int64_t reach[2] = {0, 0};
             for(int q = 0; q < NL; ++q) reach[tk.is_col[q] != 0] += (int64_t(tk.ext[q]) - 1) * tk.sstride[q];
-            far |= std::max(reach[0], reach[1]) >= (int64_t(1) << 31);
-            return count_joined(tk, 1, false, far);
+            return std::max(reach[0], reach[1]) >= (int64_t(1) << 31);
         };
-        // from 2048 tasks on several host threads: 5800 tasks of ten legs 330 us, 870 on one
-        const size_t nchunk = NT >= 2048 ? std::max<size_t>(1, std::min<size_t>(xp::WorkerPool::get().size(), size_t(NT) / 1024)) : 1;
+        // on several host threads from 16384 tasks on: they sleep between plans, and waking them for a few
+        // thousand tasks takes longer than it gains (first permute of a seven-leg tensor with some 6000
+        // tasks: 1428 us with threads from 2048 tasks on, 820 so)
+        const size_t nchunk = NT >= 16384 ? std::max<size_t>(1, std::min<size_t>(xp::WorkerPool::get().size(), size_t(NT) / 4096)) : 1;
         std::vector<ChunkCount> cc(nchunk);
         auto chunk_lo = [&](size_t c) { return int64_t(size_t(NT) * c / nchunk); };
         auto classify = [&](size_t c) {
             ChunkCount& k = cc[c];
             for(int64_t t = chunk_lo(c); t < chunk_lo(c + 1); ++t) {
                 const xh_permute_task& tk = desc->tasks[t];
+                // a record is 304 bytes, read in parts, and often written by another thread
+                const char* ahead = reinterpret_cast<const char*>(desc->tasks + std::min(t + 6, chunk_lo(c + 1) - 1));
+                __builtin_prefetch(ahead);
+                __builtin_prefetch(ahead + 64);
+                __builtin_prefetch(ahead + offsetof(xh_permute_task, sstride));
+                __builtin_prefetch(ahead + offsetof(xh_permute_task, is_col));
                 if(tk.rows < 0 || tk.cols < 0 || tk.rows * tk.cols >= (int64_t(1) << 31))
                     throw xh::Error(XH_EINVAL, "permute plan: subblock too large for 32-bit indexing");
                 if(tk.nsrc < 0 || tk.src_begin < 0 || tk.src_begin + tk.nsrc > desc->nsources)
                     throw xh::Error(XH_EINVAL, "permute plan: source range out of bounds");
                 if(t > 0 && tk.src_begin < desc->tasks[t - 1].src_begin + desc->tasks[t - 1].nsrc) k.ordered = false;
+                // one source: most likely of every task, so row and column strides are joined only if they turn
+                // out to be needed
+                const bool abs = tk.nsrc == 1;
+                const int64_t ld = abs ? desc->sources[tk.src_begin].src_ld : 1;
                 int64_t rprod = 1, cprod = 1;
+                LegJoin join;
                 for(int q = 0; q < NL; ++q) {
                     if(tk.ext[q] == 0) throw xh::Error(XH_EINVAL, "permute plan: zero extent");
                     if(tk.sstride[q] < 0 || tk.sstride[q] >= (int64_t(1) << 31)) throw xh::Error(XH_EINVAL, "permute plan: source stride out of range");
                     (q < desc->new_rank ? rprod : cprod) *= tk.ext[q];
+                    const bool is_col = tk.is_col[q] != 0;
+                    join.add(q, tk.ext[q], is_col ? tk.sstride[q] * ld : tk.sstride[q], !abs & is_col);
                 }
                 if(rprod != tk.rows || cprod != tk.cols) throw xh::Error(XH_EINVAL, "permute plan: leg extents do not match the subblock shape");
                 const double elems = double(tk.rows) * double(tk.cols);
@@ -591,14 +593,10 @@ extern "C" int xh_permute_plan_create(xh_ctx* ctx, const xh_permute_desc* desc, 
                     slot[t] = k.ngather;
                     ++k.ngather;
                     k.total += tk.rows * tk.cols;
-                    // one source: most likely of every task, so row and column strides are counted only
-                    // if they turn out to be needed
-                    bool far = false;
-                    if(tk.nsrc == 1)
-                        k.nl1 = std::max(k.nl1, count_joined(tk, desc->sources[tk.src_begin].src_ld, true, far));
-                    else
-                        k.nl2 = std::max(k.nl2, count_rows_cols(tk, far));
-                    if(far) k.near = false;
+                    heads[t] = join.heads;
+                    int& nl = abs ? k.nl1 : k.nl2;
+                    nl = std::max(nl, __builtin_popcount(join.heads));
+                    if(join.far || (!abs && far_reach(tk))) k.near = false;
                 }
             }
         };
@@ -626,9 +624,12 @@ extern "C" int xh_permute_plan_create(xh_ctx* ctx, const xh_permute_desc* desc, 
         if(!single)  // tasks with one source among tasks with several
             for(int64_t t = 0; t < NT; ++t)
                 if(route[t] <= 0 && desc->tasks[t].nsrc == 1) {
-                    bool far = false;
-                    cc[0].nl2 = std::max(cc[0].nl2, count_rows_cols(desc->tasks[t], far));
-                    if(far) cc[0].near = false;
+                    const xh_permute_task& tk = desc->tasks[t];
+                    LegJoin join;
+                    for(int q = 0; q < NL; ++q) join.add(q, tk.ext[q], tk.sstride[q], tk.is_col[q] != 0);
+                    heads[t] = join.heads;
+                    cc[0].nl2 = std::max(cc[0].nl2, __builtin_popcount(join.heads));
+                    if(join.far || far_reach(tk)) cc[0].near = false;
                 }
         int nl = 0;
         bool ordered = true;
@@ -690,19 +691,18 @@ extern "C" int xh_permute_plan_create(xh_ctx* ctx, const xh_permute_desc* desc, 
                         const xh_permute_source* so = single ? desc->sources + tk.src_begin : nullptr;
                         const xh::FastDiv fd = xh::make_fastdiv(uint32_t(std::max<int64_t>(tk.rows, 1)));
                         LegC* L = legc + slot[t] * nl;
-                        Joined J[XH_MAXLEGS + 1], j{1, 0, 0};
-                        for(int k = 1; k <= nl; ++k) J[k] = j;
-                        uint32_t n = 0;
-                        join_legs(tk, so ? so->src_ld : 1, single, [&](bool fresh, uint32_t e, int32_t col, int64_t st) {
-                            n += fresh;
-                            j = Joined{(fresh ? 1 : j.ext) * e, fresh ? col : j.col, fresh ? st : j.st};
-                            J[n] = j;
-                        });
-                        for(int k = 0; k < nl; ++k) {
-                            const xh::FastDiv d = xh::make_fastdiv(J[k + 1].ext);
-                            L[k] = LegC{d.d, d.magic, d.shift | uint32_t(J[k + 1].col << 8), static_cast<uint32_t>(J[k + 1].st)};
+                        int n = 0;
+                        for(uint32_t m = heads[t]; m; ++n) {  // joined legs: from a head to the next, past legs of extent 1
+                            const int q = __builtin_ctz(m);
+                            m &= m - 1;
+                            uint32_t ext = tk.ext[q];
+                            for(int k = q + 1, next = m ? __builtin_ctz(m) : NL; k < next; ++k) ext *= tk.ext[k];
+                            const bool is_col = tk.is_col[q] != 0;
+                            const xh::FastDiv d = xh::make_fastdiv(ext);
+                            L[n] = LegC{ext, d.magic, d.shift | (!so && is_col ? 256u : 0u), static_cast<uint32_t>(so && is_col ? tk.sstride[q] * so->src_ld : tk.sstride[q])};
                         }
-                        taskc[slot[t]] = TaskC{tk.dst_off, tk.dst_ld, so ? so->src_off : 0, so ? so->coeff : 0.0, uint32_t(tk.rows), fd.magic, fd.shift, n,
+                        for(int k = n; k < nl; ++k) L[k] = LegC{1, 1, 0, 0};
+                        taskc[slot[t]] = TaskC{tk.dst_off, tk.dst_ld, so ? so->src_off : 0, so ? so->coeff : 0.0, uint32_t(tk.rows), fd.magic, fd.shift, uint32_t(n),
                                                tk.nsrc, tk.src_begin};
                         continue;
                     }
