@@ -66,6 +66,15 @@ class _GatherDesc(C.Structure):
 @pytest.mark.parametrize("ns", [(1, 3, 8, 11), (1, 5, 8), (17, 32)], ids=["n11", "n8", "n32"])
 @pytest.mark.parametrize("kmax", [12, 32])
 def test_gather_product(rt, kmax, ns, far):
+    gather_product(rt, kmax, ns, far, 40)
+
+
+def test_gather_product_of_many_trees(rt):
+    """Plan tables filled by several host threads."""
+    gather_product(rt, 16, (3,), 0, 8000)
+
+
+def gather_product(rt, kmax, ns, far, ntrees):
     """far: one domain leg of extent 2 whose source entries lie 2^32 elements apart (a 34 GB source)."""
     r = np.random.default_rng(kmax)
     L, ctx = lib(), rt.ctx()
@@ -74,7 +83,7 @@ def test_gather_product(rt, kmax, ns, far):
     tasks, sources, starts, gitems, gemms, ops = [], [], [], [], [], []
     bo = co = 0
     for n in ns:
-        dom = [[int(x) for x in (r.choice([1, 2, 45]), r.choice([1, 3]), 2 if far else r.choice([1, 2, 7]))] for _ in range(40)]
+        dom = [[int(x) for x in (r.choice([1, 2, 45]), r.choice([1, 3]), 2 if far else r.choice([1, 2, 7]))] for _ in range(ntrees)]
         cod = []
         while sum(a * b for a, b in cod) < kmax - 4:
             cod.append((int(r.integers(1, 3)), int(r.integers(1, 3))))

@@ -619,6 +619,12 @@ __global__ __launch_bounds__(SK_THREADS) void k_gemm_skinny(GemmArgs g, const Ti
 constexpr int GA_MAXR = 8;  // domain legs of a gather plan's permuted tensor (checked at plan creation)
 constexpr int GA_SEG = SK_THREADS / 64;  // domain trees one block may meet
 constexpr int GA_RUN = 16;  // consecutive blocks that run on one XCD (with scalar operands: 155 and 153 us above, runs of 1 157 and 160, whole eighths 225, as they differ in work)
+// Table entries (columns, strides) per host thread of a plan: the threads sleep between plans, and waking
+// them takes as long as writing some ten thousand.  First contraction of a five-leg tensor with 2401 trees:
+// 418 us with threads from 512 trees on, 283 so; of a seven-leg one with 15625: 1060 us with 4096 entries a
+// thread, 947 so.  Joining the legs in the checks, which have the tasks at hand and run on several threads
+// anyway, took the device plans of a CTMRG step at chi 96 (permutes too) from 145 to 86 ms on one thread.
+constexpr int64_t GA_GRAIN = 65536;
 struct GatherBlock {
     int64_t b_off, c_off;    // the item's
     int64_t trees;           // its first domain tree in legs and neg
@@ -1919,7 +1925,22 @@ extern "C" int xh_gather_plan_create(xh_ctx* ctx, const xh_gemm_plan* gemm, cons
                     throw xh::Error(XH_EINVAL, "gather plan: source subblock out of bounds");
             }
         });
-        // every item: its trees tile the A block, and its tasks have the trees' shapes
+        // every item: its trees tile the A block, and its tasks have the trees' shapes.  The domain legs of a
+        // tree are joined on the way: a leg goes on with the one before it if it does so in every task.
+        struct Tree {
+            int32_t item;
+            uint32_t heads = 0;  // domain legs that start a joined leg
+        };
+        std::vector<int64_t> tree0(size_t(d->nitems));  // an item's first tree
+        int64_t ntrees = 0;
+        for(int64_t j = 0; j < d->nitems; ++j) {
+            const xh_gemm_item& it = gemm->h_items[j];
+            tree0[j] = ntrees;
+            if(it.m != 0 && it.n != 0) ntrees += std::clamp<int64_t>(d->items[j].ndom, 0, it.m);
+        }
+        std::vector<Tree> trees(size_t(ntrees), Tree{0});
+        std::vector<uint8_t> item_far(size_t(d->nitems), 0);  // a domain stride of 2^32 or more
+        auto stride_of = [&pd](const xh_permute_task& tk, int k, int64_t ld) { return tk.is_col[k] ? tk.sstride[k] * ld : tk.sstride[k]; };
         xp::parallel_ranges(size_t(d->nitems), 1, [&](size_t j0, size_t j1) {
             for(size_t j = j0; j < j1; ++j) {
                 const xh_gemm_item& it = gemm->h_items[j];
@@ -1930,18 +1951,32 @@ extern "C" int xh_gather_plan_create(xh_ctx* ctx, const xh_gemm_plan* gemm, cons
                     throw xh::Error(XH_EINVAL, "gather plan: item tables out of range");
                 const int32_t* ds = d->starts + gi.starts_off;
                 const int32_t* cs = ds + gi.ndom + 1;
-                if(ds[0] != 0 || ds[gi.ndom] != it.m || cs[0] != 0 || cs[gi.ncod] != it.k) throw xh::Error(XH_EINVAL, "gather plan: tree starts do not cover the A block");
+                if(gi.ndom > it.m || ds[0] != 0 || ds[gi.ndom] != it.m || cs[0] != 0 || cs[gi.ncod] != it.k) throw xh::Error(XH_EINVAL, "gather plan: tree starts do not cover the A block");
                 if(gi.ncod > 0xffff) throw xh::Error(XH_EINVAL, "gather plan: too many codomain trees");
+                bool far_stride = false;
                 // the kernel decodes a row with the domain-leg extents of one task of its tree
                 for(int a = 0; a < gi.ndom; ++a) {
                     const xh_permute_task& t0 = pd.tasks[gi.task_base + int64_t(a) * gi.ncod];
+                    uint32_t heads = 0;
                     for(int b = 0; b < gi.ncod; ++b) {
                         const xh_permute_task& tk = pd.tasks[gi.task_base + int64_t(a) * gi.ncod + b];
                         if(ds[a + 1] - ds[a] != tk.rows || cs[b + 1] - cs[b] != tk.cols) throw xh::Error(XH_EINVAL, "gather plan: task shape does not match its trees");
-                        for(int k = 0; k < NR; ++k)
+                        const int64_t ld = pd.sources[tk.src_begin].src_ld;
+                        int64_t end = 0;  // where the leg before ends
+                        uint32_t h = 0;
+                        for(int k = 0; k < NR; ++k) {
                             if(tk.ext[k] != t0.ext[k]) throw xh::Error(XH_EINVAL, "gather plan: domain-leg extents differ within a domain tree");
+                            const int64_t st = stride_of(tk, k, ld);
+                            const bool one = tk.ext[k] == 1;
+                            h |= uint32_t(!one & ((h == 0) | (st != end))) << k;
+                            far_stride |= !one & (st >= (int64_t(1) << 32));
+                            end = one ? end : st * tk.ext[k];
+                        }
+                        heads |= h;
                     }
+                    trees[tree0[j] + a] = Tree{int32_t(j), heads};
                 }
+                item_far[j] = far_stride;
             }
         });
         plan->h_ndom.assign(size_t(d->nitems), 0);
@@ -1960,26 +1995,15 @@ extern "C" int xh_gather_plan_create(xh_ctx* ctx, const xh_gemm_plan* gemm, cons
         }
         // blocks of at most SK_THREADS rows meeting at most GA_SEG domain trees, in the GEMM plan's
         // item order, and the places of the items' tables
-        struct TreeAt {
-            int32_t item, a;
-            int32_t nl = 0;
-            bool far = false;
-            uint8_t leg[GA_MAXR] = {};  // first domain leg of each joined leg
-            uint32_t ext[GA_MAXR] = {};
-        };
         std::vector<GatherBlock> blocks;
         std::vector<GatherBlock> items(size_t(d->nitems));  // an item's part of its blocks
-        std::vector<TreeAt> trees;
         int64_t noffs = 0, npairs = 0;
         {
-            size_t nt = 0, nb = 0;
+            size_t nb = 0;
             for(int64_t j = 0; j < d->nitems; ++j) {
                 const xh_gemm_item& it = gemm->h_items[j];
-                if(it.m == 0 || it.n == 0) continue;
-                nt += size_t(d->items[j].ndom);
-                nb += size_t(it.m / SK_THREADS + d->items[j].ndom / GA_SEG + 2);
+                if(it.m != 0 && it.n != 0) nb += size_t(it.m / SK_THREADS + d->items[j].ndom / GA_SEG + 2);
             }
-            trees.reserve(nt);
             blocks.reserve(nb);
         }
         for(int64_t j = 0; j < d->nitems; ++j) {
@@ -1988,11 +2012,10 @@ extern "C" int xh_gather_plan_create(xh_ctx* ctx, const xh_gemm_plan* gemm, cons
             if(it.m == 0 || it.n == 0) continue;
             const int32_t* ds = d->starts + g.starts_off;
             const int32_t* cs = ds + g.ndom + 1;
-            items[j] = GatherBlock{it.b_off, it.c_off, int64_t(trees.size()), noffs, npairs, int32_t(j), it.m, it.n, it.k, g.ncod, 0, 0, 0, 0, {}, {}};
+            items[j] = GatherBlock{it.b_off, it.c_off, tree0[j], noffs, npairs, int32_t(j), it.m, it.n, it.k, g.ncod, 0, 0, 0, 0, {}, {}};
             for(int b = 0; b < g.ncod; ++b) items[j].first |= 1u << cs[b];
             noffs += int64_t(g.ndom) * it.k;
             npairs += int64_t(g.ndom) * g.ncod;
-            for(int a = 0; a < g.ndom; ++a) trees.push_back(TreeAt{int32_t(j), a});
             int a = 0;
             for(int r = 0; r < it.m;) {
                 GatherBlock bl = items[j];
@@ -2010,47 +2033,15 @@ extern "C" int xh_gather_plan_create(xh_ctx* ctx, const xh_gemm_plan* gemm, cons
             }
         }
         if(blocks.size() > 0x7fffffff - NPART * GA_RUN) throw xh::Error(XH_EINVAL, "gather plan: too many blocks");
-        auto task_of = [&](const TreeAt& tr, int b) -> const xh_permute_task& {
-            const xh_gather_item& g = d->items[tr.item];
-            return pd.tasks[g.task_base + int64_t(tr.a) * g.ncod + b];
-        };
-        auto stride_of = [&](const xh_permute_task& tk, int k) { return tk.is_col[k] ? tk.sstride[k] * pd.sources[tk.src_begin].src_ld : tk.sstride[k]; };
-        // per domain tree: its joined legs
-        xp::parallel_ranges(trees.size(), 256, [&](size_t i0, size_t i1) {
-            for(size_t i = i0; i < i1; ++i) {
-                TreeAt& tr = trees[i];
-                const int ncod = d->items[tr.item].ncod;
-                const xh_permute_task& t0 = task_of(tr, 0);
-                for(int k = 0; k < NR; ++k) {
-                    if(t0.ext[k] == 1) continue;
-                    bool join = tr.nl > 0;
-                    for(int b = 0; b < ncod; ++b) {
-                        const xh_permute_task& tk = task_of(tr, b);
-                        const int64_t st = stride_of(tk, k);
-                        if(st >= (int64_t(1) << 32)) tr.far = true;
-                        if(join && st != stride_of(tk, tr.leg[tr.nl - 1]) * tr.ext[tr.nl - 1]) join = false;
-                    }
-                    if(join) {
-                        tr.ext[tr.nl - 1] *= t0.ext[k];
-                    } else {
-                        tr.leg[tr.nl] = k;
-                        tr.ext[tr.nl++] = t0.ext[k];
-                    }
-                }
-            }
-        });
         int nl = 0;
-        bool far = false;
-        for(const TreeAt& tr : trees) {
-            nl = std::max(nl, int(tr.nl));
-            far = far || tr.far;
-        }
+        for(const Tree& tr : trees) nl = std::max(nl, __builtin_popcount(tr.heads));
+        const bool far = std::find(item_far.begin(), item_far.end(), 1) != item_far.end();
         for(GatherBlock& bl : items) bl.strides *= nl;
         for(GatherBlock& bl : blocks) bl.strides *= nl;
         xh::PackedUpload& up = plan->up;
-        const size_t ntrees = trees.size(), nst = size_t(npairs * nl), nhi = far ? nst : 0;
+        const size_t nst = size_t(npairs * nl), nhi = far ? nst : 0;
         const size_t bytes = xh::PackedUpload::packed_bytes({blocks.size() * sizeof(GatherBlock), size_t(noffs) * sizeof(int64_t),
-                                                             nst * sizeof(uint32_t), nhi * sizeof(uint32_t), ntrees * nl * sizeof(RowLeg), ntrees * sizeof(uint32_t)});
+                                                             nst * sizeof(uint32_t), nhi * sizeof(uint32_t), size_t(ntrees * nl) * sizeof(RowLeg), size_t(ntrees) * sizeof(uint32_t)});
         if(bytes >= (size_t(1) << 18)) up.begin_pinned(ctx, bytes);
         auto put = [&up](const auto& vec) {
             using T = typename std::decay_t<decltype(vec)>::value_type;
@@ -2060,30 +2051,38 @@ extern "C" int xh_gather_plan_create(xh_ctx* ctx, const xh_gemm_plan* gemm, cons
         };
         const size_t o_bl = put(blocks);
         const size_t o_of = up.reserve<int64_t>(noffs), o_st = up.reserve<uint32_t>(int64_t(nst)), o_hi = up.reserve<uint32_t>(int64_t(nhi)),
-                     o_lg = up.reserve<RowLeg>(int64_t(ntrees * nl)), o_ng = up.reserve<uint32_t>(int64_t(ntrees));
+                     o_lg = up.reserve<RowLeg>(ntrees * nl), o_ng = up.reserve<uint32_t>(ntrees);
         int64_t* h_of = up.host_ptr<int64_t>(o_of);
         uint32_t *h_st = up.host_ptr<uint32_t>(o_st), *h_hi = up.host_ptr<uint32_t>(o_hi), *h_ng = up.host_ptr<uint32_t>(o_ng);
         RowLeg* h_lg = up.host_ptr<RowLeg>(o_lg);
-        xp::parallel_ranges(ntrees, 256, [&](size_t i0, size_t i1) {
+        const int64_t work = noffs + npairs * (nl + 2);
+        xp::parallel_ranges(size_t(ntrees), size_t(std::max<int64_t>(1, ntrees * GA_GRAIN / std::max<int64_t>(work, 1))), [&](size_t i0, size_t i1) {
             for(size_t i = i0; i < i1; ++i) {
-                const TreeAt& tr = trees[i];
+                const Tree& tr = trees[i];
                 const GatherBlock& gi = items[tr.item];
-                for(int q = 0; q < nl; ++q) {
-                    const uint32_t ext = q < tr.nl ? tr.ext[q] : 1u;
+                const int64_t a = int64_t(i) - gi.trees;
+                const xh_permute_task* tasks = pd.tasks + d->items[tr.item].task_base + a * gi.ncod;
+                int head[GA_MAXR] = {}, n = 0;
+                for(uint32_t m = tr.heads; m; ++n) {  // from a head to the next, past legs of extent 1
+                    const int q = head[n] = __builtin_ctz(m);
+                    m &= m - 1;
+                    uint32_t ext = tasks[0].ext[q];
+                    for(int k = q + 1, next = m ? __builtin_ctz(m) : NR; k < next; ++k) ext *= tasks[0].ext[k];
                     const xh::FastDiv fd = xh::make_fastdiv(ext);
-                    h_lg[i * nl + q] = RowLeg{ext, fd.magic, fd.shift, 0};
+                    h_lg[i * nl + n] = RowLeg{ext, fd.magic, fd.shift, 0};
                 }
-                int64_t* off = h_of + gi.offs + int64_t(tr.a) * gemm->h_items[tr.item].k;
+                for(int q = n; q < nl; ++q) h_lg[i * nl + q] = RowLeg{1, 1, 0, 0};
+                int64_t* off = h_of + gi.offs + a * gi.k;
+                int64_t at = gi.strides + a * gi.ncod * nl;
                 uint32_t neg = 0;
                 int kk = 0;
-                for(int b = 0; b < gi.ncod; ++b) {
-                    const xh_permute_task& tk = task_of(tr, b);
+                for(int b = 0; b < gi.ncod; ++b, at += nl) {
+                    const xh_permute_task& tk = tasks[b];
                     const xh_permute_source& so = pd.sources[tk.src_begin];
                     for(int q = 0; q < nl; ++q) {
-                        const uint64_t st = q < tr.nl ? uint64_t(stride_of(tk, tr.leg[q])) : 0;
-                        const int64_t at = gi.strides + (int64_t(tr.a) * gi.ncod + b) * nl + q;
-                        h_st[at] = uint32_t(st);
-                        if(far) h_hi[at] = uint32_t(st >> 32);
+                        const uint64_t st = q < n ? uint64_t(stride_of(tk, head[q], so.src_ld)) : 0;
+                        h_st[at + q] = uint32_t(st);
+                        if(far) h_hi[at + q] = uint32_t(st >> 32);
                     }
                     // columns kk of the codomain tree, their indices along its legs counted up
                     uint32_t x[XH_MAXLEGS] = {};
@@ -2092,7 +2091,7 @@ extern "C" int xh_gather_plan_create(xh_ctx* ctx, const xh_gemm_plan* gemm, cons
                         off[kk] = o;
                         if(so.coeff < 0.0) neg |= 1u << kk;
                         for(int k = NR; k < NL; ++k) {
-                            const int64_t st = stride_of(tk, k);
+                            const int64_t st = stride_of(tk, k, so.src_ld);
                             if(++x[k] < tk.ext[k]) {
                                 o += st;
                                 break;
